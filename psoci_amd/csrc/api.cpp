@@ -265,8 +265,8 @@ int psoci_direct_ras_info(psoci_ctx* ctx, int* m, int* n_external, int* nsectors
     if (nsectors) *nsectors = (int)P.sec.size();
     if (nblocks) *nblocks = (int)P.blk.size();
     if (ndet) *ndet = P.ndet;
-    if (w_per_column) *w_per_column = P.wunit;
-    if (flops_per_column) *flops_per_column = P.gemm_flops_per_col;
+    if (w_per_column) *w_per_column = P.cwunit;
+    if (flops_per_column) *flops_per_column = P.cflops_per_col;
     return PSOCI_OK;
   });
 }

@@ -105,15 +105,17 @@ struct Ctx {
   DevBuf<uint32_t> d_rasadd;
   DevBuf<int32_t> d_rasrem;
   DevBuf<RasBlockDev> d_rasblk;
-  DevBuf<int16_t> d_rasq, d_raspidx;
-  DevBuf<uint64_t> d_rasqm;  // per block and chunk: bits of the first-added orbitals
+  DevBuf<RasCmp> d_rascmp;
+  DevBuf<int16_t> d_raspidx;
+  DevBuf<RasTile> d_rastile[4];        // product tiles for chunks of 16, 8, 4 and 2 columns
+  std::vector<RasLaunch> ras_launch[4];  // and their launches
   DevBuf<RasSef> d_rassef;
-  DevBuf<double> d_rasg64;
+  DevBuf<double> d_rasg64;  // the compact products' matrices
   DevBuf<float> d_rasg32;
   DevBuf<RasView> d_rasview;
-  DevBuf<char> d_rasc, d_rasw;  // determinant vectors [2 ndet + 2][16 FP32 | ras_kc64 FP64], W [wunit][same]
+  DevBuf<char> d_rasc, d_rasw;  // determinant vectors [2 ndet + 2][16 FP32 | ras_kc64 FP64], W [cwunit][same]
   int ras_kc64 = 8;             // FP64 columns per chunk (16 when memory allows, else 8)
-  DevBuf<int32_t> d_rasdidx;    // [dunit]: signed vector row (2 det + negative) of every D entry
+  DevBuf<int32_t> d_rasdidx;    // [cdunit]: signed vector row (2 det + negative) of every D entry
   DevBuf<int64_t> d_rastoff;    // nsef + 1: first term of each SEF
   int64_t ras_nterm = 0;        // terms over all SEFs (after merging mirrored pairs)
   DevBuf<int32_t> d_rasterm;    // signed W offsets (bit 31: negative)
@@ -127,9 +129,12 @@ struct Ctx {
     d_rasadd.release();
     d_rasrem.release();
     d_rasblk.release();
-    d_rasq.release();
-    d_rasqm.release();
+    d_rascmp.release();
     d_raspidx.release();
+    for (int k = 0; k < 4; ++k) {
+      d_rastile[k].release();
+      ras_launch[k].clear();
+    }
     d_rassef.release();
     d_rasg64.release();
     d_rasg32.release();

@@ -104,6 +104,74 @@ struct Ranker {
   }
 };
 
+// The compact layout of block B (RasCmp), appended to the plan's totals.
+// Level: the cheapest in multiply-adds over the tiles' rows (groups padded
+// to the 8 rows of a 16-column tile; the pairs to 16) among those whose
+// matrices stay small next to the rows that use them: nqp <= 32 rows of a
+// group keeps the matrices' elements within twice the block's 16-column W.
+// On 10 + 24 orbitals, 8 electrons (2.62e11 -> 1.44e11 flops and 5.24e8 ->
+// 3.61e8 W elements per column): level 2 for the alpha-beta classes with
+// external electrons in w (24-row groups, 580 -> 416 pairs), level 1 for the
+// internal ones (1156 -> 1054) and the same-spin products (285 -> 220, 45 ->
+// 28).  Sigma of 16 columns: FP32 48.7 -> 31.4 ms, FP64 86.0 -> 52.1 ms; on
+// 8 + 24 orbitals, 6 electrons (5.8e9 -> 4.2e9 flops) FP64 8 columns 1.36 ->
+// 1.02 ms.
+RasCmp compact(RasPlan& P, const RasBlockDev& B, int nI, int nE) {
+  const Binom& Bn = binom();
+  RasCmp C;
+  std::memset(&C, 0, sizeof(C));
+  C.kind = B.kind;
+  C.sector = B.sector;
+  C.tri = B.tri;
+  C.budget = B.budget;
+  C.swap = B.kind == 2;
+  C.lo = C.swap ? B.lw : B.lu;
+  C.li = C.swap ? B.lu : B.lw;
+  const int co = C.swap ? B.cw : B.cu, ci = C.swap ? B.cu : B.cw;
+  C.nIo = (int)Bn(nI, C.lo - co);
+  C.nEo = (int)Bn(nE, co);
+  C.nIi = (int)Bn(nI, C.li - ci);
+  C.nEi = (int)Bn(nE, ci);
+  C.o0 = C.swap ? B.w0 : B.u0;
+  C.i0 = C.swap ? B.u0 : B.w0;
+  C.nrows = B.nrows;
+  auto live = [&](int level) {
+    const int a = nI - (level >= 1 ? C.lo - co : 0), b = C.budget;
+    if (C.kind == 0) {
+      const int r = nI - (level == 2 ? C.li - ci : 0);
+      return a * r + (b >= 1 ? (a + r) * nE : 0) + (b >= 2 ? nE * nE : 0);
+    }
+    return a * (a - 1) / 2 + (b >= 1 ? a * nE : 0) + (b >= 2 ? nE * (nE - 1) / 2 : 0);
+  };
+  double best = 0.0;
+  for (int level = 0; level <= (C.kind == 0 ? 2 : 1); ++level) {
+    RasCmp T = C;
+    T.level = level;
+    const double nqp = (live(level) + 15) / 16 * 16;
+    double cost = 0.0;
+    int64_t nvar = 0, most = 0;
+    ras_cmp_groups(T, [&](int64_t, int64_t, int64_t rows) {
+      cost += (double)((rows + 7) / 8 * 8) * nqp * nqp;
+      most = std::max(most, rows);
+      ++nvar;
+    });
+    if (level > 0 && (cost >= best || nqp > 32.0 * (double)most)) continue;
+    best = cost;
+    C.level = level;
+    C.nvar = nvar;
+    C.nq = live(level);
+  }
+  C.nqp = (C.nq + 15) / 16 * 16;
+  C.gbase = P.cgunit;
+  C.wbase = P.cwunit;
+  C.dbase = P.cdunit;
+  P.cgunit += C.nvar * C.nqp * C.nqp;
+  P.cwunit += C.nrows * C.nqp;
+  P.cdunit += C.nrows * C.nqp;
+  P.cflops_per_col += 2.0 * (double)C.nrows * C.nq * C.nq;
+  return C;
+}
+
 }  // namespace
 
 void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two) {
@@ -389,6 +457,7 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two)
     }
   }
   (void)nb2;
+  for (const RasBlockDev& B : P.blk) P.cmp.push_back(compact(P, B, rk.nI, rk.nE));
   if (wunit >= ((int64_t)1 << 31)) return fail("more than 2^31 W elements per column");
   if (dunit >= ((int64_t)1 << 31)) return fail("more than 2^31 D index entries");
   P.wunit = wunit;
@@ -478,6 +547,8 @@ RasView ras_host_view(const RasPlan& P) {
   v.nsef = (int64_t)P.sef.size();
   v.ndet = P.ndet;
   v.wunit = P.wunit;
+  v.emask = P.emask;
+  v.imask = (P.nbf == 64 ? ~0ull : (1ull << P.nbf) - 1ull) & ~P.emask;
   return v;
 }
 

@@ -101,6 +101,47 @@ struct RasBlockDev {
   int64_t qmoff, umoff;
 };
 
+// The compact layout of one dense product (the one the GPU evaluates).  An
+// orbital that the outer string of a row already holds (the (N-1)- or
+// (N-2)-electron string that gains electrons: u, or w for the beta-beta
+// products) cannot be added to it, so about half of the full product's pairs
+// multiply zeros and half of its outputs are never read.  Rows are ordered
+// by the internal parts of their strings, (outer internal oi, inner internal
+// ii, outer external oe, inner external ie), and cut into groups whose rows
+// share the internal orbitals that the pairs drop:
+//   level 0  one group, nothing dropped;
+//   level 1  a group per oi, pairs without oi's orbitals;
+//   level 2  (alpha-beta only) a group per (oi, ii), p without oi's and r
+//            without ii's orbitals.
+// Every group of a block has the same number nq of live pairs (padded to
+// nqp), listed by ras_cmp_pair; each has its own integral matrix ("variant")
+// at gbase + variant * nqp * nqp.  W element (wbase + row * nqp + pair) per
+// column, D index entry dbase + row * nqp + pair.
+struct RasCmp {
+  int level, kind, sector, tri;
+  int budget, nq, nqp;
+  int swap;          // 1: the outer string is w (beta-beta)
+  int lo, li;        // levels of the outer and inner strings
+  int nIo, nEo, nIi, nEi;  // internal and external parts of the class's strings
+  int64_t o0, i0;    // first string of the class (global index within the level)
+  int64_t nrows, nvar, gbase, wbase, dbase;
+};
+
+// One tile of a product: nrows rows (the tile's first at the W and D
+// offsets) times p-pairs [p0, p0 + 16 niv) of the group's nqp.
+struct RasTile {
+  int64_t g, w, d;   // the group's matrix, W per column, D index table
+  int32_t nqp;
+  uint16_t p0;
+  uint8_t nrows, niv;
+};
+
+// One launch's tiles in the tile table: all of one kind and tile width.
+struct RasLaunch {
+  int pt, kind;
+  int64_t tile0, ntiles;
+};
+
 // The determinants of one SEF (one or two): alpha / beta global string
 // indices, sector, and flags (bit 0 negative coefficient, bit 1 closed
 // shell: coefficient +-1 instead of +-1/sqrt(2)); n = 1 or 2.
@@ -126,6 +167,9 @@ struct RasView {
   const RasSef* sef;
   int64_t nsef;
   int64_t ndet, wunit;  // determinants and W elements per column (bounds of every index)
+  uint64_t imask, emask;  // internal and external orbitals
+  // the blocks' compact layouts; null: W offsets of the full products
+  const RasCmp* cmp;
 };
 
 // triangular row of (u, w), u <= w < n (local indices), and its inverse
@@ -150,12 +194,41 @@ PSOCI_HD int64_t ras_det(const RasView& v, int s, int ca, int64_t ra, int cb, in
 // class of global string index g of level n
 PSOCI_HD int ras_cls_of(const RasView& v, int n, int64_t g) { return v.cls[v.lev[n].mask_off + g]; }
 
-// the determinant (and sign) of D-entry (row, pair j) of block B: -1 when
-// the pair cannot be added to the row strings
+// the determinant (and sign) that adding the pair (q, s) to the strings u, w
+// of a product of the given kind gives: -1 when it cannot be added
+PSOCI_HD int64_t ras_d_det(const RasView& v, int kind, int sector, int lu, int lw, int64_t u, int64_t w, int q, int s,
+                           int& neg) {
+  const RasSectorDev& S = v.sec[sector];
+  if (kind == 0) {
+    const uint32_t ea = v.add[v.lev[lu].add_off + u * v.nbf + q];
+    const uint32_t eb = v.add[v.lev[lw].add_off + w * v.nbf + s];
+    if (ea == kRasNone || eb == kRasNone) return -1;
+    neg = ras_neg(ea) ^ ras_neg(eb);
+    return ras_det(v, sector, ras_cls(ea), ras_rank(ea), ras_cls(eb), ras_rank(eb));
+  }
+  // same spin: add s, then q (q > s), to the N-2 string; the other spin's
+  // string is the row's own
+  const int l2 = kind == 1 ? lu : lw;
+  const int64_t k2 = kind == 1 ? u : w;
+  const uint32_t e1 = v.add[v.lev[l2].add_off + k2 * v.nbf + s];
+  if (e1 == kRasNone) return -1;
+  const int64_t g1 = v.lev[l2 + 1].cls_off[ras_cls(e1)] + ras_rank(e1);
+  const uint32_t e2 = v.add[v.lev[l2 + 1].add_off + g1 * v.nbf + q];
+  if (e2 == kRasNone) return -1;
+  neg = ras_neg(e1) ^ ras_neg(e2);
+  if (kind == 1) {
+    const int cb = ras_cls_of(v, S.nb, w);
+    return ras_det(v, sector, ras_cls(e2), ras_rank(e2), cb, w - v.lev[S.nb].cls_off[cb]);
+  }
+  const int ca = ras_cls_of(v, S.na, u);
+  return ras_det(v, sector, ca, u - v.lev[S.na].cls_off[ca], ras_cls(e2), ras_rank(e2));
+}
+
+// the determinant (and sign) of D-entry (row, pair j) of block B's full
+// layout: -1 when the pair cannot be added to the row strings
 PSOCI_HD int64_t ras_d_entry(const RasView& v, const RasBlockDev& B, int64_t row, int j, int& neg) {
   const int16_t qs = v.qlist[B.qoff + j];
   if (qs < 0) return -1;
-  const int q = qs & 0xff, s = (qs >> 8) & 0xff;
   int64_t u, w;
   if (B.tri) {
     ras_tri_uw(row, B.nu, u, w);
@@ -165,30 +238,109 @@ PSOCI_HD int64_t ras_d_entry(const RasView& v, const RasBlockDev& B, int64_t row
     u = B.u0 + row / B.nw;
     w = B.w0 + row % B.nw;
   }
-  const RasSectorDev& S = v.sec[B.sector];
-  if (B.kind == 0) {
-    const uint32_t ea = v.add[v.lev[B.lu].add_off + u * v.nbf + q];
-    const uint32_t eb = v.add[v.lev[B.lw].add_off + w * v.nbf + s];
-    if (ea == kRasNone || eb == kRasNone) return -1;
-    neg = ras_neg(ea) ^ ras_neg(eb);
-    return ras_det(v, B.sector, ras_cls(ea), ras_rank(ea), ras_cls(eb), ras_rank(eb));
+  return ras_d_det(v, B.kind, B.sector, B.lu, B.lw, u, w, qs & 0xff, (qs >> 8) & 0xff, neg);
+}
+
+// ---- compact layout (RasCmp) ----
+
+// first row of cell (oi, ii) (triangular blocks: oi <= ii; their diagonal
+// cells hold the oe <= ie triangle)
+PSOCI_HD int64_t ras_cmp_cell(const RasCmp& C, int64_t oi, int64_t ii) {
+  const int64_t F = (int64_t)C.nEo * C.nEi;
+  if (!C.tri) return (oi * C.nIi + ii) * F;
+  const int64_t Dg = (int64_t)C.nEo * (C.nEo + 1) / 2;
+  const int64_t cell = ras_tri_row(oi, ii, C.nIo), nd = oi + (ii > oi ? 1 : 0);
+  return nd * Dg + (cell - nd) * F;
+}
+// row of local strings o, i
+PSOCI_HD int64_t ras_cmp_row(const RasCmp& C, int64_t o, int64_t i) {
+  const int64_t oi = o / C.nEo, oe = o % C.nEo, ii = i / C.nEi, ie = i % C.nEi;
+  const int64_t b = ras_cmp_cell(C, oi, ii);
+  return C.tri && oi == ii ? b + ras_tri_row(oe, ie, C.nEo) : b + oe * C.nEi + ie;
+}
+// local strings of a row
+PSOCI_HD void ras_cmp_unrow(const RasCmp& C, int64_t row, int64_t& o, int64_t& i) {
+  const int64_t F = (int64_t)C.nEo * C.nEi;
+  int64_t oi, ii, oe, ie;
+  if (!C.tri) {
+    const int64_t cell = row / F, r = row % F;
+    oi = cell / C.nIi;
+    ii = cell % C.nIi;
+    oe = r / C.nEi;
+    ie = r % C.nEi;
+  } else {
+    int64_t lo = 0, hi = C.nIo - 1;  // the last oi whose rows start at or before row
+    while (lo < hi) {
+      const int64_t mid = (lo + hi + 1) >> 1;
+      if (ras_cmp_cell(C, mid, mid) <= row) lo = mid;
+      else hi = mid - 1;
+    }
+    oi = lo;
+    const int64_t r = row - ras_cmp_cell(C, oi, oi), Dg = (int64_t)C.nEo * (C.nEo + 1) / 2;
+    if (r < Dg) {
+      ii = oi;
+      ras_tri_uw(r, C.nEo, oe, ie);
+    } else {
+      ii = oi + 1 + (r - Dg) / F;
+      oe = (r - Dg) % F / C.nEi;
+      ie = (r - Dg) % F % C.nEi;
+    }
   }
-  // same spin: add s, then q (q > s), to the N-2 string; the other spin's
-  // string is the row's own
-  const int l2 = B.kind == 1 ? B.lu : B.lw;
-  const int64_t k2 = B.kind == 1 ? u : w;
-  const uint32_t e1 = v.add[v.lev[l2].add_off + k2 * v.nbf + s];
-  if (e1 == kRasNone) return -1;
-  const int64_t g1 = v.lev[l2 + 1].cls_off[ras_cls(e1)] + ras_rank(e1);
-  const uint32_t e2 = v.add[v.lev[l2 + 1].add_off + g1 * v.nbf + q];
-  if (e2 == kRasNone) return -1;
-  neg = ras_neg(e1) ^ ras_neg(e2);
-  if (B.kind == 1) {
-    const int cb = ras_cls_of(v, S.nb, w);
-    return ras_det(v, B.sector, ras_cls(e2), ras_rank(e2), cb, w - v.lev[S.nb].cls_off[cb]);
+  o = oi * C.nEo + oe;
+  i = ii * C.nEi + ie;
+}
+// the integral variant of a row's cell
+PSOCI_HD int64_t ras_cmp_var(const RasCmp& C, int64_t oi, int64_t ii) {
+  if (C.level == 0) return 0;
+  if (C.level == 1) return oi;
+  return C.tri ? ras_tri_row(oi, ii, C.nIo) : oi * C.nIi + ii;
+}
+// the internal orbitals that the pairs of cell (oi, ii) drop: from p (both
+// electrons for the same-spin products) and, at level 2, from r
+PSOCI_HD void ras_cmp_drop(const RasView& v, const RasCmp& C, int64_t oi, int64_t ii, uint64_t& op, uint64_t& ir) {
+  op = C.level >= 1 ? v.mask[v.lev[C.lo].mask_off + C.o0 + oi * C.nEo] & v.imask : 0ull;
+  ir = C.level == 2 ? v.mask[v.lev[C.li].mask_off + C.i0 + ii * C.nEi] & v.imask : 0ull;
+}
+// position of the live pair (p, r) (same spin: p > r) among the pairs that
+// drop op / ir; pairs are p-major, both ascending
+PSOCI_HD int ras_cmp_pair(const RasView& v, const RasCmp& C, uint64_t op, uint64_t ir, int p, int r) {
+  const int nE = popc(v.emask), b = C.budget;
+  const uint64_t bp = (1ull << p) - 1ull, br = (1ull << r) - 1ull;
+  const int ep = (int)((v.emask >> p) & 1);
+  if (C.kind == 0) {
+    const uint64_t ri = v.imask & ~ir;
+    const int nr = popc(ri);
+    int k = popc(v.imask & ~op & bp) * (nr + (b >= 1 ? nE : 0));
+    if (b >= 1) k += popc(v.emask & bp) * (nr + (b >= 2 ? nE : 0));
+    return k + popc((ri | (b - ep >= 1 ? v.emask : 0ull)) & br);
   }
-  const int ca = ras_cls_of(v, S.na, u);
-  return ras_det(v, B.sector, ca, u - v.lev[S.na].cls_off[ca], ras_cls(e2), ras_rank(e2));
+  const uint64_t li = v.imask & ~op;
+  int k = 0;
+  for (uint64_t x = (li | (b >= 1 ? v.emask : 0ull)) & bp; x; x &= x - 1) {
+    const int o = ctz(x);
+    const int eo = (int)((v.emask >> o) & 1);
+    k += popc((li | (b - eo >= 1 ? v.emask : 0ull)) & ((1ull << o) - 1ull));
+  }
+  return k + popc((li | (b - ep >= 1 ? v.emask : 0ull)) & br);
+}
+// calls f(position, p, r) for every live pair of the cell's variant
+template <class F>
+PSOCI_HD void ras_cmp_pairs(const RasView& v, const RasCmp& C, uint64_t op, uint64_t ir, F&& f) {
+  int k = 0;
+  for (uint64_t x = (v.imask & ~op) | (C.budget >= 1 ? v.emask : 0ull); x; x &= x - 1) {
+    const int p = ctz(x);
+    const int ep = (int)((v.emask >> p) & 1);
+    uint64_t y = (v.imask & ~(C.kind == 0 ? ir : op)) | (C.budget - ep >= 1 ? v.emask : 0ull);
+    if (C.kind != 0) y &= (1ull << p) - 1ull;
+    for (; y; y &= y - 1) f(k++, p, ctz(y));
+  }
+}
+// W offset per column of pair (p, r) at the block's local strings (u, w)
+PSOCI_HD int64_t ras_cmp_off(const RasView& v, const RasCmp& C, int64_t u, int64_t w, int p, int r) {
+  const int64_t o = C.swap ? w : u, i = C.swap ? u : w;
+  uint64_t op, ir;
+  ras_cmp_drop(v, C, o / C.nEo, i / C.nEi, op, ir);
+  return C.wbase + ras_cmp_row(C, o, i) * C.nqp + ras_cmp_pair(v, C, op, ir, p, r);
 }
 
 // Calls f(block index, W element offset per column (wbase + row * nqp +
@@ -249,7 +401,7 @@ PSOCI_HD void ras_terms(const RasView& v, int s, int64_t a, int64_t b, F&& f) {
           continue;
         }
         const int64_t row = B.tri ? ras_tri_row(ul, wl, B.nu) : ul * B.nw + wl;
-        f(bi, B.wbase + row * B.nqp + pi, (tp + tr) & 1);
+        f(bi, v.cmp ? ras_cmp_off(v, v.cmp[bi], ul, wl, pp, rr) : B.wbase + row * B.nqp + pi, (tp + tr) & 1);
       }
     }
   }
@@ -281,9 +433,10 @@ PSOCI_HD void ras_terms(const RasView& v, int s, int64_t a, int64_t b, F&& f) {
           f(-1, (int64_t)-1, 0);
           continue;
         }
-        const int64_t row =
-            (spin == 0 || mir) ? (k2 - B.u0) * B.nw + (o - B.w0) : (o - B.u0) * B.nw + (k2 - B.w0);
-        f(bi, B.wbase + row * B.nqp + pi, (tp + tr) & 1);
+        const int64_t ul = (spin == 0 || mir) ? k2 - B.u0 : o - B.u0;
+        const int64_t wl = (spin == 0 || mir) ? o - B.w0 : k2 - B.w0;
+        f(bi, v.cmp ? ras_cmp_off(v, v.cmp[bi], ul, wl, p, r) : B.wbase + (ul * B.nw + wl) * B.nqp + pi,
+          (tp + tr) & 1);
       }
     }
   }
@@ -378,7 +531,33 @@ struct RasPlan {
   int64_t wunit = 0;  // W elements per column
   int64_t dunit = 0;  // D index table entries
   double gemm_flops_per_col = 0.0;  // 2 * sum over blocks of rows * nq^2
+  // the compact layout: per block, its totals (per column) and flops
+  std::vector<RasCmp> cmp;
+  int64_t cwunit = 0, cdunit = 0, cgunit = 0;
+  double cflops_per_col = 0.0;
 };
+
+// rows and first row of every group of a block, in the row order: calls
+// f(variant, first row, rows)
+template <class F>
+inline void ras_cmp_groups(const RasCmp& C, F&& f) {
+  if (C.level == 0) {
+    f((int64_t)0, (int64_t)0, C.nrows);
+    return;
+  }
+  for (int64_t oi = 0; oi < C.nIo; ++oi) {
+    if (C.level == 1) {
+      const int64_t r0 = ras_cmp_cell(C, oi, C.tri ? oi : 0);
+      const int64_t r1 = oi + 1 < C.nIo ? ras_cmp_cell(C, oi + 1, C.tri ? oi + 1 : 0) : C.nrows;
+      f(oi, r0, r1 - r0);
+      continue;
+    }
+    for (int64_t ii = C.tri ? oi : 0; ii < C.nIi; ++ii) {
+      f(ras_cmp_var(C, oi, ii), ras_cmp_cell(C, oi, ii),
+        C.tri && oi == ii ? (int64_t)C.nEo * (C.nEo + 1) / 2 : (int64_t)C.nEo * C.nEi);
+    }
+  }
+}
 
 // Builds the plan for the space and integrals; plan.ok = false (with a
 // reason) when the space is not a complete RAS space of the supported kind.

@@ -12,11 +12,12 @@
 //               without collisions; both signs, so a product reads an entry
 //               of either sign without arithmetic), rows 2 ndet and 2 ndet +
 //               1 zero;
-//   k_ras_gemm  per block: W[row][p-pair][KC] = sum over q-pairs of
-//               G[p-pair][q-pair] D[row][q-pair][KC], D gathered from c into
-//               LDS through the signed row of each entry (built once from
-//               the string addition tables by k_ras_didx), the product on
-//               MFMA (v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64);
+//   k_ras_gemm  per tile of the compact products (RasCmp, ras.hpp): W[row]
+//               [p-pair][KC] = sum over q-pairs of G[p-pair][q-pair]
+//               D[row][q-pair][KC], D gathered from c into LDS through the
+//               signed row of each entry (built once from the string addition
+//               tables by k_ras_didx), the product on MFMA
+//               (v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64);
 //   k_ras_y     per SEF and column: y = scale * sum of +-W over the RI
 //               terms of its determinants (the term list -- signed W offsets
 //               -- is built once at setup by k_ras_terms), written once (a
@@ -33,46 +34,8 @@ namespace psoci {
 
 namespace {
 
-// GEMM tile shape, LDS layout and schedule (compile-time tuning knobs; the
-// defaults are the fastest measured on mrci10x24: FP32 16-pair chunks
-// without register prefetch, which keeps 6 wavefronts per SIMD, and FP64
-// 16-pair chunks with the next chunk's loads issued before the MFMA steps)
-#ifndef PSOCI_RAS_QC
-#define PSOCI_RAS_QC 16
-#endif
-#ifndef PSOCI_RAS_QC64
-#define PSOCI_RAS_QC64 16
-#endif
-#ifndef PSOCI_RAS_GPAD
-#define PSOCI_RAS_GPAD 1
-#endif
-#ifndef PSOCI_RAS_DPAD
-#define PSOCI_RAS_DPAD 4
-#endif
-#ifndef PSOCI_RAS_VSTORE
-#define PSOCI_RAS_VSTORE 1
-#endif
-#ifndef PSOCI_RAS_PIPE
-#define PSOCI_RAS_PIPE 0
-#endif
-#ifndef PSOCI_RAS_PIPE64
-#define PSOCI_RAS_PIPE64 1
-#endif
-// 16- and 8-column chunks through the LDS-copy product k_ras_gemm_lds (0:
-// the register-staged k_ras_gemm for every width)
-#ifndef PSOCI_RAS_DMA
-#define PSOCI_RAS_DMA 1
-#endif
-// FP32 LDS-copy products in chunks of 32 pairs (0: 16)
-#ifndef PSOCI_RAS_LQC32
-#define PSOCI_RAS_LQC32 0
-#endif
-constexpr int kMT = 128;            // (row, column) values per GEMM tile
-// q-pairs per LDS chunk (FP32, FP64)
-template <typename T>
-constexpr int ras_qc() {
-  return sizeof(T) == 8 ? PSOCI_RAS_QC64 : PSOCI_RAS_QC;
-}
+constexpr int kMT = 128;  // (row, column) values per product tile
+constexpr int kQC = 16;   // q-pairs per LDS chunk
 
 inline unsigned nblk(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
@@ -143,213 +106,105 @@ __global__ __launch_bounds__(256) void k_ras_x2c(int64_t nsef, int64_t ndet, con
   }
 }
 
-template <typename T, int N>
-struct VecN;
-template <>
-struct VecN<float, 4> {
-  typedef float type __attribute__((ext_vector_type(4)));
-};
-template <>
-struct VecN<double, 2> {
-  typedef double type __attribute__((ext_vector_type(2)));
-};
+// Pair table of the compact products (built once): per block and variant the
+// nqp pairs as p | r << 8 and their positions in the full product's list, -1
+// for padding.
+__global__ __launch_bounds__(64) void k_ras_pairs(const RasView* __restrict__ vp, int bi, int16_t* __restrict__ pr,
+                                                  int16_t* __restrict__ pos) {
+  const RasView& v = *vp;
+  const RasCmp& C = v.cmp[bi];
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= C.nvar) return;
+  int64_t oi = C.level == 0 ? 0 : g, ii = 0;
+  if (C.level == 2) {
+    if (C.tri) {
+      ras_tri_uw(g, C.nIo, oi, ii);
+    } else {
+      oi = g / C.nIi;
+      ii = g % C.nIi;
+    }
+  }
+  uint64_t op, ir;
+  ras_cmp_drop(v, C, oi, ii, op, ir);
+  const int16_t* __restrict__ px = v.pidx + (int64_t)((C.kind ? 1 : 0) * (v.m + 1) + C.budget) * v.nbf * v.nbf;
+  ras_cmp_pairs(v, C, op, ir, [&](int j, int p, int r) {
+    if (j >= C.nq) return;
+    pr[g * C.nqp + j] = (int16_t)(p | (r << 8));
+    pos[g * C.nqp + j] = px[p * v.nbf + r];
+  });
+  for (int j = C.nq; j < C.nqp; ++j) pr[g * C.nqp + j] = pos[g * C.nqp + j] = -1;
+}
+
+// The variants' integral matrices, gathered from the block's full matrix
+// (np x np); zero rows and columns for padding.
+__global__ __launch_bounds__(256) void k_ras_gvar(int64_t gbase, int64_t n, int nqp, int np,
+                                                  const int16_t* __restrict__ pos, const double* __restrict__ full,
+                                                  double* __restrict__ g64, float* __restrict__ g32) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  const int64_t row = e / nqp;  // variant * nqp + p-pair
+  const int i = pos[row], j = pos[row / nqp * nqp + e % nqp];
+  const double x = (i < 0 || j < 0) ? 0.0 : full[(int64_t)i * np + j];
+  g64[gbase + e] = x;
+  g32[gbase + e] = (float)x;
+}
 
 // Signed vector row of every D entry (built once): didx[dbase + row * nqp +
-// j] = 2 det + negative for pair j of block row `row`, the zero row 2 ndet
-// when the pair cannot be added to the row's strings (ras_d_entry) and for
-// the padding rows past nrows (up to a multiple of 16, so that whole tiles
-// read their entries without bounds checks).
-__global__ __launch_bounds__(256) void k_ras_didx(const RasView* __restrict__ vp, int bi, int32_t* __restrict__ didx) {
+// j] = 2 det + negative for live pair j of row `row`, the zero row 2 ndet
+// when the pair cannot be added to the row's strings (ras_d_det).
+__global__ __launch_bounds__(256) void k_ras_didx(const RasView* __restrict__ vp, int bi,
+                                                  const int16_t* __restrict__ pr, int32_t* __restrict__ didx) {
   const RasView& v = *vp;
   const RasBlockDev& B = v.blk[bi];
+  const RasCmp& C = v.cmp[bi];
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (B.nrows + 15) / 16 * 16 * B.nqp) return;
-  const int64_t row = e / B.nqp;
-  const int j = (int)(e % B.nqp);
+  if (e >= C.nrows * C.nqp) return;
+  const int64_t row = e / C.nqp;
+  const int j = (int)(e % C.nqp);
+  int64_t o, i;
+  ras_cmp_unrow(C, row, o, i);
+  const int16_t qs = pr[ras_cmp_var(C, o / C.nEo, i / C.nEi) * C.nqp + j];
+  const int64_t u = C.swap ? C.i0 + i : C.o0 + o, w = C.swap ? C.o0 + o : C.i0 + i;
   int neg = 0;
-  const int64_t det = row < B.nrows ? ras_d_entry(v, B, row, j, neg) : -1;
-  didx[B.dbase + e] = (det < 0 || det >= v.ndet) ? (int32_t)(2 * v.ndet) : (int32_t)(2 * det + neg);
+  const int64_t det = qs < 0 ? -1 : ras_d_det(v, C.kind, C.sector, B.lu, B.lw, u, w, qs & 0xff, (qs >> 8) & 0xff, neg);
+  didx[C.dbase + e] = (det < 0 || det >= v.ndet) ? (int32_t)(2 * v.ndet) : (int32_t)(2 * det + neg);
 }
 
-// One tile of W = D G^T for block bi: PT p-pairs x kMT (row, column)
-// values.  Four wavefronts, each PT p-pairs x 32 values (PT / 16 x 2 MFMA
-// tiles); PT = 64, or the whole (16-padded) pair count when it is at most
-// 112, so that no tile computes rows past it.
-// Per chunk of kQC q-pairs: G[p][q] rows and the D entries (c rows of the
-// determinants in didx) into LDS, then kQC / 4 MFMA steps; the global loads
-// of the next chunk are issued before the MFMA steps of the current one
-// (software pipelining through registers).  Tiles are dealt so that XCD x
-// runs the contiguous tiles [x per, (x + 1) per): the p-tiles of one row
-// tile, which gather the same c rows, share an L2.
-template <typename T, int KC, int PT>
-__global__ __launch_bounds__(256) void k_ras_gemm(const RasBlockDev* __restrict__ blk, int bi,
-                                                  const int32_t* __restrict__ didx, const T* __restrict__ G,
-                                                  const T* __restrict__ c, int32_t zrow, T* __restrict__ W,
-                                                  int64_t ntiles, int npt) {
-  typedef Mfma<T> M;
-  constexpr int kQC = ras_qc<T>();
-  typedef typename M::v4 v4;
-  constexpr int RT = kMT / KC;          // block rows per tile
-  constexpr int DPT = kMT * kQC / 256;        // D values per thread and chunk
-  constexpr int VPT = KC < DPT ? KC : DPT;     // consecutive columns one thread gathers per entry
-  constexpr int CPT = DPT / VPT;               // (row, pair) entries per thread and chunk
-  constexpr int TPC = KC / VPT;                // threads per entry
-  constexpr int GN = (PT * kQC + 255) / 256;   // G values per thread and chunk (at most)
-  constexpr int NI = PT / 16;                  // p-subtiles per wavefront
-  constexpr bool pipe = sizeof(T) == 8 ? PSOCI_RAS_PIPE64 : PSOCI_RAS_PIPE;
-  // row strides of the LDS tiles (compile-time knobs)
-  __shared__ __align__(16) T Gs[PT][kQC + PSOCI_RAS_GPAD];
-  __shared__ __align__(16) T Ds[kQC][kMT + PSOCI_RAS_DPAD];
-  const int64_t per = (ntiles + 7) / 8;
-  const int64_t tile = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (tile >= ntiles) return;  // uniform per workgroup
-  const int64_t mt = tile / npt;
-  const int pt = (int)(tile % npt);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const RasBlockDev& B = blk[bi];
-  const int64_t nrows = B.nrows;
-  const int nqp = B.nqp;
-  const T* __restrict__ Gb = G + B.goff;
-  const int32_t* __restrict__ dx = didx + B.dbase;
-  v4 acc[NI][2];
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = v4{0, 0, 0, 0};
+// One group of rows with its matrix, and its first tile per chunk width
+// (built on the host; the tile table is written from it).
+struct RasGroup {
+  int64_t g, w, d, rows;
+  int32_t nqp, nq, pt, pad;
+  int64_t tile0[4];
+};
 
-  // per-thread staging of one chunk: G values tid + 256 i (row e / kQC,
-  // pair e % kQC of the tile's G slice), D entries below
-  T gv[GN];
-  T dv[CPT][VPT];
-  // chunks of kQC pairs; nqp is a multiple of 16, so the last chunk may
-  // hold 16: its other half is loaded as zeros
-  auto load = [&](int q0) {
-    const int wq = nqp - q0 < kQC ? nqp - q0 : kQC;
-#pragma unroll
-    for (int i = 0; i < GN; ++i) {
-      const int e = tid + 256 * i, gp = e / kQC, gq = e % kQC, gpg = pt * PT + gp;
-      gv[i] = (e < PT * kQC && gpg < nqp && gq < wq) ? Gb[(int64_t)gpg * nqp + q0 + gq] : (T)0;
-    }
-#pragma unroll
-    for (int ci = 0; ci < CPT; ++ci) {
-      const int ent = (tid / TPC) * CPT + ci;  // (row, pair) entry: rl * kQC + jq
-      const int v0 = (tid % TPC) * VPT;
-      const int rl = ent / kQC, jq = ent % kQC;
-      const int64_t row = mt * RT + rl;
-      // the entry's signed row (the zero row past the block or the pairs)
-      const int32_t e = (row < nrows && jq < wq) ? dx[row * nqp + q0 + jq] : zrow;
-      const T* __restrict__ src = c + (int64_t)e * KC + v0;
-      if constexpr (VPT * sizeof(T) % 16 == 0) {
-        typedef typename VecN<T, 16 / sizeof(T)>::type V;
-        constexpr int W16 = 16 / sizeof(T);
-#pragma unroll
-        for (int i = 0; i < VPT / W16; ++i) {
-          const V x = reinterpret_cast<const V*>(src)[i];
-#pragma unroll
-          for (int w = 0; w < W16; ++w) dv[ci][i * W16 + w] = x[w];
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) dv[ci][i] = src[i];
-      }
-    }
-  };
-  auto store = [&]() {
-    typedef typename VecN<T, 16 / sizeof(T)>::type V;
-    constexpr int W16 = 16 / sizeof(T);
-    constexpr bool vec = PSOCI_RAS_VSTORE && (kMT + PSOCI_RAS_DPAD) % W16 == 0;
-#pragma unroll
-    for (int i = 0; i < GN; ++i) {
-      const int e = tid + 256 * i;
-      if (e < PT * kQC) Gs[e / kQC][e % kQC] = gv[i];
-    }
-#pragma unroll
-    for (int ci = 0; ci < CPT; ++ci) {
-      const int ent = (tid / TPC) * CPT + ci;
-      const int v0 = (tid % TPC) * VPT;
-      const int rl = ent / kQC, jq = ent % kQC;
-      if constexpr (vec && VPT % W16 == 0) {
-#pragma unroll
-        for (int i = 0; i < VPT / W16; ++i) {
-          V x;
-#pragma unroll
-          for (int w = 0; w < W16; ++w) x[w] = dv[ci][i * W16 + w];
-          *reinterpret_cast<V*>(&Ds[jq][rl * KC + v0 + i * W16]) = x;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) Ds[jq][rl * KC + v0 + i] = dv[ci][i];
-      }
-    }
-  };
-  if (pipe) {
-    load(0);
-    store();
-    __syncthreads();
+// Tiles of every group for one chunk width (rt rows per tile): row tiles
+// major, the p-tiles that gather the same c rows next to each other.
+__global__ __launch_bounds__(64) void k_ras_tiles(const RasGroup* __restrict__ grp, int which, int rt,
+                                                  RasTile* __restrict__ out) {
+  const RasGroup G = grp[blockIdx.x];
+  const int npt = (G.nqp + G.pt - 1) / G.pt;
+  const int64_t n = (G.rows + rt - 1) / rt * npt;
+  for (int64_t t = threadIdx.x; t < n; t += blockDim.x) {
+    const int64_t r0 = t / npt * rt;
+    const int p0 = (int)(t % npt) * G.pt;
+    const int left = G.nq - p0 < G.pt ? G.nq - p0 : G.pt;
+    RasTile T;
+    T.g = G.g;
+    T.w = G.w + r0 * G.nqp;
+    T.d = G.d + r0 * G.nqp;
+    T.nqp = G.nqp;
+    T.p0 = (uint16_t)p0;
+    T.nrows = (uint8_t)(G.rows - r0 < rt ? G.rows - r0 : rt);
+    T.niv = (uint8_t)((left + 15) / 16);
+    out[G.tile0[which] + t] = T;
   }
-  for (int q0 = 0; q0 < nqp; q0 += kQC) {
-    const bool more = q0 + kQC < nqp;
-    if (pipe) {
-      if (more) load(q0 + kQC);  // in flight during the MFMA steps below
-    } else {
-      load(q0);
-      store();
-      __syncthreads();
-    }
-#pragma unroll
-    for (int kk = 0; kk < kQC / 4; ++kk) {
-      T a[NI], b[2];
-#pragma unroll
-      for (int i = 0; i < NI; ++i) a[i] = Gs[16 * i + (lane & 15)][4 * kk + (lane >> 4)];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = Ds[4 * kk + (lane >> 4)][32 * wave + 16 * j + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = M::op(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-    if (pipe) {
-      if (more) store();
-      __syncthreads();
-    }
-  }
-  const int64_t wb = B.wbase;
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int m = 32 * wave + 16 * j + (lane & 15);
-      const int64_t row = mt * RT + m / KC;
-      const int vq = m % KC;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int p = pt * PT + 16 * i + M::row(t, lane);
-        if (row < nrows && p < nqp) W[(wb + row * nqp + p) * KC + vq] = acc[i][j][t];
-      }
-    }
 }
 
-// The 16- and 8-column product with its operands copied straight from global
-// memory into LDS (global_load_lds_dwordx4: each lane names its own 16-byte
-// source, the wavefront's 64 pieces land contiguously at one LDS address),
-// into two LDS stages: the copies of chunk n + 1 are in flight while the
-// MFMA steps consume chunk n, with one barrier per chunk and no staging
-// registers.  Layouts in LDS:
-//   G stage [q][PT] -- q-pair rows of the tile's p-pairs, read from G's q
-//     rows (G is symmetric, so row q holds column q); at FP32 the 16-byte
-//     pieces of odd rows swap halves of every 128 bytes when PT / 16 is even,
-//     which keeps the two rows one 32-lane operand read touches in separate
-//     banks;
-//   D stage [row][q][KC] -- one KC-value piece per (row, pair) entry, copied
-//     from the entry's signed row of c (the zero row for a missing
-//     determinant or a padding row), so no arithmetic touches the operands
-//     between the copy and the MFMA; wave w copies and reads only its own
-//     rows of the tile (2w, 2w + 1 at 16 columns; 4w .. 4w + 3 at 8).
-// wavefronts per SIMD the LDS-copy product is compiled for (a register
-// budget: the compiler would otherwise hold more k-steps' operands in flight
-// than occupancy can afford; at FP32 and 64 p-pairs the budget of 6 spills a
-// few set-up values outside the chunk loop, measured 2 % faster than 5)
+// wavefronts per SIMD the product is compiled for (a register budget: the
+// compiler would otherwise hold more k-steps' operands in flight than
+// occupancy can afford; at FP32 and 64 p-pairs the budget of 6 spills a few
+// set-up values outside the chunk loop, measured 2 % faster than 5)
 template <typename T, int PT>
 constexpr int ras_lds_waves() {
   return sizeof(T) == 8 ? (PT <= 64 ? 3 : 2) : (PT <= 64 ? 6 : 4);
@@ -362,7 +217,7 @@ struct IntC {
 
 // 16 bytes from this lane's global address to LDS at byte address lds + 16
 // * lane (lds uniform over the wavefront); completion is counted by vmcnt.  Written as
-// an asm statement so that the compiler, which cannot tell the two LDS
+// asm statements so that the compiler, which cannot tell the two LDS
 // stages apart, does not wait for every copy in flight before each LDS read:
 // the kernel waits for its copies itself (vmcnt(0) before the barrier that
 // publishes a stage).  M0 carries the LDS address; nothing else in the
@@ -370,158 +225,132 @@ struct IntC {
 __device__ __forceinline__ void lds_copy16(const void* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
 }
+// the same from a uniform base plus this lane's byte offset
+__device__ __forceinline__ void lds_copy16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
 // LDS byte address of a __shared__ location, uniform over the wavefront
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p);
 }
 
-template <typename T, int KC, int PT, int QC = 16, int WPE = ras_lds_waves<T, PT>()>
+// The products: one workgroup per tile (PT p-pairs x 128 (row, column)
+// values; RasTile), four wavefronts of PT x 32 values (PT / 16 x 2 MFMA
+// tiles).  Operands are copied straight from global memory into LDS
+// (global_load_lds_dwordx4: each lane names its own 16-byte source, the
+// wavefront's 64 pieces land contiguously at one LDS address), into two LDS
+// stages: the copies of chunk n + 1 are in flight while the MFMA steps
+// consume chunk n, with one barrier per chunk and no staging registers.
+// Layouts in LDS:
+//   G stage [q][PT] -- q-pair rows of the tile's p-pairs, read from G's q
+//     rows (G is symmetric, so row q holds column q); at FP32 the 16-byte
+//     pieces of odd rows swap halves of every 128 bytes when PT / 16 is even,
+//     which keeps the two rows one 32-lane operand read touches in separate
+//     banks;
+//   D stage [wavefront][q][32] -- the wavefront's rows x KC columns for each
+//     q (the halves of 16 swapped for odd q, for the same reason), each
+//     (row, q) entry copied from its signed row of c (the zero row for a
+//     missing determinant), so no arithmetic touches the operands between
+//     the copy and the MFMA; one layout for every KC whose row of c is a
+//     whole number of 16-byte pieces (narrower blocks run at 4 FP32 or 2
+//     FP64 columns).
+// A tile's rows past its group's last repeat that row (not stored).  The
+// chunk loop is unrolled over the two stages, so every LDS address is a
+// constant offset, and the matrix and index addresses advance in scalar
+// registers.
+// One launch covers every block of one tile width PT (27 blocks on 10 + 24
+// orbitals, 8 electrons: 5 launches instead of 27), heavy tiles first; tiles
+// are dealt to the 8 XCDs in runs of 2^sh, so that the tiles of a row group
+// (the same c rows and matrix) share an L2.
+template <typename T, int KC, int PT, int WPE = ras_lds_waves<T, PT>()>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE)))
-void k_ras_gemm_lds(const RasBlockDev* __restrict__ blk, int bi, const int32_t* __restrict__ didx,
-                    const T* __restrict__ G, const T* __restrict__ c, int32_t zrow, T* __restrict__ W, int64_t ntiles,
-                    int npt, const uint64_t* __restrict__ qm, const uint64_t* __restrict__ smask) {
+void k_ras_gemm(const RasTile* __restrict__ tiles, int64_t ntiles, int sh, const int32_t* __restrict__ didx,
+                const T* __restrict__ G, const T* __restrict__ c, T* __restrict__ W) {
   typedef Mfma<T> M;
   typedef typename M::v4 v4;
-  static_assert(KC == 8 || KC == 16, "8 or 16 columns");
-  static_assert(QC == 16 || QC == 32, "chunks of 16 or 32 pairs");
-  constexpr int RT = kMT / KC;           // 8 or 16 block rows per tile
+  constexpr int RT = kMT / KC;           // rows per tile
   constexpr int RW = RT / 4;             // rows per wavefront
   constexpr int NI = PT / 16;            // p-subtiles per wavefront
   constexpr int SL = 16 / sizeof(T);     // values per 16-byte piece
   constexpr int SPE = KC / SL;           // pieces per D entry
-  constexpr int EPI = 64 / SPE;          // D entries per copy instruction
-  constexpr int DI = RW * QC / EPI;      // D copies per wavefront and chunk
+  constexpr int DI = 32 * kQC / (64 * SL);  // D copies per wavefront and chunk
   constexpr int GSR = PT / SL;           // pieces per G row
-  constexpr int GI = QC * GSR / 64;      // G copies per chunk
+  constexpr int GI = kQC * GSR / 64;     // G copies per chunk
   constexpr int GW = (GI + 3) / 4;       // G copies per wavefront (at most)
   constexpr bool SWZ = sizeof(T) == 4 && (PT / 16) % 2 == 0;
-  static_assert(QC * GSR % 64 == 0 && RW * QC % EPI == 0, "copy shapes");
-  __shared__ __align__(16) T Gs[2][QC * PT];
-  __shared__ __align__(16) T Ds[2][RT * QC * KC];
-  const int64_t per = (ntiles + 7) / 8;
-  const int64_t tile = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (tile >= ntiles) return;  // uniform per workgroup
-  const int64_t mt = tile / npt;
-  const int pt = (int)(tile % npt);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const RasBlockDev& B = blk[bi];
-  const int64_t nrows = B.nrows;
-  // chunks of QC pairs; with QC = 32 the last one may hold 16 (nqp is a
-  // multiple of 16): its other half reads the zero row and G row nqp - 1
-  const int nqp = B.nqp, nch = (nqp + QC - 1) / QC;
+  static_assert(KC % SL == 0 && RW >= 2 && kQC * GSR % 64 == 0, "copy shapes");
+  __shared__ __align__(16) T Gs[2][kQC * PT];
+  __shared__ __align__(16) T Ds[2][kQC * kMT];
+  const int64_t b = blockIdx.x >> 3;
+  const int64_t ti = ((((b >> sh) << 3) + (blockIdx.x & 7)) << sh) + (b & ((1 << sh) - 1));
+  if (ti >= ntiles) return;  // uniform per workgroup
+  const RasTile tile = tiles[ti];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nrows = tile.nrows, nqp = tile.nqp, p0 = tile.p0, niv = tile.niv;
+  const int nch = nqp / kQC;
 
-  // this lane's sources as offsets advanced by one chunk per step: its D
-  // entries in the index table (rows padded to whole tiles: no bounds
-  // checks) and its G pieces (rows q of G's symmetric tile; a piece past nqp
-  // repeats its row's first, feeding only output rows that are not stored)
-  const int32_t* __restrict__ dx = didx + B.dbase;
-  const T* __restrict__ Gb = G + B.goff;
-  int dxo[DI];
+  // this lane's sources: its D entries' offsets in the index table and its G
+  // pieces' byte offsets, both from bases that advance by a chunk (a G piece
+  // past nqp repeats its row's first, feeding only output rows that are not
+  // stored)
+  const int32_t* __restrict__ dx = didx + tile.d;
+  const T* __restrict__ Gb = G + tile.g + p0;
+  uint32_t dxo[DI];
 #pragma unroll
   for (int d = 0; d < DI; ++d) {
-    const int en = d * EPI + lane / SPE;  // entry among the wavefront's RW x QC
-    dxo[d] = (int)((mt * RT + RW * wave + en / QC) * nqp + en % QC);
+    const int slot = d * 64 + lane;
+    const int q = slot / (SPE * RW), r = ((slot / SPE) % RW) ^ ((q & 1) * (RW / 2));
+    const int row = RW * wave + r;
+    dxo[d] = (uint32_t)((row < nrows ? row : nrows - 1) * nqp + q);
   }
-  int go[GW];
+  uint32_t go[GW];
 #pragma unroll
   for (int gi = 0; gi < GW; ++gi) {
     const int sl = 64 * (wave + 4 * gi) + lane, k = sl / GSR;
     const int r = SWZ ? (sl % GSR) ^ (4 * (k & 1)) : sl % GSR;
-    const int p = pt * PT + r * SL;
-    go[gi] = k * nqp + (p < nqp ? p : 0);
+    go[gi] = (uint32_t)((k * nqp + (p0 + r * SL < nqp ? r * SL : 0)) * sizeof(T));
   }
-  const int v0 = SL * (lane % SPE);
+  const T* __restrict__ cl = c + SL * (lane % SPE);
   // LDS addresses of this wavefront's first D copy and first G copy (stage 0)
-  const uint32_t dl0 = lds_addr(&Ds[0][RW * wave * QC * KC]);
+  const uint32_t dl0 = lds_addr(&Ds[0][32 * kQC * wave]);
   const uint32_t gl0 = lds_addr(&Gs[0][64 * wave * SL]);
-  auto fetch_idx = [&](int ch, int32_t (&ix)[DI]) {
+  auto fetch_idx = [&](int32_t (&ix)[DI]) {
 #pragma unroll
-    for (int d = 0; d < DI; ++d) {
-      if (QC == 16 || ch * QC + (d * EPI + lane / SPE) % QC < nqp) ix[d] = dx[dxo[d] + ch * QC];
-      else ix[d] = zrow;
-    }
+    for (int d = 0; d < DI; ++d) ix[d] = dx[dxo[d]];
+    dx += kQC;
   };
-  // the copies of chunk ch into stage st: D pieces first (they use the
-  // indices loaded a chunk earlier, which the compiler waits for), then G
-  auto issue = [&](int ch, int st, const int32_t (&ix)[DI]) {
+  // the copies of the next chunk into stage ST: D pieces first (they use the
+  // indices loaded a chunk earlier), then G
+  auto issue = [&](auto stc, const int32_t (&ix)[DI]) {
+    constexpr int ST = decltype(stc)::value;
     // every source address is formed (its index load waited for) before
     // the first copy issues: a wait for an index load placed between two
     // copies would also wait for the copy before it
     const T* src[DI];
 #pragma unroll
-    for (int d = 0; d < DI; ++d) src[d] = c + (int64_t)ix[d] * KC + v0;
+    for (int d = 0; d < DI; ++d) src[d] = cl + (uint64_t)(uint32_t)ix[d] * KC;
 #pragma unroll
     for (int d = 0; d < DI; ++d) asm volatile("" : "+v"(src[d]));
 #pragma unroll
     for (int d = 0; d < DI; ++d)
-      lds_copy16(src[d], dl0 + (uint32_t)((st * RT * QC * KC + d * EPI * KC) * sizeof(T)));
-    const int q0 = ch * QC;
+      lds_copy16(src[d], dl0 + (uint32_t)((ST * kQC * kMT + d * 64 * SL) * sizeof(T)));
 #pragma unroll
     for (int gi = 0; gi < GW; ++gi) {
       if (wave + 4 * gi >= GI) continue;
-      const int k = (64 * (wave + 4 * gi) + lane) / GSR;  // row of the chunk
-      const int qo = (QC == 16 || q0 + k < nqp) ? q0 * nqp : (nqp - 1 - k) * nqp;
-      lds_copy16(Gb + (go[gi] + qo), gl0 + (uint32_t)((st * QC * PT + 64 * 4 * gi * SL) * sizeof(T)));
+      lds_copy16(Gb, go[gi], gl0 + (uint32_t)((ST * kQC * PT + 64 * 4 * gi * SL) * sizeof(T)));
     }
+    Gb += (int64_t)kQC * nqp;
   };
 
   // lane offsets of the MFMA operand reads (k row kr = lane / 16 within a
   // step): p-subtile i of G sits at a0[i & 1] + 16 i (with the swap of
-  // 64-byte halves on odd rows: 16 (i ^ 1) = 16 i -+ 16); the B operand's
-  // column lane & 15 is value vl of row RW wave + rl (+ 16 j / KC for
-  // subtile j)
-  const int kr = lane >> 4;
+  // 64-byte halves on odd rows: 16 (i ^ 1) = 16 i -+ 16); value subtile j of
+  // D at b0[j] (its halves swapped on odd rows)
+  const int kr = lane >> 4, l15 = lane & 15;
   const int sw = SWZ ? 16 * (kr & 1) : 0;
-  const int a0[2] = {kr * PT + (lane & 15) + sw, kr * PT + (lane & 15) - sw};
-  const int rl = (lane & 15) / KC, vl = (lane & 15) % KC;
-  const int boff = ((RW * wave + rl) * QC + kr) * KC + vl;
-  // pairs past nq are padding (zero G rows and columns, zero D entries): a
-  // tile's last p-subtiles that hold only padding are skipped
-  const int nq = B.nq;
-  const int niv = ((nq - pt * PT < PT ? nq - pt * PT : PT) + 15) / 16;
-  // chunks with only zero D entries are skipped: when every row of the tile
-  // has the same first string u (alpha-beta and alpha-alpha products, rows
-  // u-major), a chunk whose pairs all add an orbital u holds (bit of qm not
-  // in u's mask) contributes nothing.  live[0..1]: bits of the first 128
-  // chunks (later ones are always live); uniform over the workgroup.
-  uint64_t live[2] = {~0ull, ~0ull};
-  if (B.kind != 2) {
-    const int64_t r0 = mt * RT, r1 = (r0 + RT < nrows ? r0 + RT : nrows) - 1;
-    int64_t ua, ub, wdum;
-    if (B.tri) {
-      ras_tri_uw(r0, B.nu, ua, wdum);
-      ras_tri_uw(r1, B.nu, ub, wdum);
-    } else {
-      ua = r0 / B.nw;
-      ub = r1 / B.nw;
-    }
-    if (ua == ub) {
-      const uint64_t um = smask[B.umoff + B.u0 + ua];
-      constexpr int H = QC / 16;  // 16-pair pieces of a chunk (qm is per piece)
-      for (int ch = 0; ch < nch && ch < 128; ++ch) {
-        bool dead = true;
-        for (int h = 0; h < H; ++h)
-          if (ch * H + h < nqp / 16 && (qm[B.qmoff + ch * H + h] & ~um) != 0) dead = false;
-        if (dead) live[ch >> 6] &= ~(1ull << (ch & 63));
-      }
-    }
-  }
-  // first live chunk after chunk x (nch when none): a find-first-set on
-  // the masks (bits past nch are set)
-  auto next_live = [&](int x) {
-    int y = x + 1;
-    if (y < 64) {
-      const uint64_t m = live[0] >> y;
-      if (m) return min(y + (int)__builtin_ctzll(m), nch);
-      y = 64;
-    }
-    if (y < 128) {
-      const uint64_t m = live[1] >> (y - 64);
-      if (m) return min(y + (int)__builtin_ctzll(m), nch);
-      y = 128;
-    }
-    return min(y, nch);
-  };
+  const int a0[2] = {kr * PT + l15 + sw, kr * PT + l15 - sw};
+  const int b0[2] = {32 * (kQC * wave + kr) + l15 + 16 * (kr & 1), 32 * (kQC * wave + kr) + l15 + 16 - 16 * (kr & 1)};
 
   // the whole tile with NV live p-subtiles
   auto run = [&](auto nvc) {
@@ -531,60 +360,54 @@ void k_ras_gemm_lds(const RasBlockDev* __restrict__ blk, int bi, const int32_t* 
     for (int i = 0; i < NV; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = v4{0, 0, 0, 0};
-    // one k-step of 4 pairs on stage st
-    auto step = [&](int st, int kk) {
-      const T* __restrict__ gs = Gs[st];
-      const T* __restrict__ ds = Ds[st];
-      T a[NV], b[2];
+    int32_t ixn[DI];
+    fetch_idx(ixn);
+    issue(IntC<0>{}, ixn);
+    if (nch > 1) fetch_idx(ixn);
+    // one chunk on stage ST; `left` chunks follow
+    auto chunk = [&](auto stc, int left) {
+      constexpr int ST = decltype(stc)::value;
+      // this wavefront's copies of the chunk have landed, every wavefront's
+      // have after the barrier, and the other stage is free (its reads ended
+      // before the barrier)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (left > 0) {
+        issue(IntC<1 - ST>{}, ixn);
+        if (left > 1) fetch_idx(ixn);
+      }
+      const T* __restrict__ gs = Gs[ST];
+      const T* __restrict__ ds = Ds[ST];
 #pragma unroll
-      for (int i = 0; i < NV; ++i) a[i] = gs[a0[i & 1] + 16 * i + 4 * kk * PT];
+      for (int kk = 0; kk < kQC / 4; ++kk) {
+        T a[NV], bb[2];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = ds[boff + (16 / KC * j * QC + 4 * kk) * KC];
+        for (int i = 0; i < NV; ++i) a[i] = gs[a0[i & 1] + 16 * i + 4 * kk * PT];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bb[j] = ds[b0[j] + 4 * kk * 32];
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = M::op(a[i], bb[j], acc[i][j]);
+      }
+    };
+    for (int left = nch - 1; left >= 0; left -= 2) {
+      chunk(IntC<0>{}, left);
+      if (left > 0) chunk(IntC<1>{}, left - 1);
+    }
+    T* __restrict__ Wt = W + tile.w * KC;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int m = 16 * j + l15, row = RW * wave + m / KC;
+      if (row >= nrows) continue;
 #pragma unroll
       for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = M::op(a[i], b[j], acc[i][j]);
-    };
-    // the live chunks in order: c0 (in the stage being read), c1 (copies in
-    // flight), c2 (indices in flight)
-    int32_t ixn[DI];
-    int c0 = next_live(-1);
-    int c1 = c0 < nch ? next_live(c0) : nch;
-    int c2 = c1 < nch ? next_live(c1) : nch;
-    if (c0 < nch) {
-      fetch_idx(c0, ixn);
-      issue(c0, 0, ixn);
-      if (c1 < nch) fetch_idx(c1, ixn);
-    }
-    for (int it = 0; c0 < nch; ++it) {
-      const int st = it & 1;
-      // this wavefront's copies of chunk c0 have landed, every wavefront's
-      // have after the barrier, and stage st ^ 1 is free (its reads of the
-      // chunk before ended before the barrier)
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (c1 < nch) {
-        issue(c1, st ^ 1, ixn);
-        if (c2 < nch) fetch_idx(c2, ixn);
-      }
-#pragma unroll
-      for (int kk = 0; kk < QC / 4; ++kk) step(st, kk);
-      c0 = c1;
-      c1 = c2;
-      c2 = c2 < nch ? next_live(c2) : nch;
-    }
-    const int64_t wb = B.wbase;
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int64_t row = mt * RT + RW * wave + 16 / KC * j + rl;
-#pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const int p = pt * PT + 16 * i + M::row(t, lane);
-          if (row < nrows && p < nqp) W[(wb + row * nqp + p) * KC + vl] = acc[i][j][t];
+          const int p = p0 + 16 * i + M::row(t, lane);
+          if (p < nqp) Wt[(row * nqp + p) * KC + m % KC] = acc[i][j][t];
         }
-      }
+    }
   };
   // tiles cover the pairs exactly except, for some widths, the last one
   if (niv >= NI) {
@@ -750,57 +573,37 @@ void ras_chunk(Ctx& c, const TIO* X, int ldx, TIO* Y, int ldy, int col0, int kw,
                      c.d_rasrows.p, X, ldx, col0, kw, cv);
   PSOCI_HIP(hipGetLastError());
   if (tm) tm->mark(c.stream, 0);
-  for (int bi = 0; bi < (int)P.blk.size(); ++bi) {
-    const RasBlockDev& B = P.blk[bi];
-    const int pt_w = ras_tile_width(B.nqp);
-    const int npt = (B.nqp + pt_w - 1) / pt_w;
-    const int64_t nmt = (B.nrows * KC + kMT - 1) / kMT;
-    const int64_t ntiles = nmt * npt;
-    const unsigned grid = (unsigned)(8 * ((ntiles + 7) / 8));
-    const RasBlockDev* blk = c.d_rasblk.p;
-    const int32_t* didx = c.d_rasdidx.p;
-    const int32_t zrow = (int32_t)(2 * P.ndet);  // the zero row of c
-    const uint64_t* qm = c.d_rasqm.p;
-    const uint64_t* smask = c.d_rasmask.p;
-    if constexpr ((KC == 16 || KC == 8) && PSOCI_RAS_DMA) {
-      constexpr int LQC = sizeof(T) == 4 && PSOCI_RAS_LQC32 ? 32 : 16;
-      switch (pt_w) {
-#define PSOCI_RAS_GEMML(PTV)                                                                                    \
-  case PTV:                                                                                                    \
-    hipLaunchKernelGGL((k_ras_gemm_lds<T, KC, PTV, LQC>), dim3(grid), dim3(256), 0, c.stream, blk, bi, didx, G, cv, \
-                       zrow, W, ntiles, npt, qm, smask);                                                       \
-    break;
-        PSOCI_RAS_GEMML(16)
-        PSOCI_RAS_GEMML(32)
-        PSOCI_RAS_GEMML(48)
-        PSOCI_RAS_GEMML(80)
-        PSOCI_RAS_GEMML(96)
-        PSOCI_RAS_GEMML(112)
-#undef PSOCI_RAS_GEMML
-        default:
-          hipLaunchKernelGGL((k_ras_gemm_lds<T, KC, 64, LQC>), dim3(grid), dim3(256), 0, c.stream, blk, bi, didx, G,
-                             cv, zrow, W, ntiles, npt, qm, smask);
-      }
-    } else
-    switch (pt_w) {
-#define PSOCI_RAS_GEMM(PTV)                                                                                  \
-  case PTV:                                                                                                 \
-    hipLaunchKernelGGL((k_ras_gemm<T, KC, PTV>), dim3(grid), dim3(256), 0, c.stream, blk, bi, didx, G, cv, zrow, \
-                       W, ntiles, npt);                                                                     \
+  constexpr int ki = KC == 16 ? 0 : KC == 8 ? 1 : KC == 4 ? 2 : 3;
+  const std::vector<RasLaunch>& L = c.ras_launch[ki];
+  for (size_t i = 0; i < L.size();) {
+    // every kind of one tile width in one launch; a timed sigma times them
+    // one by one
+    size_t e = i + 1;
+    int64_t nt = L[i].ntiles;
+    for (; !tm && e < L.size() && L[e].pt == L[i].pt; ++e) nt += L[e].ntiles;
+    int sh = 5;  // runs of 32 tiles per XCD, shorter where they would leave XCDs idle
+    while (sh > 0 && nt < (int64_t)8 * 8 << sh) --sh;
+    const unsigned grid = (unsigned)(((nt + ((int64_t)8 << sh) - 1) >> (sh + 3)) << (sh + 3));
+    const RasTile* tiles = c.d_rastile[ki].p + L[i].tile0;
+    switch (L[i].pt) {
+#define PSOCI_RAS_GEMM(PTV)                                                                                     \
+  case PTV:                                                                                                     \
+    hipLaunchKernelGGL((k_ras_gemm<T, KC, PTV>), dim3(grid), dim3(256), 0, c.stream, tiles, nt, sh, c.d_rasdidx.p, \
+                       G, cv, W);                                                                               \
     break;
       PSOCI_RAS_GEMM(16)
       PSOCI_RAS_GEMM(32)
       PSOCI_RAS_GEMM(48)
+      PSOCI_RAS_GEMM(64)
       PSOCI_RAS_GEMM(80)
       PSOCI_RAS_GEMM(96)
       PSOCI_RAS_GEMM(112)
 #undef PSOCI_RAS_GEMM
-      default:
-        hipLaunchKernelGGL((k_ras_gemm<T, KC, 64>), dim3(grid), dim3(256), 0, c.stream, blk, bi, didx, G, cv, zrow,
-                           W, ntiles, npt);
+      default: throw Error(PSOCI_ERR_STATE, "string-driven sigma: no product of this tile width");
     }
     PSOCI_HIP(hipGetLastError());
-    if (tm) tm->mark(c.stream, 1 + B.kind);
+    if (tm) tm->mark(c.stream, 1 + L[i].kind);
+    i = e;
   }
   hipLaunchKernelGGL((k_ras_y<T, KC, TIO>), dim3(nblk(nsef * KC, 256)), dim3(256), 0, c.stream, c.d_rastoff.p,
                      c.d_rasterm.p, c.d_rasscl.p, W, nsef, Y, ldy, col0, kw);
@@ -818,13 +621,68 @@ void ras_any_k(Ctx& c, int k, const TIO* X, int ldx, TIO* Y, int ldy, RasTiming*
     if (kw > 8)
       ras_chunk<T, 16, TIO>(c, X, ldx, Y, ldy, c0, kw, tm);
     else if (kw > 4) ras_chunk<T, 8, TIO>(c, X, ldx, Y, ldy, c0, kw, tm);
-    else if (kw > 2) ras_chunk<T, 4, TIO>(c, X, ldx, Y, ldy, c0, kw, tm);
-    else if (kw > 1) ras_chunk<T, 2, TIO>(c, X, ldx, Y, ldy, c0, kw, tm);
-    else ras_chunk<T, 1, TIO>(c, X, ldx, Y, ldy, c0, kw, tm);
+    else if (kw > 2 || sizeof(T) == 4) ras_chunk<T, 4, TIO>(c, X, ldx, Y, ldy, c0, kw, tm);
+    else if constexpr (sizeof(T) == 8) ras_chunk<T, 2, TIO>(c, X, ldx, Y, ldy, c0, kw, tm);
   }
 }
 
 }  // namespace
+
+// Groups of every block, ordered by (tile width, kind, pairs descending), and
+// the tile table and launches of each chunk width (16, 8, 4 and, for FP64, 2
+// columns).
+static void ras_tile_tables(Ctx& c) {
+  const RasPlan& P = c.ras;
+  std::vector<int> order;
+  for (int bi = 0; bi < (int)P.cmp.size(); ++bi)
+    if (P.cmp[bi].nq > 0) order.push_back(bi);
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    const RasCmp &A = P.cmp[x], &B = P.cmp[y];
+    const int pa = ras_tile_width(A.nqp), pb = ras_tile_width(B.nqp);
+    if (pa != pb) return pa > pb;
+    if (A.kind != B.kind) return A.kind < B.kind;
+    return A.nqp > B.nqp;
+  });
+  std::vector<RasGroup> grp;
+  int64_t nt[4] = {0, 0, 0, 0};
+  for (int k = 0; k < 4; ++k) c.ras_launch[k].clear();
+  for (int bi : order) {
+    const RasCmp& C = P.cmp[bi];
+    const int pt = ras_tile_width(C.nqp), npt = (C.nqp + pt - 1) / pt;
+    for (int k = 0; k < 4; ++k)
+      if (c.ras_launch[k].empty() || c.ras_launch[k].back().pt != pt || c.ras_launch[k].back().kind != C.kind)
+        c.ras_launch[k].push_back(RasLaunch{pt, C.kind, nt[k], 0});
+    ras_cmp_groups(C, [&](int64_t g, int64_t r0, int64_t rows) {
+      RasGroup R;
+      R.g = C.gbase + g * C.nqp * C.nqp;
+      R.w = C.wbase + r0 * C.nqp;
+      R.d = C.dbase + r0 * C.nqp;
+      R.rows = rows;
+      R.nqp = C.nqp;
+      R.nq = C.nq;
+      R.pt = pt;
+      R.pad = 0;
+      for (int k = 0; k < 4; ++k) {
+        const int rt = kMT / (16 >> k);
+        const int64_t n = (rows + rt - 1) / rt * npt;
+        R.tile0[k] = nt[k];
+        nt[k] += n;
+        c.ras_launch[k].back().ntiles += n;
+      }
+      grp.push_back(R);
+    });
+  }
+  DevBuf<RasGroup> dg;
+  dg.upload(grp, c.stream);
+  for (int k = 0; k < 4; ++k) {
+    c.d_rastile[k].alloc(nt[k]);
+    if (grp.empty()) continue;
+    hipLaunchKernelGGL(k_ras_tiles, dim3((unsigned)grp.size()), dim3(64), 0, c.stream, dg.p, k, kMT / (16 >> k),
+                       c.d_rastile[k].p);
+    PSOCI_HIP(hipGetLastError());
+  }
+  c.sync();
+}
 
 // Builds the string plan and its device tables; false (c.ras_why says why)
 // when the space does not qualify.
@@ -850,13 +708,13 @@ bool build_ras(Ctx& c) {
         const RasSectorDev& S = P.sec[e.sec[d]];
         terms += (int64_t)S.na * S.nb + (int64_t)S.na * (S.na - 1) / 2 + (int64_t)S.nb * (S.nb - 1) / 2;
       }
-    const double need = (double)P.wunit * 64 + (double)P.dunit * 4 + (double)P.ndet * 128 + (double)terms * 4 +
-                        (double)P.sef.size() * 9;
+    const double need = (double)P.cwunit * 64 + (double)P.cdunit * 4 + (double)P.cgunit * 12 + (double)P.ndet * 128 +
+                        (double)terms * 4 + (double)P.sef.size() * 9;
     size_t fr = 0, tot = 0;
     PSOCI_HIP(hipMemGetInfo(&fr, &tot));
     // FP64 in chunks of 16 columns (whole 128-byte W and c pieces) when W and
     // c fit twice over in 60 % of the free memory, else chunks of 8
-    c.ras_kc64 = need + (double)P.wunit * 64 + (double)P.ndet * 128 <= 0.6 * (double)fr ? 16 : 8;
+    c.ras_kc64 = need + (double)P.cwunit * 64 + (double)P.ndet * 128 <= 0.6 * (double)fr ? 16 : 8;
     if (need > 0.6 * (double)fr) {
       c.ras_why = "needs " + std::to_string((int64_t)(need / 1e9)) + " GB of device memory, " +
                   std::to_string((int64_t)(fr / 1000000000)) + " GB free";
@@ -885,31 +743,50 @@ bool build_ras(Ctx& c) {
   c.d_rasadd.upload(P.add, c.stream);
   c.d_rasrem.upload(P.rem, c.stream);
   c.d_rasblk.upload(P.blk, c.stream);
-  c.d_rasq.upload(P.qlist, c.stream);
-  c.d_rasqm.upload(P.qm, c.stream);
+  c.d_rascmp.upload(P.cmp, c.stream);
   c.d_raspidx.upload(P.pidx, c.stream);
   c.d_rassef.upload(P.sef, c.stream);
-  c.d_rasg64.upload(P.G, c.stream);
-  std::vector<float> g32(P.G.begin(), P.G.end());
-  c.d_rasg32.upload(g32, c.stream);
   RasView v = ras_host_view(P);
   v.mask = c.d_rasmask.p;
   v.cls = c.d_rascls.p;
   v.add = c.d_rasadd.p;
   v.rem = c.d_rasrem.p;
   v.blk = c.d_rasblk.p;
-  v.qlist = c.d_rasq.p;
+  v.qlist = nullptr;
+  v.cmp = c.d_rascmp.p;
+  v.wunit = P.cwunit;
   v.pidx = c.d_raspidx.p;
   v.sef = c.d_rassef.p;
   c.d_rasview.upload(&v, 1, c.stream);
   // determinant vectors and W: 16 FP32 or ras_kc64 FP64 columns per chunk
   c.d_rasc.alloc((size_t)(2 * P.ndet + 2) * (c.ras_kc64 == 16 ? 16 * sizeof(double) : 16 * sizeof(float)));
-  // the D entries' signed rows
-  c.d_rasdidx.alloc(P.dunit);
-  for (int bi = 0; bi < (int)P.blk.size(); ++bi) {
-    const int64_t n = (P.blk[bi].nrows + 15) / 16 * 16 * P.blk[bi].nqp;
-    hipLaunchKernelGGL(k_ras_didx, dim3(nblk(n, 256)), dim3(256), 0, c.stream, c.d_rasview.p, bi, c.d_rasdidx.p);
-    PSOCI_HIP(hipGetLastError());
+  // the compact products' matrices and the D entries' signed rows
+  c.d_rasg64.alloc(P.cgunit);
+  c.d_rasg32.alloc(P.cgunit);
+  c.d_rasdidx.alloc(P.cdunit);
+  {
+    DevBuf<double> full;
+    full.upload(P.G, c.stream);
+    int64_t most = 0;
+    for (const RasCmp& C : P.cmp) most = std::max(most, C.nvar * C.nqp);
+    DevBuf<int16_t> pr, pos;
+    pr.alloc(most);
+    pos.alloc(most);
+    for (int bi = 0; bi < (int)P.cmp.size(); ++bi) {
+      const RasCmp& C = P.cmp[bi];
+      if (C.nq == 0) continue;
+      hipLaunchKernelGGL(k_ras_pairs, dim3(nblk(C.nvar, 64)), dim3(64), 0, c.stream, c.d_rasview.p, bi, pr.p, pos.p);
+      PSOCI_HIP(hipGetLastError());
+      const int64_t ng = C.nvar * C.nqp * C.nqp;
+      hipLaunchKernelGGL(k_ras_gvar, dim3(nblk(ng, 256)), dim3(256), 0, c.stream, C.gbase, ng, C.nqp, P.blk[bi].nqp,
+                         pos.p, full.p + P.blk[bi].goff, c.d_rasg64.p, c.d_rasg32.p);
+      PSOCI_HIP(hipGetLastError());
+      hipLaunchKernelGGL(k_ras_didx, dim3(nblk(C.nrows * C.nqp, 256)), dim3(256), 0, c.stream, c.d_rasview.p, bi, pr.p,
+                         c.d_rasdidx.p);
+      PSOCI_HIP(hipGetLastError());
+    }
+    ras_tile_tables(c);
+    c.sync();
   }
   // the SEF term lists (merged where an SEF's two determinants read the
   // same W elements): count, scan, fill
@@ -943,7 +820,7 @@ bool build_ras(Ctx& c) {
     PSOCI_CHECK(!b, PSOCI_ERR_STATE, "string-driven sigma: inconsistent term lists");
     c.ras_nterm = nterm;
   }
-  c.d_rasw.alloc((size_t)P.wunit * (c.ras_kc64 == 16 ? 16 * sizeof(double) : 16 * sizeof(float)));
+  c.d_rasw.alloc((size_t)P.cwunit * (c.ras_kc64 == 16 ? 16 * sizeof(double) : 16 * sizeof(float)));
   c.sync();
   c.have_ras = true;
   return true;
@@ -985,7 +862,7 @@ void ras_timing(Ctx& c, int prec, int k, int reps, double* ms, double* flops) {
   for (int g = 0; g < 5; ++g) ms[g] = acc[g] / reps;
   if (flops) {
     for (int g = 0; g < 3; ++g) flops[g] = 0.0;
-    for (const RasBlockDev& B : c.ras.blk) flops[B.kind] += 2.0 * (double)B.nrows * B.nq * B.nq * k;
+    for (const RasCmp& C : c.ras.cmp) flops[C.kind] += 2.0 * (double)C.nrows * C.nq * C.nq * k;
   }
 }
 
