@@ -113,13 +113,14 @@ struct Ctx {
   DevBuf<double> d_rasg64;  // the compact products' matrices
   DevBuf<float> d_rasg32;
   DevBuf<RasView> d_rasview;
-  DevBuf<char> d_rasc, d_rasw;  // determinant vectors [2 ndet + 2][16 FP32 | ras_kc64 FP64], W [cwunit][same]
+  DevBuf<char> d_rasc, d_rasw;  // determinant vectors [2 ndet + 1][16 FP32 | ras_kc64 FP64], W [cwunit][same]
   int ras_kc64 = 8;             // FP64 columns per chunk (16 when memory allows, else 8)
-  DevBuf<int32_t> d_rasdidx;    // [cdunit]: signed vector row (2 det + negative) of every D entry
+  DevBuf<int32_t> d_rasdidx;    // [cdunit]: signed vector row (det + negative * ndet) of every D entry
   DevBuf<int64_t> d_rastoff;    // nsef + 1: first term of each SEF
   int64_t ras_nterm = 0;        // terms over all SEFs (after merging mirrored pairs)
   DevBuf<int32_t> d_rasterm;    // signed W offsets (bit 31: negative)
   DevBuf<int8_t> d_rasscl;      // per SEF: 0 1/sqrt(2), 1 sqrt(2), 2 one
+  DevBuf<int32_t> d_rasorder;   // the order the SEFs are walked in (d_rastoff, d_rasscl, d_rasrows follow it)
   DevBuf<int2> d_rasrows;       // per SEF: signed rows of its determinants' coefficients
   void drop_ras() {
     have_ras = ras_tried = false;
@@ -146,6 +147,7 @@ struct Ctx {
     d_rasterm.release();
     d_rasscl.release();
     d_rasrows.release();
+    d_rasorder.release();
   }
 
   // transition Hamiltonian (rows: this list's SEFs; columns: a second

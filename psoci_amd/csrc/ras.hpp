@@ -115,8 +115,10 @@ struct RasBlockDev {
 //            without ii's orbitals.
 // Every group of a block has the same number nq of live pairs (padded to
 // nqp), listed by ras_cmp_pair; each has its own integral matrix ("variant")
-// at gbase + variant * nqp * nqp.  W element (wbase + row * nqp + pair) per
-// column, D index entry dbase + row * nqp + pair.
+// at gbase + variant * nqp * nqp.  D index entry dbase + row * nqp + pair; W
+// element per column wbase + (first row of the group) * nqp + pair * (rows of
+// the group) + row within the group, so that a pair's terms of consecutive
+// rows are consecutive.
 struct RasCmp {
   int level, kind, sector, tri;
   int budget, nq, nqp;
@@ -127,13 +129,16 @@ struct RasCmp {
   int64_t nrows, nvar, gbase, wbase, dbase;
 };
 
-// One tile of a product: nrows rows (the tile's first at the W and D
-// offsets) times p-pairs [p0, p0 + 16 niv) of the group's nqp.
+// One tile of a product: nrows rows (the W and D offsets are the first one's)
+// times p-pairs [p0, p0 + 16 niv) of the group's nqp; niv is the live pairs
+// where nqp <= 64.
 struct RasTile {
   int64_t g, w, d;   // the group's matrix, W per column, D index table
   int32_t nqp;
   uint16_t p0;
   uint8_t nrows, niv;
+  int32_t rows;  // rows of the group (the W stride of a pair)
+  int32_t flip;  // 1: the second wavefront pair takes the larger half of the p-subtiles
 };
 
 // One launch's tiles in the tile table: all of one kind and tile width.
@@ -335,12 +340,31 @@ PSOCI_HD void ras_cmp_pairs(const RasView& v, const RasCmp& C, uint64_t op, uint
     for (; y; y &= y - 1) f(k++, p, ctz(y));
   }
 }
+// first row and rows of the group of cell (oi, ii)
+PSOCI_HD void ras_cmp_group(const RasCmp& C, int64_t oi, int64_t ii, int64_t& r0, int64_t& rows) {
+  if (C.level == 0) {
+    r0 = 0;
+    rows = C.nrows;
+  } else if (C.level == 1) {
+    r0 = ras_cmp_cell(C, oi, C.tri ? oi : 0);
+    rows = (oi + 1 < C.nIo ? ras_cmp_cell(C, oi + 1, C.tri ? oi + 1 : 0) : C.nrows) - r0;
+  } else {
+    r0 = ras_cmp_cell(C, oi, ii);
+    rows = C.tri && oi == ii ? (int64_t)C.nEo * (C.nEo + 1) / 2 : (int64_t)C.nEo * C.nEi;
+  }
+}
+// W offset per column of a group's pair at one of its rows
+PSOCI_HD int64_t ras_cmp_w(const RasCmp& C, int64_t r0, int64_t rows, int64_t row, int pair) {
+  return C.wbase + r0 * C.nqp + pair * rows + (row - r0);
+}
 // W offset per column of pair (p, r) at the block's local strings (u, w)
 PSOCI_HD int64_t ras_cmp_off(const RasView& v, const RasCmp& C, int64_t u, int64_t w, int p, int r) {
   const int64_t o = C.swap ? w : u, i = C.swap ? u : w;
   uint64_t op, ir;
   ras_cmp_drop(v, C, o / C.nEo, i / C.nEi, op, ir);
-  return C.wbase + ras_cmp_row(C, o, i) * C.nqp + ras_cmp_pair(v, C, op, ir, p, r);
+  int64_t r0, rows;
+  ras_cmp_group(C, o / C.nEo, i / C.nEi, r0, rows);
+  return ras_cmp_w(C, r0, rows, ras_cmp_row(C, o, i), ras_cmp_pair(v, C, op, ir, p, r));
 }
 
 // Calls f(block index, W element offset per column (wbase + row * nqp +
@@ -537,26 +561,15 @@ struct RasPlan {
   double cflops_per_col = 0.0;
 };
 
-// rows and first row of every group of a block, in the row order: calls
-// f(variant, first row, rows)
+// every group of a block in the row order: calls f(variant, first row, rows)
 template <class F>
 inline void ras_cmp_groups(const RasCmp& C, F&& f) {
-  if (C.level == 0) {
-    f((int64_t)0, (int64_t)0, C.nrows);
-    return;
-  }
-  for (int64_t oi = 0; oi < C.nIo; ++oi) {
-    if (C.level == 1) {
-      const int64_t r0 = ras_cmp_cell(C, oi, C.tri ? oi : 0);
-      const int64_t r1 = oi + 1 < C.nIo ? ras_cmp_cell(C, oi + 1, C.tri ? oi + 1 : 0) : C.nrows;
-      f(oi, r0, r1 - r0);
-      continue;
+  for (int64_t oi = 0; oi < (C.level == 0 ? 1 : C.nIo); ++oi)
+    for (int64_t ii = C.level == 2 && C.tri ? oi : 0; ii < (C.level == 2 ? C.nIi : 1); ++ii) {
+      int64_t r0, rows;
+      ras_cmp_group(C, oi, ii, r0, rows);
+      f(ras_cmp_var(C, oi, ii), r0, rows);
     }
-    for (int64_t ii = C.tri ? oi : 0; ii < C.nIi; ++ii) {
-      f(ras_cmp_var(C, oi, ii), ras_cmp_cell(C, oi, ii),
-        C.tri && oi == ii ? (int64_t)C.nEo * (C.nEo + 1) / 2 : (int64_t)C.nEo * C.nEi);
-    }
-  }
 }
 
 // Builds the plan for the space and integrals; plan.ok = false (with a

@@ -7,11 +7,9 @@
 // :13036-13115), which regenerates every configuration-pair block.  One
 // sigma call of K columns is, per chunk of KC <= 16 columns (FP64: 8 when
 // device memory is short):
-//   k_ras_x2c   SEF vectors -> determinant vectors c[2 det + s][KC] = (-1)^s
-//               c_det (each determinant belongs to one SEF: a scatter
-//               without collisions; both signs, so a product reads an entry
-//               of either sign without arithmetic), rows 2 ndet and 2 ndet +
-//               1 zero;
+//   k_ras_x2c   SEF vectors -> determinant vectors, both signs (each
+//               determinant belongs to one SEF: a scatter without collisions;
+//               a product reads an entry of either sign without arithmetic);
 //   k_ras_gemm  per tile of the compact products (RasCmp, ras.hpp): W[row]
 //               [p-pair][KC] = sum over q-pairs of G[p-pair][q-pair]
 //               D[row][q-pair][KC], D gathered from c into LDS through the
@@ -22,8 +20,13 @@
 //               terms of its determinants (the term list -- signed W offsets
 //               -- is built once at setup by k_ras_terms), written once (a
 //               gather: deterministic, no atomics).
-// HBM layout: c [2 ndet + 2][KC] (64 B per row at KC = 16 FP32), W [block
-// rows][nqp][KC] so that a term of k_ras_y reads KC contiguous values.
+// HBM layout: c [2 ndet + 1][KC] (64 B per row at KC = 16 FP32; every +c, then
+// every -c, then a zero row) and W [group][pair][row][KC], so that the
+// determinants that consecutive rows of a product gather, and the W terms of
+// consecutive SEFs (in the order of k_ras_order), share cache lines: on 10 +
+// 24 orbitals, 8 electrons, 16 FP32 columns, L2 misses of the products 95 ->
+// 77 GB and of k_ras_y 43 -> 35 GB against +c and -c side by side, W
+// [row][pair] and the list's own order.
 #include <algorithm>
 #include <cstdlib>
 
@@ -59,50 +62,96 @@ struct Mfma<double> {
   static __device__ __forceinline__ int row(int t, int l) { return 4 * t + (l >> 4); }
 };
 
-// The signed rows of every SEF's determinant coefficients (built once):
-// rows.x = 2 det + negative of its first determinant; rows.y the same for
-// the second, or -1 (one determinant, coefficient 1/sqrt(2)) or -2 (a
-// closed shell, coefficient 1); -3 marks a determinant outside the plan
-// (never, for a plan that passes its host checks).
-__global__ __launch_bounds__(256) void k_ras_sefrows(const RasView* __restrict__ vp, int2* __restrict__ rows) {
+// determinant d of a SEF, or -1 outside the plan (never, for a plan that
+// passes its host checks)
+__device__ __forceinline__ int64_t ras_sef_det(const RasView& v, const RasSef& e, int d) {
+  const RasSectorDev& S = v.sec[e.sec[d]];
+  const int ca = ras_cls_of(v, S.na, e.a[d]), cb = ras_cls_of(v, S.nb, e.b[d]);
+  const int64_t det =
+      ras_det(v, e.sec[d], ca, e.a[d] - v.lev[S.na].cls_off[ca], cb, e.b[d] - v.lev[S.nb].cls_off[cb]);
+  return det >= 0 && det < v.ndet ? det : -1;
+}
+
+// The order in which the scatter and the gather walk the SEFs (built once):
+// by the lower of their determinants.  Consecutive SEFs then differ in the
+// external part of one string, as do consecutive rows of a product's group,
+// so a wavefront's determinant rows and W terms are consecutive in memory (a
+// list in file order puts such SEFs far apart).  k_ras_mark: flag and SEF of
+// each such determinant; k_ras_order: order[rank] = SEF.
+__global__ __launch_bounds__(256) void k_ras_mark(const RasView* __restrict__ vp, int64_t* __restrict__ flag,
+                                                  int32_t* __restrict__ sef) {
   const RasView& v = *vp;
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= v.nsef) return;
   const RasSef e = v.sef[s];
-  int r[2] = {-3, (e.flag[0] & 2) ? -2 : -1};
-  for (int d = 0; d < e.n; ++d) {
-    const RasSectorDev& S = v.sec[e.sec[d]];
-    const int ca = ras_cls_of(v, S.na, e.a[d]), cb = ras_cls_of(v, S.nb, e.b[d]);
-    const int64_t det =
-        ras_det(v, e.sec[d], ca, e.a[d] - v.lev[S.na].cls_off[ca], cb, e.b[d] - v.lev[S.nb].cls_off[cb]);
-    r[d] = (det >= 0 && det < v.ndet) ? (int)(2 * det + (e.flag[d] & 1)) : -3;
+  int64_t k = ras_sef_det(v, e, 0);
+  if (e.n > 1) {
+    const int64_t k1 = ras_sef_det(v, e, 1);
+    k = k1 < k ? k1 : k;
   }
-  rows[s] = make_int2(r[0], r[1]);
+  if (k < 0) return;
+  flag[k] = 1;
+  sef[k] = (int32_t)s;
+}
+__global__ __launch_bounds__(256) void k_ras_order(int64_t ndet, const int64_t* __restrict__ flag,
+                                                   const int64_t* __restrict__ rank, const int32_t* __restrict__ sef,
+                                                   int32_t* __restrict__ order) {
+  const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (d < ndet && flag[d]) order[rank[d]] = sef[d];
+}
+__global__ __launch_bounds__(256) void k_ras_zero64(int64_t n, int64_t* __restrict__ p) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) p[t] = 0;
 }
 
-// c[row][KC] = (-1)^(row & 1 ^ negative) * magnitude * x[sef][col0 + q]
-// (zero for q >= kw) for both signed rows of each of the SEF's
-// determinants; the zero rows 2 ndet, 2 ndet + 1.  X may be wider than T
-// (FP64 vectors rounded to the FP32 computation on the fly).
+// The signed rows of every SEF's determinant coefficients, in that order
+// (built once): rows.x = det + negative * ndet of its first determinant; rows.y the same for the second, or -1 (one determinant, coefficient
+// 1/sqrt(2)) or -2 (a closed shell, coefficient 1); -3 marks a determinant
+// outside the plan.
+__global__ __launch_bounds__(256) void k_ras_sefrows(const RasView* __restrict__ vp,
+                                                     const int32_t* __restrict__ order, int2* __restrict__ rows) {
+  const RasView& v = *vp;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= v.nsef) return;
+  const RasSef e = v.sef[order[i]];
+  int r[2] = {-3, (e.flag[0] & 2) ? -2 : -1};
+  for (int d = 0; d < e.n; ++d) {
+    const int64_t det = ras_sef_det(v, e, d);
+    r[d] = det >= 0 ? (int)(det + (e.flag[d] & 1) * v.ndet) : -3;
+  }
+  rows[i] = make_int2(r[0], r[1]);
+}
+
+// c[row][KC] = +-magnitude * x[sef][col0 + q] (zero for q >= kw) for both
+// signed rows (det, and ndet + det: -c_det) of each of the SEF's
+// determinants; the zero row 2 ndet.  Threads follow the SEF order of k_ras_y,
+// whose determinants are consecutive, so the four row writes per SEF stream
+// and only the one read is scattered.  X may be wider than T (FP64 vectors
+// rounded to the FP32 computation on the fly).
 template <typename T, int KC, typename TX = T>
-__global__ __launch_bounds__(256) void k_ras_x2c(int64_t nsef, int64_t ndet, const int2* __restrict__ rows,
-                                                 const TX* __restrict__ X, int ldx, int col0, int kw,
-                                                 T* __restrict__ c) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < 2 * KC) c[2 * ndet * KC + t] = (T)0;
-  const int64_t s = t / KC;
+__global__ __launch_bounds__(256) void k_ras_x2c(int64_t nsef, int64_t ndet, const int32_t* __restrict__ order,
+                                                 const int2* __restrict__ rows, const TX* __restrict__ X, int ldx,
+                                                 int col0, int kw, T* __restrict__ c) {
+  // (parts per XCD as in k_ras_y, for rows shorter than a cache line)
+  const int64_t per = gridDim.x >> 3;
+  const int64_t t =
+      (sizeof(T) == 4 ? (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3) : (int64_t)blockIdx.x) * blockDim.x +
+      threadIdx.x;
+  if (t < KC) c[2 * ndet * KC + t] = (T)0;
+  const int64_t i = t / KC;
   const int q = (int)(t % KC);
-  if (s >= nsef) return;
-  const int2 r = rows[s];
+  if (i >= nsef) return;
+  const int64_t s = order[i];
+  const int2 r = rows[i];
   const T x = q < kw ? (T)X[s * (int64_t)ldx + col0 + q] : (T)0;
   const T y = (r.y == -2 ? (T)1 : (T)0x1.6a09e667f3bcdp-1) * x;
   if (r.x >= 0) {
     c[(int64_t)r.x * KC + q] = y;
-    c[(int64_t)(r.x ^ 1) * KC + q] = -y;
+    c[(r.x < ndet ? r.x + ndet : r.x - ndet) * KC + q] = -y;
   }
   if (r.y >= 0) {
     c[(int64_t)r.y * KC + q] = y;
-    c[(int64_t)(r.y ^ 1) * KC + q] = -y;
+    c[(r.y < ndet ? r.y + ndet : r.y - ndet) * KC + q] = -y;
   }
 }
 
@@ -150,8 +199,8 @@ __global__ __launch_bounds__(256) void k_ras_gvar(int64_t gbase, int64_t n, int 
 }
 
 // Signed vector row of every D entry (built once): didx[dbase + row * nqp +
-// j] = 2 det + negative for live pair j of row `row`, the zero row 2 ndet
-// when the pair cannot be added to the row's strings (ras_d_det).
+// j] = det + negative * ndet for live pair j of row `row`, the zero row 2
+// ndet when the pair cannot be added to the row's strings (ras_d_det).
 __global__ __launch_bounds__(256) void k_ras_didx(const RasView* __restrict__ vp, int bi,
                                                   const int16_t* __restrict__ pr, int32_t* __restrict__ didx) {
   const RasView& v = *vp;
@@ -167,8 +216,14 @@ __global__ __launch_bounds__(256) void k_ras_didx(const RasView* __restrict__ vp
   const int64_t u = C.swap ? C.i0 + i : C.o0 + o, w = C.swap ? C.o0 + o : C.i0 + i;
   int neg = 0;
   const int64_t det = qs < 0 ? -1 : ras_d_det(v, C.kind, C.sector, B.lu, B.lw, u, w, qs & 0xff, (qs >> 8) & 0xff, neg);
-  didx[C.dbase + e] = (det < 0 || det >= v.ndet) ? (int32_t)(2 * v.ndet) : (int32_t)(2 * det + neg);
+  didx[C.dbase + e] = (det < 0 || det >= v.ndet) ? (int32_t)(2 * v.ndet) : (int32_t)(det + neg * v.ndet);
 }
+
+// A W element: FP64 past the caches (W is read once, by k_ras_y, long after;
+// 10 + 24 orbitals, 16 columns: products 42.5 -> 42.3, gather 9.4 -> 8.2 ms);
+// FP32 through them (its half-line stores merge in L2: 22.9 against 23.3 ms)
+__device__ __forceinline__ void ras_store(double x, double* p) { __builtin_nontemporal_store(x, p); }
+__device__ __forceinline__ void ras_store(float x, float* p) { *p = x; }
 
 // One group of rows with its matrix, and its first tile per chunk width
 // (built on the host; the tile table is written from it).
@@ -183,31 +238,36 @@ struct RasGroup {
 __global__ __launch_bounds__(64) void k_ras_tiles(const RasGroup* __restrict__ grp, int which, int rt,
                                                   RasTile* __restrict__ out) {
   const RasGroup G = grp[blockIdx.x];
-  const int npt = (G.nqp + G.pt - 1) / G.pt;
+  // the p-subtiles of 16 spread evenly over the p-tiles
+  const int ns = G.nqp / 16, npt = (G.nqp + G.pt - 1) / G.pt, each = ns / npt, more = ns % npt;
   const int64_t n = (G.rows + rt - 1) / rt * npt;
   for (int64_t t = threadIdx.x; t < n; t += blockDim.x) {
     const int64_t r0 = t / npt * rt;
-    const int p0 = (int)(t % npt) * G.pt;
-    const int left = G.nq - p0 < G.pt ? G.nq - p0 : G.pt;
+    // (the p-tiles of a row tile differ by a subtile: their order, and the
+    // wavefront pair that takes the larger half, rotate from row tile to row
+    // tile so that no shader engine or SIMD always gets the longer ones)
+    const int64_t turn = blockIdx.x + t / npt;
+    const int pt = (int)((t + turn) % npt);
     RasTile T;
     T.g = G.g;
-    T.w = G.w + r0 * G.nqp;
+    T.w = G.w + r0;
+    T.rows = (int32_t)G.rows;
+    T.flip = (int32_t)((turn / npt) & 1);
     T.d = G.d + r0 * G.nqp;
     T.nqp = G.nqp;
-    T.p0 = (uint16_t)p0;
+    T.p0 = (uint16_t)(16 * (pt * each + (pt < more ? pt : more)));
     T.nrows = (uint8_t)(G.rows - r0 < rt ? G.rows - r0 : rt);
-    T.niv = (uint8_t)((left + 15) / 16);
+    T.niv = (uint8_t)(G.pt <= 64 ? G.nq : each + (pt < more ? 1 : 0));
     out[G.tile0[which] + t] = T;
   }
 }
 
 // wavefronts per SIMD the product is compiled for (a register budget: the
 // compiler would otherwise hold more k-steps' operands in flight than
-// occupancy can afford; at FP32 and 64 p-pairs the budget of 6 spills a few
-// set-up values outside the chunk loop, measured 2 % faster than 5)
-template <typename T, int PT>
+// occupancy can afford)
+template <typename T>
 constexpr int ras_lds_waves() {
-  return sizeof(T) == 8 ? (PT <= 64 ? 3 : 2) : (PT <= 64 ? 6 : 4);
+  return sizeof(T) == 8 ? 3 : 6;
 }
 
 template <int N>
@@ -235,9 +295,9 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p);
 }
 
-// The products: one workgroup per tile (PT p-pairs x 128 (row, column)
-// values; RasTile), four wavefronts of PT x 32 values (PT / 16 x 2 MFMA
-// tiles).  Operands are copied straight from global memory into LDS
+// The products of PT <= 64 p-pairs (nqp = PT): one workgroup per tile (PT
+// p-pairs x 128 (row, column) values; RasTile), four wavefronts of PT x 32
+// values (PT / 16 x 2 MFMA tiles).  Operands are copied straight from global memory into LDS
 // (global_load_lds_dwordx4: each lane names its own 16-byte source, the
 // wavefront's 64 pieces land contiguously at one LDS address), into two LDS
 // stages: the copies of chunk n + 1 are in flight while the MFMA steps
@@ -259,11 +319,11 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // chunk loop is unrolled over the two stages, so every LDS address is a
 // constant offset, and the matrix and index addresses advance in scalar
 // registers.
-// One launch covers every block of one tile width PT (27 blocks on 10 + 24
+// One launch covers every block of one tile width (27 blocks on 10 + 24
 // orbitals, 8 electrons: 5 launches instead of 27), heavy tiles first; tiles
 // are dealt to the 8 XCDs in runs of 2^sh, so that the tiles of a row group
 // (the same c rows and matrix) share an L2.
-template <typename T, int KC, int PT, int WPE = ras_lds_waves<T, PT>()>
+template <typename T, int KC, int PT, int WPE = ras_lds_waves<T>()>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE)))
 void k_ras_gemm(const RasTile* __restrict__ tiles, int64_t ntiles, int sh, const int32_t* __restrict__ didx,
                 const T* __restrict__ G, const T* __restrict__ c, T* __restrict__ W) {
@@ -282,34 +342,32 @@ void k_ras_gemm(const RasTile* __restrict__ tiles, int64_t ntiles, int sh, const
   static_assert(KC % SL == 0 && RW >= 2 && kQC * GSR % 64 == 0, "copy shapes");
   __shared__ __align__(16) T Gs[2][kQC * PT];
   __shared__ __align__(16) T Ds[2][kQC * kMT];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t b = blockIdx.x >> 3;
   const int64_t ti = ((((b >> sh) << 3) + (blockIdx.x & 7)) << sh) + (b & ((1 << sh) - 1));
   if (ti >= ntiles) return;  // uniform per workgroup
   const RasTile tile = tiles[ti];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nrows = tile.nrows, nqp = tile.nqp, p0 = tile.p0, niv = tile.niv;
-  const int nch = nqp / kQC;
+  const int nrows = tile.nrows, nq = tile.niv;
+  constexpr int nch = PT / kQC;
 
   // this lane's sources: its D entries' offsets in the index table and its G
-  // pieces' byte offsets, both from bases that advance by a chunk (a G piece
-  // past nqp repeats its row's first, feeding only output rows that are not
-  // stored)
+  // pieces' byte offsets, both from bases that advance by a chunk
   const int32_t* __restrict__ dx = didx + tile.d;
-  const T* __restrict__ Gb = G + tile.g + p0;
+  const T* __restrict__ Gb = G + tile.g;
   uint32_t dxo[DI];
 #pragma unroll
   for (int d = 0; d < DI; ++d) {
     const int slot = d * 64 + lane;
     const int q = slot / (SPE * RW), r = ((slot / SPE) % RW) ^ ((q & 1) * (RW / 2));
     const int row = RW * wave + r;
-    dxo[d] = (uint32_t)((row < nrows ? row : nrows - 1) * nqp + q);
+    dxo[d] = (uint32_t)((row < nrows ? row : nrows - 1) * PT + q);
   }
   uint32_t go[GW];
 #pragma unroll
   for (int gi = 0; gi < GW; ++gi) {
     const int sl = 64 * (wave + 4 * gi) + lane, k = sl / GSR;
     const int r = SWZ ? (sl % GSR) ^ (4 * (k & 1)) : sl % GSR;
-    go[gi] = (uint32_t)((k * nqp + (p0 + r * SL < nqp ? r * SL : 0)) * sizeof(T));
+    go[gi] = (uint32_t)((k * PT + r * SL) * sizeof(T));
   }
   const T* __restrict__ cl = c + SL * (lane % SPE);
   // LDS addresses of this wavefront's first D copy and first G copy (stage 0)
@@ -340,7 +398,7 @@ void k_ras_gemm(const RasTile* __restrict__ tiles, int64_t ntiles, int sh, const
       if (wave + 4 * gi >= GI) continue;
       lds_copy16(Gb, go[gi], gl0 + (uint32_t)((ST * kQC * PT + 64 * 4 * gi * SL) * sizeof(T)));
     }
-    Gb += (int64_t)kQC * nqp;
+    Gb += kQC * PT;
   };
 
   // lane offsets of the MFMA operand reads (k row kr = lane / 16 within a
@@ -352,86 +410,234 @@ void k_ras_gemm(const RasTile* __restrict__ tiles, int64_t ntiles, int sh, const
   const int a0[2] = {kr * PT + l15 + sw, kr * PT + l15 - sw};
   const int b0[2] = {32 * (kQC * wave + kr) + l15 + 16 * (kr & 1), 32 * (kQC * wave + kr) + l15 + 16 - 16 * (kr & 1)};
 
-  // the whole tile with NV live p-subtiles
+  v4 acc[NI][2];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = v4{0, 0, 0, 0};
+  int32_t ixn[DI];
+  fetch_idx(ixn);
+  issue(IntC<0>{}, ixn);
+  if (nch > 1) fetch_idx(ixn);
+  // one chunk on stage ST; `left` chunks follow
+  auto chunk = [&](auto stc, int left) {
+    constexpr int ST = decltype(stc)::value;
+    // this wavefront's copies of the chunk have landed, every wavefront's
+    // have after the barrier, and the other stage is free (its reads ended
+    // before the barrier)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (left > 0) {
+      issue(IntC<1 - ST>{}, ixn);
+      if (left > 1) fetch_idx(ixn);
+    }
+    const T* __restrict__ gs = Gs[ST];
+    const T* __restrict__ ds = Ds[ST];
+#pragma unroll
+    for (int kk = 0; kk < kQC / 4; ++kk) {
+      T a[NI], bb[2];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) a[i] = gs[a0[i & 1] + 16 * i + 4 * kk * PT];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) bb[j] = ds[b0[j] + 4 * kk * 32];
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = M::op(a[i], bb[j], acc[i][j]);
+    }
+  };
+  for (int left = nch - 1; left >= 0; left -= 2) {
+    chunk(IntC<0>{}, left);
+    if (left > 0) chunk(IntC<1>{}, left - 1);
+  }
+  T* __restrict__ Wt = W + tile.w * KC;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int m = 16 * j + l15, row = RW * wave + m / KC;
+    if (row >= nrows) continue;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int p = 16 * i + M::row(t, lane);
+        if (p < nq) ras_store(acc[i][j][t], &Wt[((int64_t)p * tile.rows + row) * KC + m % KC]);
+      }
+  }
+}
+
+// The products of more than 64 p-pairs: one workgroup per tile of up to 128
+// p-pairs x 128 (row, column) values, four wavefronts as 2 x 2 of up to 64 x 64
+// (the first pair of wavefronts takes the first half of the tile's n
+// p-subtiles of 16, the other pair the rest).  Against k_ras_gemm's 64 x 128
+// tiles a D piece is gathered by half as many tiles and an LDS operand feeds
+// four MFMAs instead of 2.7.  Copies, stages and chunk loop as in k_ras_gemm.
+// Layouts in LDS: both stages [q][128], the 16-value groups of row q at group
+// position ^ (q & 3) within their four, so that the four rows one operand
+// read touches lie in separate banks; p-subtile i of the second wavefront
+// pair sits at group 4 + i.
+template <typename T, int KC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : 3)))
+void k_ras_gemm_wide(const RasTile* __restrict__ tiles, int64_t ntiles, int sh, const int32_t* __restrict__ didx,
+                     const T* __restrict__ G, const T* __restrict__ c, T* __restrict__ W) {
+  typedef Mfma<T> M;
+  typedef typename M::v4 v4;
+  constexpr int SL = 16 / sizeof(T);       // values per 16-byte piece
+  constexpr int PR = kMT / SL;             // pieces per LDS row
+  constexpr int NC = kQC * PR / 256;       // copies of each operand per wavefront and chunk
+  static_assert(KC % SL == 0, "copy shapes");
+  __shared__ __align__(16) T Gs[2][kQC * kMT];
+  __shared__ __align__(16) T Ds[2][kQC * kMT];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t b = blockIdx.x >> 3;
+  const int64_t ti = ((((b >> sh) << 3) + (blockIdx.x & 7)) << sh) + (b & ((1 << sh) - 1));
+  if (ti >= ntiles) return;  // uniform per workgroup
+  const RasTile tile = tiles[ti];
+  const int nrows = tile.nrows, nqp = tile.nqp, p0 = tile.p0;
+  const int n0 = (tile.niv + 1) >> 1, n1 = tile.niv >> 1;  // p-subtiles of the two wavefront pairs
+  const int nch = nqp / kQC;
+
+  // this lane's sources (as in k_ras_gemm): copy d of the wavefront fills the
+  // pieces 64 (wave + 4 d) + lane of a stage
+  const int32_t* __restrict__ dx = didx + tile.d;
+  const T* __restrict__ Gb = G + tile.g + p0;
+  uint32_t dxo[NC], go[NC];
+  int vo = 0;  // column of the lane's pieces (the same for every copy)
+#pragma unroll
+  for (int d = 0; d < NC; ++d) {
+    const int sl = 64 * (wave + 4 * d) + lane, q = sl / PR;
+    const int v = ((sl % PR) * SL) ^ (16 * (q & 3));
+    const int row = v / KC;
+    dxo[d] = (uint32_t)((row < nrows ? row : nrows - 1) * nqp + q);
+    vo = v % KC;
+    const int sp = v >> 4, sub = sp < 4 ? (sp < n0 ? sp : 0) : (sp - 4 < n1 ? n0 + sp - 4 : 0);
+    go[d] = (uint32_t)((q * nqp + 16 * sub + (v & 15)) * sizeof(T));
+  }
+  const T* __restrict__ cl = c + vo;
+  const uint32_t dl0 = lds_addr(&Ds[0][64 * wave * SL]);
+  const uint32_t gl0 = lds_addr(&Gs[0][64 * wave * SL]);
+  auto fetch_idx = [&](int32_t (&ix)[NC]) {
+#pragma unroll
+    for (int d = 0; d < NC; ++d) ix[d] = dx[dxo[d]];
+    dx += kQC;
+  };
+  auto issue = [&](auto stc, const int32_t (&ix)[NC]) {
+    constexpr int ST = decltype(stc)::value;
+    const T* src[NC];
+#pragma unroll
+    for (int d = 0; d < NC; ++d) src[d] = cl + (uint64_t)(uint32_t)ix[d] * KC;
+#pragma unroll
+    for (int d = 0; d < NC; ++d) asm volatile("" : "+v"(src[d]));
+#pragma unroll
+    for (int d = 0; d < NC; ++d)
+      lds_copy16(src[d], dl0 + (uint32_t)((ST * kQC * kMT + d * 256 * SL) * sizeof(T)));
+#pragma unroll
+    for (int d = 0; d < NC; ++d)
+      lds_copy16(Gb, go[d], gl0 + (uint32_t)((ST * kQC * kMT + d * 256 * SL) * sizeof(T)));
+    Gb += (int64_t)kQC * nqp;
+  };
+  const int kr = lane >> 4, l15 = lane & 15, wr = (wave >> 1) ^ tile.flip, wc = wave & 1;
+  int a0[4], b0[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a0[i] = kr * kMT + 64 * wr + 16 * (i ^ kr) + l15;
+    b0[i] = kr * kMT + 64 * wc + 16 * (i ^ kr) + l15;
+  }
+
   auto run = [&](auto nvc) {
     constexpr int NV = decltype(nvc)::value;
-    v4 acc[NV][2];
+    v4 acc[NV][4];
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = v4{0, 0, 0, 0};
-    int32_t ixn[DI];
+      for (int j = 0; j < 4; ++j) acc[i][j] = v4{0, 0, 0, 0};
+    int32_t ixn[NC];
+    // operands of two k-steps: one is read from LDS while the other multiplies
+    T a[2][NV], bb[2][4];
+    auto read = [&](auto stc, auto kkc, auto setc) {
+      constexpr int ST = decltype(stc)::value, kk = decltype(kkc)::value, S = decltype(setc)::value;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) a[S][i] = Gs[ST][a0[i] + 4 * kk * kMT];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bb[S][j] = Ds[ST][b0[j] + 4 * kk * kMT];
+    };
+    auto mul = [&](auto setc) {
+      constexpr int S = decltype(setc)::value;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = M::op(a[S][i], bb[S][j], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // every wavefront's copies into the next stage have landed and its reads
+    // of the other have ended (the copies of the chunk after go there)
+    auto turn = [&](auto stc, int left) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (left > 0) {
+        issue(stc, ixn);
+        if (left > 1) fetch_idx(ixn);
+      }
+    };
     fetch_idx(ixn);
     issue(IntC<0>{}, ixn);
     if (nch > 1) fetch_idx(ixn);
-    // one chunk on stage ST; `left` chunks follow
+    turn(IntC<1>{}, nch - 1);
+    read(IntC<0>{}, IntC<0>{}, IntC<0>{});
+    // one chunk on stage ST; `left` chunks follow.  The barrier sits before
+    // the last k-step, whose operands are in registers, so that its MFMAs
+    // cover the first reads of the next stage
     auto chunk = [&](auto stc, int left) {
       constexpr int ST = decltype(stc)::value;
-      // this wavefront's copies of the chunk have landed, every wavefront's
-      // have after the barrier, and the other stage is free (its reads ended
-      // before the barrier)
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
+      read(IntC<ST>{}, IntC<1>{}, IntC<1>{});
+      mul(IntC<0>{});
+      read(IntC<ST>{}, IntC<2>{}, IntC<0>{});
+      mul(IntC<1>{});
+      read(IntC<ST>{}, IntC<3>{}, IntC<1>{});
+      mul(IntC<0>{});
       if (left > 0) {
-        issue(IntC<1 - ST>{}, ixn);
-        if (left > 1) fetch_idx(ixn);
+        turn(IntC<ST>{}, left - 1);
+        read(IntC<1 - ST>{}, IntC<0>{}, IntC<0>{});
       }
-      const T* __restrict__ gs = Gs[ST];
-      const T* __restrict__ ds = Ds[ST];
-#pragma unroll
-      for (int kk = 0; kk < kQC / 4; ++kk) {
-        T a[NV], bb[2];
-#pragma unroll
-        for (int i = 0; i < NV; ++i) a[i] = gs[a0[i & 1] + 16 * i + 4 * kk * PT];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) bb[j] = ds[b0[j] + 4 * kk * 32];
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = M::op(a[i], bb[j], acc[i][j]);
-      }
+      mul(IntC<1>{});
     };
     for (int left = nch - 1; left >= 0; left -= 2) {
       chunk(IntC<0>{}, left);
       if (left > 0) chunk(IntC<1>{}, left - 1);
     }
     T* __restrict__ Wt = W + tile.w * KC;
+    const int ps = p0 + (wr ? 16 * n0 : 0);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int m = 16 * j + l15, row = RW * wave + m / KC;
+    for (int j = 0; j < 4; ++j) {
+      const int m = 64 * wc + 16 * j + l15, row = m / KC;
       if (row >= nrows) continue;
 #pragma unroll
       for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int p = p0 + 16 * i + M::row(t, lane);
-          if (p < nqp) Wt[(row * nqp + p) * KC + m % KC] = acc[i][j][t];
-        }
+        for (int t = 0; t < 4; ++t) 
+            ras_store(acc[i][j][t], &Wt[((int64_t)(ps + 16 * i + M::row(t, lane)) * tile.rows + row) * KC + m % KC]);
     }
   };
-  // tiles cover the pairs exactly except, for some widths, the last one
-  if (niv >= NI) {
-    run(IntC<NI>{});
-  } else if constexpr (NI > 1) {
-    if (niv == 1) run(IntC<1>{});
-    else if (NI > 2 && niv == 2) run(IntC<(NI > 2 ? 2 : 1)>{});
-    else if (NI > 3 && niv == 3) run(IntC<(NI > 3 ? 3 : 1)>{});
-    else run(IntC<NI>{});
-  }
+  // the same number of barriers in every variant: nch
+  const int nv = wr ? n1 : n0;
+  if (nv == 4) run(IntC<4>{});
+  else if (nv == 3) run(IntC<3>{});
+  else run(IntC<2>{});
 }
 
-// The term list of every SEF (built once): FILL = false counts each SEF's
-// terms into cnt[s]; FILL = true writes them, as the W offset per column
+// The term list of every SEF (built once), in the SEF order: FILL = false
+// counts the terms of SEF order[s] into cnt[s]; FILL = true writes them, as the W offset per column
 // with bit 31 set for a negative sign (the determinants' coefficient signs
 // folded in), at toff[s] (the scanned counts), and the SEF's scale code.
 template <bool FILL>
-__global__ __launch_bounds__(256) void k_ras_terms(const RasView* __restrict__ vp, int64_t* __restrict__ cnt,
+__global__ __launch_bounds__(256) void k_ras_terms(const RasView* __restrict__ vp,
+                                                   const int32_t* __restrict__ order, int64_t* __restrict__ cnt,
                                                    const int64_t* __restrict__ toff, int32_t* __restrict__ term,
                                                    int8_t* __restrict__ scl, int* __restrict__ bad) {
   const RasView& v = *vp;
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= v.nsef) return;
-  const RasSef e = v.sef[s];
+  const RasSef e = v.sef[order[s]];
   if (!FILL) {
     int64_t n = 0;
     ras_sef_terms(v, e, bad, [&](int64_t, int) { ++n; });
@@ -455,9 +661,16 @@ __global__ __launch_bounds__(256) void k_ras_terms(const RasView* __restrict__ v
 // be wider than T: the FP32 result widened exactly)
 template <typename T, int KC, typename TY = T>
 __global__ __launch_bounds__(256) void k_ras_y(const int64_t* __restrict__ toff, const int32_t* __restrict__ term,
-                                               const int8_t* __restrict__ scl, const T* __restrict__ W, int64_t nsef,
+                                               const int8_t* __restrict__ scl, const int32_t* __restrict__ order,
+                                               const T* __restrict__ W, int64_t nsef,
                                                TY* __restrict__ Y, int ldy, int col0, int kw) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  // FP32 rows are half a cache line: each XCD takes a contiguous part of the
+  // SEFs, so that both halves are read through one L2 (10 + 24 orbitals, 16
+  // columns: 5.4 -> 5.0 ms; whole lines, FP64: 8.2 -> 8.7 ms, so not there)
+  const int64_t per = gridDim.x >> 3;
+  const int64_t t =
+      (sizeof(T) == 4 ? (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3) : (int64_t)blockIdx.x) * blockDim.x +
+      threadIdx.x;
   const int64_t s = t / KC;
   const int q = (int)(t % KC);
   if (s >= nsef) return;
@@ -482,7 +695,7 @@ __global__ __launch_bounds__(256) void k_ras_y(const int64_t* __restrict__ toff,
   }
   const int8_t sc = scl[s];
   const T f = sc == 2 ? (T)1 : (sc == 1 ? (T)0x1.6a09e667f3bcdp+0 : (T)0x1.6a09e667f3bcdp-1);
-  if (q < kw) Y[s * (int64_t)ldy + col0 + q] = (TY)(f * (a0 + a1));
+  if (q < kw) Y[order[s] * (int64_t)ldy + col0 + q] = (TY)(f * (a0 + a1));
 }
 
 // Flags (*flag = 1) a configuration pair one electron apart whose
@@ -551,15 +764,8 @@ struct RasTiming {
   }
 };
 
-// p-pairs per product tile: one tile when there are at most 112, else the
-// first of 64, 96, 80, 112 and 48 that divides the (16-padded) pair count,
-// else 64 with a narrower last tile
-inline int ras_tile_width(int nqp) {
-  if (nqp <= 112) return nqp;
-  for (int w : {64, 96, 80, 112, 48})
-    if (nqp % w == 0) return w;
-  return 64;
-}
+// p-pairs per product tile: one exact tile up to 64, else k_ras_gemm_wide's
+inline int ras_tile_width(int nqp) { return nqp <= 64 ? nqp : kMT; }
 
 template <typename T, int KC, typename TIO = T>
 void ras_chunk(Ctx& c, const TIO* X, int ldx, TIO* Y, int ldy, int col0, int kw, RasTiming* tm = nullptr) {
@@ -569,8 +775,8 @@ void ras_chunk(Ctx& c, const TIO* X, int ldx, TIO* Y, int ldy, int col0, int kw,
   const T* G = sizeof(T) == 4 ? reinterpret_cast<const T*>(c.d_rasg32.p) : reinterpret_cast<const T*>(c.d_rasg64.p);
   const int64_t nsef = (int64_t)P.sef.size();
   if (tm && tm->ev.empty()) tm->mark(c.stream, -1);
-  hipLaunchKernelGGL((k_ras_x2c<T, KC, TIO>), dim3(nblk(nsef * KC, 256)), dim3(256), 0, c.stream, nsef, P.ndet,
-                     c.d_rasrows.p, X, ldx, col0, kw, cv);
+  hipLaunchKernelGGL((k_ras_x2c<T, KC, TIO>), dim3(8 * nblk(nsef * KC, 8 * 256)), dim3(256), 0, c.stream, nsef, P.ndet,
+                     c.d_rasorder.p, c.d_rasrows.p, X, ldx, col0, kw, cv);
   PSOCI_HIP(hipGetLastError());
   if (tm) tm->mark(c.stream, 0);
   constexpr int ki = KC == 16 ? 0 : KC == 8 ? 1 : KC == 4 ? 2 : 3;
@@ -595,18 +801,17 @@ void ras_chunk(Ctx& c, const TIO* X, int ldx, TIO* Y, int ldy, int col0, int kw,
       PSOCI_RAS_GEMM(32)
       PSOCI_RAS_GEMM(48)
       PSOCI_RAS_GEMM(64)
-      PSOCI_RAS_GEMM(80)
-      PSOCI_RAS_GEMM(96)
-      PSOCI_RAS_GEMM(112)
 #undef PSOCI_RAS_GEMM
-      default: throw Error(PSOCI_ERR_STATE, "string-driven sigma: no product of this tile width");
+      default:
+        hipLaunchKernelGGL((k_ras_gemm_wide<T, KC>), dim3(grid), dim3(256), 0, c.stream, tiles, nt, sh,
+                           c.d_rasdidx.p, G, cv, W);
     }
     PSOCI_HIP(hipGetLastError());
     if (tm) tm->mark(c.stream, 1 + L[i].kind);
     i = e;
   }
-  hipLaunchKernelGGL((k_ras_y<T, KC, TIO>), dim3(nblk(nsef * KC, 256)), dim3(256), 0, c.stream, c.d_rastoff.p,
-                     c.d_rasterm.p, c.d_rasscl.p, W, nsef, Y, ldy, col0, kw);
+  hipLaunchKernelGGL((k_ras_y<T, KC, TIO>), dim3(8 * nblk(nsef * KC, 8 * 256)), dim3(256), 0, c.stream, c.d_rastoff.p,
+                     c.d_rasterm.p, c.d_rasscl.p, c.d_rasorder.p, W, nsef, Y, ldy, col0, kw);
   PSOCI_HIP(hipGetLastError());
   if (tm) tm->mark(c.stream, 4);
 }
@@ -788,6 +993,29 @@ bool build_ras(Ctx& c) {
     ras_tile_tables(c);
     c.sync();
   }
+  // the SEF order
+  {
+    const int64_t nsef = (int64_t)P.sef.size();
+    DevBuf<int64_t> flag, rank;
+    DevBuf<int32_t> sef;
+    flag.alloc(P.ndet + 1);
+    rank.alloc(P.ndet + 1);
+    sef.alloc(P.ndet);
+    c.d_rasorder.alloc(nsef);
+    hipLaunchKernelGGL(k_ras_zero64, dim3(nblk(P.ndet + 1, 256)), dim3(256), 0, c.stream, P.ndet + 1, flag.p);
+    PSOCI_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_ras_mark, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p, flag.p, sef.p);
+    PSOCI_HIP(hipGetLastError());
+    c.scan(flag.p, rank.p, P.ndet + 1);
+    int64_t found = 0;
+    PSOCI_HIP(hipMemcpyAsync(&found, rank.p + P.ndet, sizeof(int64_t), hipMemcpyDeviceToHost, c.stream));
+    c.sync();
+    PSOCI_CHECK(found == nsef, PSOCI_ERR_STATE, "string-driven sigma: inconsistent determinant map");
+    hipLaunchKernelGGL(k_ras_order, dim3(nblk(P.ndet, 256)), dim3(256), 0, c.stream, P.ndet, flag.p, rank.p, sef.p,
+                       c.d_rasorder.p);
+    PSOCI_HIP(hipGetLastError());
+    c.sync();
+  }
   // the SEF term lists (merged where an SEF's two determinants read the
   // same W elements): count, scan, fill
   {
@@ -798,8 +1026,8 @@ bool build_ras(Ctx& c) {
     bad.alloc(1);
     PSOCI_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), c.stream));
     PSOCI_HIP(hipMemsetAsync(cnt.p + nsef, 0, sizeof(int64_t), c.stream));
-    hipLaunchKernelGGL(k_ras_terms<false>, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p, cnt.p,
-                       nullptr, nullptr, nullptr, bad.p);
+    hipLaunchKernelGGL(k_ras_terms<false>, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p,
+                       c.d_rasorder.p, cnt.p, nullptr, nullptr, nullptr, bad.p);
     PSOCI_HIP(hipGetLastError());
     c.d_rastoff.alloc(nsef + 1);
     c.scan(cnt.p, c.d_rastoff.p, nsef + 1);
@@ -809,10 +1037,11 @@ bool build_ras(Ctx& c) {
     c.d_rasterm.alloc(nterm);
     c.d_rasscl.alloc(nsef);
     c.d_rasrows.alloc(nsef);
-    hipLaunchKernelGGL(k_ras_sefrows, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p, c.d_rasrows.p);
+    hipLaunchKernelGGL(k_ras_sefrows, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p,
+                       c.d_rasorder.p, c.d_rasrows.p);
     PSOCI_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_ras_terms<true>, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p, nullptr,
-                       c.d_rastoff.p, c.d_rasterm.p, c.d_rasscl.p, bad.p);
+    hipLaunchKernelGGL(k_ras_terms<true>, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p,
+                       c.d_rasorder.p, nullptr, c.d_rastoff.p, c.d_rasterm.p, c.d_rasscl.p, bad.p);
     PSOCI_HIP(hipGetLastError());
     int b = 0;
     bad.download(&b, 1, c.stream);

@@ -66,6 +66,9 @@ extern "C" int hrc_sigma(int nbf, int nelec, int ksym, int64_t ncfg, const uint8
       if (ras_cmp_var(C, oi, ii) != var[row]) return 9;
       uint64_t op, ir;
       ras_cmp_drop(v, C, oi, ii, op, ir);
+      int64_t r0, rows;
+      ras_cmp_group(C, oi, ii, r0, rows);
+      if (row < r0 || row >= r0 + rows) return 11;
       std::vector<double> D((size_t)C.nq * k, 0.0);
       std::vector<int> full(C.nq, -1);
       int n = 0;
@@ -88,7 +91,7 @@ extern "C" int hrc_sigma(int nbf, int nelec, int ksym, int64_t ncfg, const uint8
         for (int t = 0; t < k; ++t) {
           double acc = 0.0;
           for (int j = 0; j < C.nq; ++j) acc += G[(int64_t)full[a] * B.nqp + full[j]] * D[(size_t)j * k + t];
-          W[(C.wbase + row * C.nqp + a) * k + t] = acc;
+          W[ras_cmp_w(C, r0, rows, row, a) * k + t] = acc;
         }
     }
   }
