@@ -446,12 +446,20 @@ int psoci_rdm(psoci_ctx* ctx, int k, const double* C, const double* w, double* g
     PSOCI_CHECK(k >= 1 && C, PSOCI_ERR_ARG, "bad RDM arguments");
     const int64_t n = c.sp.nsef_total;
     const int64_t n1 = nndaf(c.sp.nbf), n2 = nndaf(n1);
-    if (!c.have_pairs) psoci::build_pairs(c);
+    // complete RAS spaces: the string plan (kept from the direct sigma, or
+    // built for this call unless the pair records are there already)
+    if (c.direct_engine_req != 1 && !c.have_ras && !c.ras_tried && !c.have_pairs) {
+      c.ras_tried = true;
+      psoci::build_ras(c);
+    }
+    const bool strings = c.direct_engine_req != 1 && c.have_ras && c.ras_rdm;
+    if (!strings && !c.have_pairs) psoci::build_pairs(c);
     psoci::DevBuf<double> dC, g1, g2;
     dC.upload(C, (size_t)n * k, c.stream);
     g1.alloc(n1);
     g2.alloc(n2);
-    psoci::rdm_grad(c, k, dC.p, w, g1.p, g2.p);
+    if (strings) psoci::ras_rdm_grad(c, k, dC.p, w, g1.p, g2.p);
+    else psoci::rdm_grad(c, k, dC.p, w, g1.p, g2.p);
     if (grad_one) g1.download(grad_one, n1, c.stream);
     if (grad_two) g2.download(grad_two, n2, c.stream);
     c.sync();

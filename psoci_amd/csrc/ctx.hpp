@@ -106,7 +106,7 @@ struct Ctx {
   DevBuf<int32_t> d_rasrem;
   DevBuf<RasBlockDev> d_rasblk;
   DevBuf<RasCmp> d_rascmp;
-  DevBuf<int16_t> d_raspidx;
+  DevBuf<int16_t> d_rasq, d_raspidx;
   DevBuf<RasTile> d_rastile[4];        // product tiles for chunks of 16, 8, 4 and 2 columns
   std::vector<RasLaunch> ras_launch[4];  // and their launches
   DevBuf<RasSef> d_rassef;
@@ -122,8 +122,17 @@ struct Ctx {
   DevBuf<int8_t> d_rasscl;      // per SEF: 0 1/sqrt(2), 1 sqrt(2), 2 one
   DevBuf<int32_t> d_rasorder;   // the order the SEFs are walked in (d_rastoff, d_rasscl, d_rasrows follow it)
   DevBuf<int2> d_rasrows;       // per SEF: signed rows of its determinants' coefficients
+  // the string-driven adjoint (rasrdm.hip): whether it equals the pair walk
+  // (no integral sum that the reference's blocks leave out), and its buffers
+  bool ras_rdm = false;
+  DevBuf<double> d_rdmm, d_rdmpart, d_rdmw;
+  DevBuf<char> d_rdmmat;
   void drop_ras() {
-    have_ras = ras_tried = false;
+    have_ras = ras_tried = ras_rdm = false;
+    d_rdmm.release();
+    d_rdmpart.release();
+    d_rdmw.release();
+    d_rdmmat.release();
     ras = RasPlan();
     d_rasmask.release();
     d_rascls.release();
@@ -131,6 +140,7 @@ struct Ctx {
     d_rasrem.release();
     d_rasblk.release();
     d_rascmp.release();
+    d_rasq.release();
     d_raspidx.release();
     for (int k = 0; k < 4; ++k) {
       d_rastile[k].release();
@@ -186,6 +196,11 @@ int64_t direct_det_pairs(Ctx& c);
 // (false when the space does not qualify; c.ras_why says why), and the sigma
 bool build_ras(Ctx& c);
 void sigma_ras(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy);
+// columns [col0, col0 + kw) of X [n][ldx] as FP64 determinant vectors in
+// c.d_rasc; returns their padded width (16, 8, 4 or 2)
+int ras_scatter64(Ctx& c, const double* X, int ldx, int col0, int kw);
+// the adjoint through the string plan (needs have_ras and ras_rdm)
+void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1, double* d_g2);
 // one timed sigma of k columns on internal buffers, averaged over reps: ms[5]
 // per launch group (scatter, products by kind, gather), flops[3] per kind
 void ras_timing(Ctx& c, int prec, int k, int reps, double* ms, double* flops);

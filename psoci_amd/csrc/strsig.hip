@@ -698,9 +698,9 @@ __global__ __launch_bounds__(256) void k_ras_y(const int64_t* __restrict__ toff,
   if (q < kw) Y[order[s] * (int64_t)ldy + col0 + q] = (TY)(f * (a0 + a1));
 }
 
-// Flags (*flag = 1) a configuration pair one electron apart whose
-// single-excitation sum vnt[0] is exactly zero in either orientation while
-// an exchange integral (e o|o f) its elements could use is not: the
+// Flags a configuration pair one electron apart whose single-excitation sum
+// vnt[0] is exactly zero in either orientation (bit 1), and one where an
+// exchange integral (e o|o f) its elements could use is not (bit 0): the
 // reference skips such a block (processSingleExcitation returns 0,
 // PsociHamiltonian.C:190-261), which the determinant Hamiltonian does not.
 __global__ __launch_bounds__(256) void k_ras_zero_singles(int64_t ncfg, const uint64_t* __restrict__ dm,
@@ -736,6 +736,7 @@ __global__ __launch_bounds__(256) void k_ras_zero_singles(int64_t ncfg, const ui
       pair_setup(P1, 1, 0, dI, sI, nI, dJ, sJ, nJ, nbf, one, two);
       pair_setup(P2, 1, 0, dJ, sJ, nJ, dI, sI, nI, nbf, one, two);
       if (P1.kind != 0 && P2.kind != 0) continue;
+      if (!(*(volatile int*)flag & 2)) atomicOr(flag, 2);
       for (uint64_t o = (dI | sI | dJ | sJ) & ~be & ~bf; o; o &= o - 1) {
         const int c = ctz(o);
         if (g2(two, e, c, c, f) != 0.0) {
@@ -937,7 +938,12 @@ bool build_ras(Ctx& c) {
     int f = 0;
     flag.download(&f, 1, c.stream);
     c.sync();
-    if (f) {
+    // the string-driven adjoint has no pairs that the reference leaves out
+    // (a double excitation both of whose integrals are exactly zero, a single
+    // one whose sum is)
+    c.ras_rdm = !(f & 2) && std::find(two.begin(), two.end(), 0.0) == two.end();
+    if (f & 1) {
+      c.ras_rdm = false;
       c.ras_why = "a configuration pair one electron apart has vnt[0] exactly zero with nonzero exchange terms";
       c.ras = RasPlan();
       return false;
@@ -949,6 +955,7 @@ bool build_ras(Ctx& c) {
   c.d_rasrem.upload(P.rem, c.stream);
   c.d_rasblk.upload(P.blk, c.stream);
   c.d_rascmp.upload(P.cmp, c.stream);
+  c.d_rasq.upload(P.qlist, c.stream);
   c.d_raspidx.upload(P.pidx, c.stream);
   c.d_rassef.upload(P.sef, c.stream);
   RasView v = ras_host_view(P);
@@ -957,7 +964,7 @@ bool build_ras(Ctx& c) {
   v.add = c.d_rasadd.p;
   v.rem = c.d_rasrem.p;
   v.blk = c.d_rasblk.p;
-  v.qlist = nullptr;
+  v.qlist = c.d_rasq.p;
   v.cmp = c.d_rascmp.p;
   v.wunit = P.cwunit;
   v.pidx = c.d_raspidx.p;
@@ -1093,6 +1100,27 @@ void ras_timing(Ctx& c, int prec, int k, int reps, double* ms, double* flops) {
     for (int g = 0; g < 3; ++g) flops[g] = 0.0;
     for (const RasCmp& C : c.ras.cmp) flops[C.kind] += 2.0 * (double)C.nrows * C.nq * C.nq * k;
   }
+}
+
+int ras_scatter64(Ctx& c, const double* X, int ldx, int col0, int kw) {
+  const int64_t nsef = (int64_t)c.ras.sef.size();
+  double* cv = reinterpret_cast<double*>(c.d_rasc.p);
+  const int kc = kw > 8 ? 16 : kw > 4 ? 8 : kw > 2 ? 4 : 2;
+  const dim3 grid(8 * nblk(nsef * kc, 8 * 256));
+  switch (kc) {
+#define PSOCI_RAS_SCATTER(KCV)                                                                                   \
+  case KCV:                                                                                                      \
+    hipLaunchKernelGGL((k_ras_x2c<double, KCV, double>), grid, dim3(256), 0, c.stream, nsef, c.ras.ndet,         \
+                       c.d_rasorder.p, c.d_rasrows.p, X, ldx, col0, kw, cv);                                     \
+    break;
+    PSOCI_RAS_SCATTER(16)
+    PSOCI_RAS_SCATTER(8)
+    PSOCI_RAS_SCATTER(4)
+    PSOCI_RAS_SCATTER(2)
+#undef PSOCI_RAS_SCATTER
+  }
+  PSOCI_HIP(hipGetLastError());
+  return kc;
 }
 
 void sigma_ras(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy) {
