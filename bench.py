@@ -175,8 +175,8 @@ def hbuild_measure(api, torch, with_cpu, reps=3):
            "output_bytes": int(out_bytes), "output_gbs": round(out_bytes / t / 1e9, 2),
            "tune_ms": round(float(np.median(tt)) * 1e3, 3),
            "note": ("median of 3 builds after a warm-up build (psoci_build_h_timing): every build screens the "
-                    "pairs, generates the blocks and packs the CSR anew; the stored sigma's shape autotuner that "
-                    "follows each build is tune_ms")}
+                    "pairs, generates the blocks and packs the CSR anew; the stored sigma's row-length classes and "
+                    "shapes that follow each build are tune_ms")}
     if with_cpu:
         import oracle
         threads = min(os.cpu_count() or 1, 16)

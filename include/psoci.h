@@ -164,7 +164,7 @@ int psoci_build_h(psoci_ctx* ctx, int64_t* nnz_lower);
 /* Wall time of the last psoci_build_h on this context, in seconds:
  * seconds[0] the build proper (pair screening, element blocks, packing into
  * CSR, the diagonal and the FP32 copy, synchronised), seconds[1] the stored
- * sigma's shape autotuner that follows it.  PSOCI_ERR_STATE before a build.
+ * sigma's row-length classes and shapes that follow it.  PSOCI_ERR_STATE before a build.
  * No reference counterpart (a measurement entry point; the reference's
  * build timers are PsociGAhamiltonian.C:2822-2839). */
 int psoci_build_h_timing(psoci_ctx* ctx, double* seconds);
@@ -299,21 +299,23 @@ int psoci_direct_schedule(psoci_ctx* ctx, int* order, int* chunk, double* tune_m
 int psoci_direct_schedule_prec(psoci_ctx* ctx, int prec, int* order, int* chunk, double* tune_ms);
 
 /* The stored sigma's kernel shape for precision prec (PSOCI_FP64 or
- * PSOCI_FP32) as chosen by the autotuner after psoci_build_h: lanes per
- * nonzero (1, 2, 4), rows per wavefront (1, 2, 4, 8) and the tuner's best
- * 16-column time in ms (-1 when fixed by the PSOCI_SPMM_SHAPE environment,
- * "<lanes>x<rows>").  No reference counterpart; any output may be NULL. */
+ * PSOCI_FP32) at 16 columns: lanes per nonzero (1, 2, 4) and rows per
+ * wavefront (1, 2, 4, 8), by a rule on the width, the precision and the row
+ * lengths or, for every width, as fixed by the PSOCI_SPMM_SHAPE environment
+ * ("<lanes>x<rows>") or a checkpoint with other shapes; tune_ms: -1, or the
+ * time a checkpoint's writer measured.  No reference counterpart; any output
+ * may be NULL. */
 int psoci_stored_shape(psoci_ctx* ctx, int prec, int* lanes_per_nz, int* rows_per_wave, double* tune_ms);
 
 /* The stored sigma's row-length buckets (full symmetric rows of length
  * < 64, 64-255, 256-1023, 1024-4095, >= 4096): rows[5] per bucket, the
- * tuner's shape for each (lanes_per_nz[5], rows_per_wave[5]), whether the
+ * 16-column shape of each (lanes_per_nz[5], rows_per_wave[5]), whether
  * per-bucket launches replace the single launch of psoci_stored_shape for
- * precision prec (*used: when they beat it by 3 % or more), and their
- * measured 16-column time (-1 when fewer than two buckets hold rows).  The
- * reference splits rows by length into its ELL table and the supplemental
- * overflow (PsociGAhamiltonian.C:4223-4312, 9325-9580); no other
- * counterpart.  Any output may be NULL. */
+ * precision prec (*used: when classes of a tenth of the nonzeros take
+ * another shape, or as PSOCI_SPMM_BUCKETS=0 / 1 fixes it), and bucketed_ms:
+ * -1 (nothing is timed).  The reference splits rows by length into its ELL
+ * table and the supplemental overflow (PsociGAhamiltonian.C:4223-4312,
+ * 9325-9580); no other counterpart.  Any output may be NULL. */
 int psoci_stored_buckets(psoci_ctx* ctx, int prec, int* used, int64_t* rows, int* lanes_per_nz, int* rows_per_wave,
                          double* bucketed_ms);
 

@@ -256,7 +256,7 @@ class Hamiltonian:
 
     def build_timing(self) -> dict:
         """Seconds of the last build(): the build proper and the stored
-        sigma's shape autotuner after it."""
+        sigma's row-length classes and shapes after it."""
         sec = np.zeros(2)
         self._check(self.L.psoci_build_h_timing(self._h, _p(sec)))
         return {"build_s": float(sec[0]), "tune_s": float(sec[1])}
@@ -441,7 +441,7 @@ class Hamiltonian:
         return {"order": o.value, "chunk": ch.value, "tune_ms": ms.value}
 
     def stored_shape(self, prec: int = FP32):
-        """The stored sigma's autotuned shape: dict(lanes_per_nz, rows_per_wave, tune_ms)."""
+        """The stored sigma's 16-column shape: dict(lanes_per_nz, rows_per_wave, tune_ms)."""
         g, r, ms = ctypes.c_int(), ctypes.c_int(), ctypes.c_double()
         self._check(self.L.psoci_stored_shape(self._h, prec, ctypes.byref(g), ctypes.byref(r), ctypes.byref(ms)))
         return {"lanes_per_nz": g.value, "rows_per_wave": r.value, "tune_ms": ms.value}

@@ -50,16 +50,18 @@ struct Ctx {
   DevBuf<double> d_val;       // full FP64
   DevBuf<float> d_val32;      // full FP32
   DevBuf<int32_t> d_lowcnt;   // per row: entries of the lower part (incl. diagonal)
-  // stored sigma shape per precision ([0] FP64, [1] FP32): lanes per
-  // nonzero, rows per wavefront, and the tuner's best 16-column time (-1: fixed)
+  // stored sigma shape per precision ([0] FP64, [1] FP32) at 16 columns:
+  // lanes per nonzero, rows per wavefront (spmm_fixed: for every width), and
+  // a tuner's time read from an older checkpoint (else -1)
+  bool spmm_fixed = false;
   int spmm_g[2] = {1, 1}, spmm_r[2] = {1, 1};
   double spmm_tune_ms[2] = {-1, -1};
   // row-length buckets (kSpmmBuckets length classes): the rows of each in
   // d_brows[spmm_boff[b] .. spmm_boff[b + 1]), a shape per bucket and
-  // precision, and whether the bucketed launches are used (set_buckets and
+  // precision, and whether the bucketed launches are used (count_buckets and
   // the tuner in sigma.hip)
   DevBuf<int32_t> d_brows;
-  int64_t spmm_boff[kSpmmBuckets + 1] = {0};
+  int64_t spmm_boff[kSpmmBuckets + 1] = {0}, spmm_bnnz[kSpmmBuckets] = {0};  // rows before, nonzeros of each
   int spmm_bg[2][kSpmmBuckets] = {}, spmm_br[2][kSpmmBuckets] = {};
   bool spmm_bucketed[2] = {false, false};
   double hbuild_seconds[2] = {-1.0, -1.0};  // last build_h: build proper, shape tuner
@@ -185,8 +187,14 @@ struct Ctx {
 void upload_space(Ctx& c);
 void build_pairs(Ctx& c);               // adjacency + determinant masks (direct sigma, adjoint)
 void build_h(Ctx& c);                   // stored Hamiltonian
-void tune_stored(Ctx& c);               // stored sigma shape autotuner (after build_h)
-void set_buckets(Ctx& c);               // the stored matrix's row-length buckets
+// a checkpoint's stored-sigma shapes
+struct SpmmSaved {
+  int g[2], r[2], bg[2][kSpmmBuckets], br[2][kSpmmBuckets];
+  bool bucketed[2];
+  double tune_ms[2];
+};
+// the stored sigma's shapes and row-length buckets (after build_h or a load)
+void tune_stored(Ctx& c, const SpmmSaved* saved = nullptr);
 void compute_diag(Ctx& c);              // diagonal only
 void block_on_device(Ctx& c, int64_t I, int64_t J, double* host_out, int* status);
 void sigma_stored(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy, const Staging& st = Staging{});

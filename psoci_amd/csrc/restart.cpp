@@ -301,20 +301,21 @@ void load_h(Ctx& c, const char* path) {
       for (int b = 0; b < kSpmmBuckets; ++b) shapes_ok = shapes_ok && lanes_ok(hb.lanes[p][b]) && rows_ok(hb.rows[p][b]);
     }
   }
-  if (shapes_ok && !std::getenv("PSOCI_SPMM_SHAPE")) {
-    // the writer's tuned stored-sigma shapes (and row-length buckets, which
-    // depend on the matrix alone): the same kernels, bit for bit
-    set_buckets(c);
+  if (shapes_ok) {
+    // the writer's stored-sigma shapes (and row-length buckets, which depend
+    // on the matrix alone): the same kernels, bit for bit
+    SpmmSaved sv;
     for (int p = 0; p < 2; ++p) {
-      c.spmm_g[p] = h.lanes[p];
-      c.spmm_r[p] = h.rows[p];
-      c.spmm_tune_ms[p] = h.tune_ms[p];
-      c.spmm_bucketed[p] = h.version == 2 && hb.used[p] == 1;
+      sv.g[p] = h.lanes[p];
+      sv.r[p] = h.rows[p];
+      sv.tune_ms[p] = h.tune_ms[p];
+      sv.bucketed[p] = h.version == 2 && hb.used[p] == 1;
       for (int b = 0; b < kSpmmBuckets; ++b) {
-        c.spmm_bg[p][b] = h.version == 2 ? hb.lanes[p][b] : 1;
-        c.spmm_br[p][b] = h.version == 2 ? hb.rows[p][b] : 1;
+        sv.bg[p][b] = h.version == 2 ? hb.lanes[p][b] : 1;
+        sv.br[p][b] = h.version == 2 ? hb.rows[p][b] : 1;
       }
     }
+    tune_stored(c, &sv);
   } else {
     tune_stored(c);
   }

@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 #include "ctx.hpp"
 #include "pad.hpp"
@@ -32,49 +33,160 @@ __device__ __forceinline__ float fmadd<float>(float a, float b, float c) {
   return __builtin_fmaf(a, b, c);
 }
 
+template <typename T, int N>
+struct PieceOf {
+  typedef T type __attribute__((ext_vector_type(N)));
+  typedef T loose __attribute__((ext_vector_type(N), aligned(sizeof(T))));  // any start of a row
+};
+
+// the value that lane g of this lane's group of G holds (G = 1, 2, 4: groups
+// lie within quads, one DPP move per 32 bits)
+template <int G, int g>
+__device__ __forceinline__ int32_t of_lane(int32_t x) {
+  if constexpr (G == 1) return x;
+  constexpr int ctrl = G == 2 ? (g | g << 2 | (2 + g) << 4 | (2 + g) << 6) : (g | g << 2 | g << 4 | g << 6);
+  return __builtin_amdgcn_mov_dpp(x, ctrl, 0xf, 0xf, true);
+}
+template <int G, int g>
+__device__ __forceinline__ float of_lane(float x) {
+  return __int_as_float(of_lane<G, g>(__float_as_int(x)));
+}
+template <int G, int g>
+__device__ __forceinline__ double of_lane(double x) {
+  return __hiloint2double(of_lane<G, g>(__double2hiint(x)), of_lane<G, g>(__double2loint(x)));
+}
+
 // R rows per wavefront (64/R lanes per row: short rows share a wavefront)
 // and G lanes per nonzero (each of them multiplies K/G of the K columns, so
-// the G lanes of a nonzero read one contiguous piece of its x row).  Lanes
-// of a row stride over its nonzeros; partial sums are reduced across the
-// nonzero slots of the row with shuffles.  (R, G) = (1, 1) is one wavefront
-// per row with whole x rows per lane.  rows (optional): the launch covers
-// the nrows rows listed there (one row-length bucket) instead of 0..n-1.
+// the G lanes of a nonzero read one contiguous piece of its x row).  In a
+// turn every lane of a row loads the columns and values of U consecutive
+// nonzeros (16-byte loads, one turn ahead), and the groups of G lanes walk
+// their G U nonzeros, each taken from the lane that holds it.  Four (two at 64
+// bytes of x per lane) accumulators per column, so that the chains are no
+// longer than with one row per wavefront.  Partial sums are reduced across the
+// groups of the row with shuffles.  rows (optional): the launch covers the
+// nrows rows listed there (one row-length bucket) instead of 0..n-1.
+// Bound by the matrix stream and the x gathers from L2 (a 64-byte row piece
+// per nonzero).  31,650 rows of 715 nonzeros (10 orbitals, 8 electrons), each
+// call on another matrix than the last: FP32 16 columns 169 -> 125 us, FP64 4
+// / 16 columns 200 -> 114 / 218 -> 185 us against lanes that loaded every
+// nonzero of their group themselves, one at a time.
 template <typename T, int K, int G, int R>
 __global__ __launch_bounds__(256) void k_spmm(int64_t nrows, const int32_t* __restrict__ rows,
                                               const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                                               const T* __restrict__ val, const T* __restrict__ X, int ldx,
                                               T* __restrict__ Y, int ldy) {
   constexpr int LR = kWave / R;   // lanes per row
-  constexpr int NS = LR / G;      // nonzero slots per row
   constexpr int C = K / G;        // columns per lane
+  constexpr int U = 8;            // nonzeros a lane loads per turn
+  constexpr int XB = C * sizeof(T) >= 64 ? 4 : 8;  // of which so many x pieces are in flight
+  constexpr int PW = C * sizeof(T) % 16 == 0 ? 16 / sizeof(T) : 1;  // values per x load
+  constexpr int NA = C * sizeof(T) <= 32 ? 4 : 2;                   // accumulators per column
+  constexpr int VW = 16 / sizeof(T);                                // values per load
+  typedef typename PieceOf<T, PW>::type V;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t slot_r =
       ((int64_t)blockIdx.x * (blockDim.x / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave)) * R + lane / LR;
   const bool live = slot_r < nrows;
   const int64_t r = live ? (rows ? (int64_t)rows[slot_r] : slot_r) : 0;
-  const int lr = lane % LR, slot = lr / G, cc = lr % G;
-  T acc[C];
+  const int lr = lane % LR, cc = lr % G;
+  T acc[NA][C];
 #pragma unroll
-  for (int v = 0; v < C; ++v) acc[v] = (T)0;
-  if (live) {
-    const int64_t lo = rowptr[r], hi = rowptr[r + 1];
-    for (int64_t q = lo + slot; q < hi; q += NS) {
-      const T a = val[q];
-      const T* __restrict__ x = X + (int64_t)col[q] * ldx + cc * C;
+  for (int x = 0; x < NA; ++x)
 #pragma unroll
-      for (int v = 0; v < C; ++v) acc[v] = fmadd(a, x[v], acc[v]);
+    for (int v = 0; v < C; ++v) acc[x][v] = (T)0;
+  const int64_t lo = live ? rowptr[r] : 0;
+  const int len = live ? (int)(rowptr[r + 1] - lo) : 0;
+  const T* __restrict__ vr = val + lo;
+  const int32_t* __restrict__ cr = col + lo;
+  const T* __restrict__ xc = X + cc * C;
+  // this lane's nonzeros of a turn; past the row's end the row's last one,
+  // its column complemented: left out of the sums
+  T a[U];
+  int32_t j[U];
+  auto fetch = [&](int q) {
+    if (q + U <= len) {
+#pragma unroll
+      for (int u = 0; u < U; u += VW) {
+        const auto t = *reinterpret_cast<const typename PieceOf<T, VW>::loose*>(vr + q + u);
+#pragma unroll
+        for (int i = 0; i < VW; ++i) a[u + i] = t[i];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u += 4) {
+        const auto t = *reinterpret_cast<const typename PieceOf<int32_t, 4>::loose*>(cr + q + u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) j[u + i] = t[i];
+      }
+    } else if (len > 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int t = q + u < len ? q + u : len - 1;
+        a[u] = vr[t];
+        j[u] = q + u < len ? cr[t] : ~cr[t];
+      }
+    }
+  };
+  const int q = lr * U;  // this lane's first nonzero of the turn
+  int base = 0;
+  if (len > 0) fetch(q);
+  while (base < len) {
+    T b[U];
+    int32_t jj[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      b[u] = a[u];
+      jj[u] = j[u];
+    }
+    base += LR * U;
+    if (base < len) fetch(q + base);
+    auto sub = [&](auto gc) {
+      constexpr int g = decltype(gc)::value;
+#pragma unroll
+      for (int h = 0; h < U; h += XB) {
+        V xv[XB][C / PW];
+        T w[XB];
+        int32_t c[XB];
+#pragma unroll
+        for (int u = 0; u < XB; ++u) {
+          c[u] = of_lane<G, g>(jj[h + u]);
+          w[u] = of_lane<G, g>(b[h + u]);
+          const V* x = reinterpret_cast<const V*>(xc + (int64_t)(c[u] < 0 ? ~c[u] : c[u]) * ldx);
+#pragma unroll
+          for (int p = 0; p < C / PW; ++p) xv[u][p] = x[p];
+        }
+#pragma unroll
+        for (int u = 0; u < XB; ++u)
+#pragma unroll
+          for (int v = 0; v < C; ++v) {
+            const T f = fmadd(w[u], xv[u][v / PW][v % PW], acc[u % NA][v]);
+            acc[u % NA][v] = c[u] < 0 ? acc[u % NA][v] : f;
+          }
+      }
+    };
+    sub(std::integral_constant<int, 0>{});
+    if constexpr (G >= 2) sub(std::integral_constant<int, 1>{});
+    if constexpr (G >= 4) {
+      sub(std::integral_constant<int, 2>{});
+      sub(std::integral_constant<int, 3>{});
     }
   }
-  // reduce over the nonzero slots of the row (lane bits G .. LR-1)
+  T sum[C];
+#pragma unroll
+  for (int v = 0; v < C; ++v) {
+    sum[v] = acc[0][v] + acc[1][v];
+    if constexpr (NA == 4) sum[v] += acc[2][v] + acc[3][v];
+  }
+  // reduce over the groups of the row (lane bits G .. LR-1)
 #pragma unroll
   for (int off = G; off < LR; off <<= 1) {
 #pragma unroll
-    for (int v = 0; v < C; ++v) acc[v] += __shfl_xor(acc[v], off, kWave);
+    for (int v = 0; v < C; ++v) sum[v] += __shfl_xor(sum[v], off, kWave);
   }
-  if (live && slot == 0) {
+  if (live && lr < G) {
     T* y = Y + r * ldy + cc * C;
 #pragma unroll
-    for (int v = 0; v < C; ++v) y[v] = acc[v];
+    for (int v = 0; v < C; ++v) y[v] = sum[v];
   }
 }
 
@@ -120,19 +232,47 @@ void launch_shape(Ctx& c, int g0, int r, const T* val, const T* X, int ldx, T* Y
   launch_gr<T, K, 1, 1>(c, val, X, ldx, Y, ldy, rows, nrows);
 }
 
-// the tuned shape(s) of this precision: one launch over all rows, or one
-// per non-empty row-length bucket with that bucket's shape
+// Shape rule of a launch of K columns: each lane reads 16 bytes of an x row
+// (G = K sizeof / 16 lanes, at most 4), eight rows share a wavefront (64
+// nonzeros of each are in flight per turn), four where FP32 sums would get
+// longer chains (G = 4), one for rows that fill a wavefront many times over,
+// fewer where the launch would not fill the GPU.  us per call on that matrix
+// (G x R): FP32 1 / 4 / 8 / 16 / 32 columns 1x8 70 / 1x8 89 / 2x8 102 / 4x4 125
+// / 4x4 172, against 1x4 76 / 96 / 140 / 210 / 413; FP64 1x8 91 / 2x8 114 / 4x8
+// 134 / 4x8 185 / 4x8 479, against 1x4 98 / 149 / 220 / 440 / 805.
+struct SpmmShape {
+  int g, r;
+};
+inline int spmm_rows_of_len(size_t es, int g, double len) {
+  if (len > 4096.0) return 1;
+  return es == 4 && g == 4 ? 4 : 8;
+}
+inline SpmmShape spmm_shape(size_t es, int K, int64_t rows, double len) {
+  SpmmShape s;
+  s.g = std::max(1, std::min(4, (int)(K * es) / 16));
+  s.r = spmm_rows_of_len(es, s.g, len);
+  while (s.r > 1 && rows < (int64_t)2048 * s.r) s.r >>= 1;
+  return s;
+}
+
+// one launch over all rows, or one per non-empty row-length bucket; the
+// rule's shape, or the fixed one
 template <typename T, int K>
 void launch_spmm(Ctx& c, const T* val, const T* X, int ldx, T* Y, int ldy) {
   const int pi = sizeof(T) == 4 ? 1 : 0;
   if (!c.spmm_bucketed[pi]) {
-    launch_shape<T, K>(c, c.spmm_g[pi], c.spmm_r[pi], val, X, ldx, Y, ldy, nullptr, c.sp.nsef_total);
+    const int64_t n = c.sp.nsef_total;
+    SpmmShape s = spmm_shape(sizeof(T), K, n, (double)c.nnz_full / (double)n);
+    if (c.spmm_fixed) s = {c.spmm_g[pi], c.spmm_r[pi]};
+    launch_shape<T, K>(c, s.g, s.r, val, X, ldx, Y, ldy, nullptr, n);
     return;
   }
   for (int b = 0; b < kSpmmBuckets; ++b) {
     const int64_t lo = c.spmm_boff[b], cnt = c.spmm_boff[b + 1] - lo;
-    if (cnt > 0)
-      launch_shape<T, K>(c, c.spmm_bg[pi][b], c.spmm_br[pi][b], val, X, ldx, Y, ldy, c.d_brows.p + lo, cnt);
+    if (cnt <= 0) continue;
+    SpmmShape s = spmm_shape(sizeof(T), K, cnt, (double)c.spmm_bnnz[b] / (double)cnt);
+    if (c.spmm_fixed) s = {c.spmm_bg[pi][b], c.spmm_br[pi][b]};
+    launch_shape<T, K>(c, s.g, s.r, val, X, ldx, Y, ldy, c.d_brows.p + lo, cnt);
   }
 }
 
@@ -152,124 +292,134 @@ void spmm_any_k(Ctx& c, const T* val, int k, const T* X, int ldx, T* Y, int ldy,
 
 }  // namespace
 
-// Shape autotuner of the stored sigma: for each precision, every (lanes per
-// nonzero, rows per wavefront) pair times the 16-column product on the built
-// matrix (best of two after a warm-up) and the fastest is kept for all
-// widths.  PSOCI_SPMM_SHAPE=<G>x<R> fixes it instead.
-// best of two timed 16-column launches (after a warm-up) of f
-template <class F>
-double time_ms(Ctx& c, hipEvent_t e0, hipEvent_t e1, F&& f) {
-  double t = 1e300;
-  for (int rep = 0; rep < 3; ++rep) {
-    PSOCI_HIP(hipEventRecord(e0, c.stream));
-    f();
-    PSOCI_HIP(hipEventRecord(e1, c.stream));
-    PSOCI_HIP(hipEventSynchronize(e1));
-    float ms = 0.f;
-    PSOCI_HIP(hipEventElapsedTime(&ms, e0, e1));
-    if (rep > 0) t = std::min(t, (double)ms);
-  }
-  return t;
-}
+namespace {
+const int64_t kBucketLim[kSpmmBuckets] = {64, 256, 1024, 4096, INT64_MAX};
 
-// Per precision: the best (lanes per nonzero, rows per wavefront) for all
-// rows in one launch, and the best for each row-length bucket on its own;
-// the bucketed launches are kept when together they beat the single one by
-// 3 % or more (PSOCI_SPMM_BUCKETS=0 / 1 fixes the choice).
-template <typename T>
-double tune_prec(Ctx& c, const T* val, hipEvent_t e0, hipEvent_t e1) {
-  const int pi = sizeof(T) == 4 ? 1 : 0;
-  const int64_t n = c.sp.nsef_total;
-  const int K = 16;
-  DevBuf<T> X, Y;
-  X.alloc((size_t)n * K);
-  Y.alloc((size_t)n * K);
-  PSOCI_HIP(hipMemsetAsync(X.p, 0, (size_t)n * K * sizeof(T), c.stream));
-  const int gs[] = {1, 2, 4}, rs[] = {1, 2, 4, 8};
-  auto best_shape = [&](const int32_t* rows, int64_t nrows, int& bg, int& br) {
-    double best = 1e300;
-    bg = br = 1;
-    for (int g : gs)
-      for (int r : rs) {
-        const double t = time_ms(c, e0, e1, [&] { launch_shape<T, 16>(c, g, r, val, X.p, K, Y.p, K, rows, nrows); });
-        if (t < best) {
-          best = t;
-          bg = g;
-          br = r;
-        }
-      }
-    return best;
-  };
-  c.spmm_bucketed[pi] = false;
-  const double single = best_shape(nullptr, n, c.spmm_g[pi], c.spmm_r[pi]);
-  int nonempty = 0;
-  for (int b = 0; b < kSpmmBuckets; ++b) {
-    const int64_t cnt = c.spmm_boff[b + 1] - c.spmm_boff[b];
-    c.spmm_bg[pi][b] = c.spmm_br[pi][b] = 1;
-    if (cnt > 0) {
-      ++nonempty;
-      best_shape(c.d_brows.p + c.spmm_boff[b], cnt, c.spmm_bg[pi][b], c.spmm_br[pi][b]);
-    }
+// rows (out[b]) and nonzeros (out[kSpmmBuckets + b]) per row-length class
+__global__ __launch_bounds__(256) void k_bucket_count(int64_t n, const int64_t* __restrict__ rowptr,
+                                                      unsigned long long* __restrict__ out) {
+  __shared__ unsigned long long cnt[2 * kSpmmBuckets];
+  if (threadIdx.x < 2 * kSpmmBuckets) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t len = rowptr[r + 1] - rowptr[r];
+    const int b = len < 64 ? 0 : len < 256 ? 1 : len < 1024 ? 2 : len < 4096 ? 3 : 4;
+    atomicAdd(&cnt[b], 1ull);
+    atomicAdd(&cnt[kSpmmBuckets + b], (unsigned long long)len);
   }
-  if (nonempty > 1) {
-    c.spmm_bucketed[pi] = true;
-    const double bucketed = time_ms(c, e0, e1, [&] { launch_spmm<T, 16>(c, val, X.p, K, Y.p, K); });
-    c.spmm_bucketed[pi] = bucketed < 0.97 * single;
-    c.spmm_bucket_ms[pi] = bucketed;
-    // PSOCI_SPMM_BUCKETS=0 / 1 fixes the choice instead
-    if (const char* eb = std::getenv("PSOCI_SPMM_BUCKETS")) c.spmm_bucketed[pi] = eb[0] == '1';
-  } else {
-    c.spmm_bucket_ms[pi] = -1.0;
-  }
-  return c.spmm_bucketed[pi] ? c.spmm_bucket_ms[pi] : single;
+  __syncthreads();
+  if (threadIdx.x < 2 * kSpmmBuckets && cnt[threadIdx.x]) atomicAdd(&out[threadIdx.x], cnt[threadIdx.x]);
 }
+__global__ void k_bucket_zero(unsigned long long* out) {
+  if (threadIdx.x < 2 * kSpmmBuckets) out[threadIdx.x] = 0;
+}
+}  // namespace
 
 // Row-length buckets of the stored matrix (full symmetric rows): lengths
 // < 64, 64-255, 256-1023, 1024-4095, >= 4096; the row lists in ascending
-// order per bucket.  A property of the matrix alone, so a loaded checkpoint
-// gets the same buckets.
-void set_buckets(Ctx& c) {
+// order per bucket, made when the bucketed launches are used.  A property of
+// the matrix alone, so a loaded checkpoint gets the same buckets.
+static void count_buckets(Ctx& c) {
+  const int64_t n = c.sp.nsef_total;
+  DevBuf<unsigned long long> d;
+  d.alloc(2 * kSpmmBuckets);
+  hipLaunchKernelGGL(k_bucket_zero, dim3(1), dim3(64), 0, c.stream, d.p);
+  hipLaunchKernelGGL(k_bucket_count, dim3((unsigned)std::min<int64_t>(256, (n + 255) / 256)), dim3(256), 0, c.stream, n,
+                     c.d_rowptr.p, d.p);
+  PSOCI_HIP(hipGetLastError());
+  unsigned long long h[2 * kSpmmBuckets];
+  d.download(h, 2 * kSpmmBuckets, c.stream);
+  c.sync();
+  c.spmm_boff[0] = 0;
+  for (int b = 0; b < kSpmmBuckets; ++b) {
+    c.spmm_boff[b + 1] = c.spmm_boff[b] + (int64_t)h[b];
+    c.spmm_bnnz[b] = (int64_t)h[kSpmmBuckets + b];
+  }
+}
+static void list_buckets(Ctx& c) {
   const int64_t n = c.sp.nsef_total;
   std::vector<int64_t> rp(n + 1);
   c.d_rowptr.download(rp.data(), n + 1, c.stream);
   c.sync();
   std::vector<int32_t> rows;
   rows.reserve(n);
-  const int64_t lim[kSpmmBuckets] = {64, 256, 1024, 4096, INT64_MAX};
-  c.spmm_boff[0] = 0;
   for (int b = 0; b < kSpmmBuckets; ++b) {
-    const int64_t lo = b ? lim[b - 1] : 0;
+    const int64_t lo = b ? kBucketLim[b - 1] : 0;
     for (int64_t r = 0; r < n; ++r) {
       const int64_t len = rp[r + 1] - rp[r];
-      if (len >= lo && len < lim[b]) rows.push_back((int32_t)r);
+      if (len >= lo && len < kBucketLim[b]) rows.push_back((int32_t)r);
     }
-    c.spmm_boff[b + 1] = (int64_t)rows.size();
   }
   c.d_brows.upload(rows, c.stream);
   c.sync();
 }
 
-void tune_stored(Ctx& c) {
-  set_buckets(c);
-  c.spmm_bucketed[0] = c.spmm_bucketed[1] = false;
-  const char* env = std::getenv("PSOCI_SPMM_SHAPE");
-  if (env) {
+// The stored sigma's shapes (spmm_shape; those at 16 columns are reported)
+// and whether the rows are launched by length class: where the classes of at
+// least a tenth of the nonzeros take another R than the mean row does.
+// PSOCI_SPMM_SHAPE=<G>x<R> fixes one shape for every width,
+// PSOCI_SPMM_BUCKETS=0 / 1 the other choice.  saved (a checkpoint's shapes):
+// kept, and fixed where they are not the rule's.
+void tune_stored(Ctx& c, const SpmmSaved* saved) {
+  count_buckets(c);
+  const int64_t n = c.sp.nsef_total;
+  const double mean = n ? (double)c.nnz_full / (double)n : 0.0;
+  c.spmm_fixed = false;
+  int eg = 0, er = 0;
+  if (const char* env = std::getenv("PSOCI_SPMM_SHAPE")) {
     int g = 1, r = 1;
     if (std::sscanf(env, "%dx%d", &g, &r) == 2 && (g == 1 || g == 2 || g == 4) &&
         (r == 1 || r == 2 || r == 4 || r == 8)) {
-      c.spmm_g[0] = c.spmm_g[1] = g;
-      c.spmm_r[0] = c.spmm_r[1] = r;
+      eg = g;
+      er = r;
+      c.spmm_fixed = true;
+      saved = nullptr;
     }
-    c.spmm_tune_ms[0] = c.spmm_tune_ms[1] = -1.0;
-    return;
   }
-  hipEvent_t e0, e1;
-  PSOCI_HIP(hipEventCreate(&e0));
-  PSOCI_HIP(hipEventCreate(&e1));
-  c.spmm_tune_ms[1] = tune_prec<float>(c, c.d_val32.p, e0, e1);
-  c.spmm_tune_ms[0] = tune_prec<double>(c, c.d_val.p, e0, e1);
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  for (int pi = 0; pi < 2; ++pi) {
+    const size_t es = pi ? 4 : 8;
+    const SpmmShape s = spmm_shape(es, 16, n, mean);
+    c.spmm_g[pi] = eg ? eg : s.g;
+    c.spmm_r[pi] = er ? er : s.r;
+    c.spmm_tune_ms[pi] = c.spmm_bucket_ms[pi] = -1.0;
+    int64_t other = 0;
+    int nonempty = 0;
+    for (int b = 0; b < kSpmmBuckets; ++b) {
+      const int64_t cnt = c.spmm_boff[b + 1] - c.spmm_boff[b];
+      c.spmm_bg[pi][b] = eg ? eg : 1;
+      c.spmm_br[pi][b] = er ? er : 1;
+      if (cnt <= 0) continue;
+      ++nonempty;
+      const double len = (double)c.spmm_bnnz[b] / (double)cnt;
+      const SpmmShape t = spmm_shape(es, 16, cnt, len);
+      if (!eg) {
+        c.spmm_bg[pi][b] = t.g;
+        c.spmm_br[pi][b] = t.r;
+      }
+      if (spmm_rows_of_len(es, s.g, len) != spmm_rows_of_len(es, s.g, mean)) other += c.spmm_bnnz[b];
+    }
+    c.spmm_bucketed[pi] = nonempty > 1 && 10 * other >= c.nnz_full;
+    if (const char* eb = std::getenv("PSOCI_SPMM_BUCKETS")) c.spmm_bucketed[pi] = nonempty > 1 && eb[0] == '1';
+    if (eg) c.spmm_bucketed[pi] = false;
+    if (!saved) continue;
+    bool same = saved->g[pi] == c.spmm_g[pi] && saved->r[pi] == c.spmm_r[pi];
+    for (int b = 0; b < kSpmmBuckets; ++b)
+      if (saved->bucketed[pi])
+        same = same && saved->bg[pi][b] == c.spmm_bg[pi][b] && saved->br[pi][b] == c.spmm_br[pi][b];
+    if (!same) c.spmm_fixed = true;
+  }
+  if (saved)
+    for (int pi = 0; pi < 2; ++pi) {
+      c.spmm_g[pi] = saved->g[pi];
+      c.spmm_r[pi] = saved->r[pi];
+      c.spmm_tune_ms[pi] = saved->tune_ms[pi];
+      c.spmm_bucketed[pi] = saved->bucketed[pi];
+      for (int b = 0; b < kSpmmBuckets; ++b) {
+        c.spmm_bg[pi][b] = saved->bg[pi][b];
+        c.spmm_br[pi][b] = saved->br[pi][b];
+      }
+    }
+  if (c.spmm_bucketed[0] || c.spmm_bucketed[1]) list_buckets(c);
 }
 
 void sigma_stored(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy, const Staging& st) {
