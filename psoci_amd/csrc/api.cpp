@@ -236,6 +236,7 @@ int psoci_direct_engine(psoci_ctx* ctx, int request, int* engine) {
   return guarded(ctx, [&](Ctx& c) {
     PSOCI_CHECK(request >= -1 && request <= 2, PSOCI_ERR_ARG, "request must be -1, 0, 1 or 2");
     const int before = c.direct_engine_req;
+    const bool tried = c.ras_tried;
     if (request >= 0) {
       c.direct_engine_req = request;
       if (request == 1 && c.have_ras) c.drop_ras();
@@ -247,6 +248,7 @@ int psoci_direct_engine(psoci_ctx* ctx, int request, int* engine) {
         psoci::build_direct(c);
       } catch (...) {
         c.direct_engine_req = before;  // a request that cannot be met leaves the choice as it was
+        if (!c.have_ras) c.ras_tried = tried;
         throw;
       }
       *engine = psoci::direct_engine(c);

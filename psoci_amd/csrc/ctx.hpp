@@ -122,6 +122,7 @@ struct Ctx {
   int64_t ras_nterm = 0;        // terms over all SEFs (after merging mirrored pairs)
   DevBuf<int32_t> d_rasterm;    // signed W offsets (bit 31: negative)
   DevBuf<int8_t> d_rasscl;      // per SEF: 0 1/sqrt(2), 1 sqrt(2), 2 one
+  DevBuf<int32_t> d_rasabsent;  // determinants of no SEF (a list that is part of its space)
   DevBuf<int32_t> d_rasorder;   // the order the SEFs are walked in (d_rastoff, d_rasscl, d_rasrows follow it)
   DevBuf<int2> d_rasrows;       // per SEF: signed rows of its determinants' coefficients
   // the string-driven adjoint (rasrdm.hip): whether it equals the pair walk
@@ -160,6 +161,7 @@ struct Ctx {
     d_rasscl.release();
     d_rasrows.release();
     d_rasorder.release();
+    d_rasabsent.release();
   }
 
   // transition Hamiltonian (rows: this list's SEFs; columns: a second
@@ -218,7 +220,9 @@ void ras_timing(Ctx& c, int prec, int k, int reps, double* ms, double* flops);
 void build_direct(Ctx& c);
 // the engine a direct sigma uses with what is built now (0: none yet)
 inline int direct_engine(const Ctx& c) {
-  if (c.direct_engine_req != 1 && c.have_ras) return 2;
+  // (a plan of the automatic choice's wider spaces does not serve a request)
+  const bool wide = c.ras.fill < 1.0 || c.ras.frac;
+  if (c.have_ras && (c.direct_engine_req == 0 || (c.direct_engine_req == 2 && !wide))) return 2;
   if (c.direct_engine_req != 2 && c.have_pairs) return 1;
   return 0;
 }

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <numeric>
 
@@ -48,8 +49,10 @@ const Binom& binom() {
 // The RAS description: the external orbitals E (orbitals ordered by how many
 // configurations occupy them; the least occupied form E) and the largest
 // external electron count m, such that the list holds exactly every
-// occupation with at most m electrons in E.  False when no split fits.
-bool detect(const Space& sp, uint64_t& emask, int& m) {
+// occupation with at most m electrons in E.  False when no split fits; with
+// partial set, the split whose space holds the list with the fewest
+// configurations then (*fill: the list's share of it).
+bool detect(const Space& sp, uint64_t& emask, int& m, bool partial, double& fill) {
   const int nbf = sp.nbf;
   const int64_t ncfg = sp.ncfg;
   std::vector<std::pair<uint64_t, uint64_t>> keys(ncfg);
@@ -62,6 +65,7 @@ bool detect(const Space& sp, uint64_t& emask, int& m) {
   std::vector<int> order(nbf);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cnt[x] > cnt[y]; });
+  double best = 0.0;
   for (int t = nbf; t >= 1; --t) {
     uint64_t e = 0;
     for (int i = t; i < nbf; ++i) e |= 1ull << order[i];
@@ -72,10 +76,17 @@ bool detect(const Space& sp, uint64_t& emask, int& m) {
     if (expect == (double)ncfg) {
       emask = e;
       m = mm;
+      fill = 1.0;
       return true;
     }
+    if (partial && mm < kRasMaxCls && (best == 0.0 || expect < best)) {
+      best = expect;
+      emask = e;
+      m = mm;
+    }
   }
-  return false;
+  fill = best > 0.0 ? (double)ncfg / best : 0.0;
+  return best > 0.0;
 }
 
 struct Ranker {
@@ -103,6 +114,49 @@ struct Ranker {
     r = ri * B(nE, ke) + re;
   }
 };
+
+// Whether the products of a general plan (a part of a space, or an odd
+// electron count) cost less than the list's pair records, for 8 FP64 columns:
+// the products (rows times the square of their live pairs) at 45 TFLOP/s plus
+// W at 12 TB/s plus a dozen launches, the records at 8e10 connected
+// determinant pairs a second, of which the list has about its squared share
+// of the space's.  Measured on MI355X (us, strings / records): 8 + 24
+// orbitals, 6 electrons, a share of 0.1 / 0.15 / 0.2 / 0.3 / 0.6 / 0.9: 840 to
+// 920 / 501, 705, 1056, 2076, 6449, 14838; 6 + 12 orbitals, 6 electrons, 0.3:
+// 110 / 300; odd electron counts, 8 + 24 orbitals, 5 electrons: 499 / 8425;
+// 5 + 8 orbitals, 3 electrons: 75 / 51.  The records' set-up (their schedule
+// is timed) takes two to twelve times the strings'.  Counted from the space
+// alone, before any table is built.
+bool strings_pay(int nI, int nE, int m, const std::vector<std::pair<int, int>>& secs, bool sym, double fill) {
+  const Binom& Bn = binom();
+  double flops = 0.0, w = 0.0;
+  auto strings = [&](int n, int c) -> double { return n < c ? 0.0 : (double)Bn(nI, n - c) * (double)Bn(nE, c); };
+  for (const auto& s : secs) {
+    const bool half = sym && s.first == s.second;
+    for (int cu = 0; cu <= m; ++cu)
+      for (int cw = 0; cw + cu <= m; ++cw) {
+        const int b = m - cu - cw;
+        if (s.first >= 1 && s.second >= 1) {
+          const double u = nI - (s.first - 1 - cu), r = nI - (s.second - 1 - cw);
+          const double d = u * r + (b >= 1 ? (u + r) * nE : 0.0) + (b >= 2 ? (double)nE * nE : 0.0);
+          const double rows = strings(s.first - 1, cu) * strings(s.second - 1, cw) * (half ? 0.5 : 1.0);
+          flops += 2.0 * rows * d * d;
+          w += rows * d;
+        }
+        for (int spin = 0; spin < (half ? 1 : 2); ++spin) {
+          const int n = spin ? s.second : s.first, o = spin ? s.first : s.second;
+          if (n < 2) continue;
+          const double u = nI - (n - 2 - cu);
+          const double d = u * (u - 1) / 2 + (b >= 1 ? u * nE : 0.0) + (b >= 2 ? nE * (nE - 1.0) / 2 : 0.0);
+          const double rows = strings(n - 2, cu) * strings(o, cw);
+          flops += 2.0 * rows * d * d;
+          w += rows * d;
+        }
+      }
+  }
+  const double pairs = 0.5 * flops * fill * fill;
+  return 45e-6 + pairs / 8e10 > 70e-6 + 8.0 * flops / 45e12 + 128.0 * w / 12e12;
+}
 
 // The compact layout of block B (RasCmp), appended to the plan's totals.
 // Level: the cheapest in multiply-adds over the tiles' rows (groups padded
@@ -174,20 +228,20 @@ RasCmp compact(RasPlan& P, const RasBlockDev& B, int nI, int nE) {
 
 }  // namespace
 
-void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two) {
+void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two, bool general, bool all) {
   P = RasPlan();
   const int nbf = sp.nbf, N = sp.nelec;
   auto fail = [&](const char* why) {
     P.ok = false;
     P.why = why;
   };
-  if (sp.frac) return fail("odd electron count (one determinant per SEF)");
+  if (sp.frac && !general) return fail("odd electron count (one determinant per SEF)");
   if (sp.odd) return fail("ODD determinant class");
   if (sp.mixed) return fail("configurations of more than one jsym");
   if (N < 2 || N > kRasMaxN) return fail("electron count outside 2..32");
   uint64_t emask = 0;
   int m = 0;
-  if (!detect(sp, emask, m)) return fail("not a complete RAS configuration space");
+  if (!detect(sp, emask, m, general, P.fill)) return fail("not a complete RAS configuration space");
   if (m >= kRasMaxCls) return fail("more than 6 external electrons");
   P.nbf = nbf;
   P.N = N;
@@ -198,9 +252,23 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two)
   rk.init(nbf, emask);
   const Binom& Bn = binom();
 
-  // sectors n_alpha - n_beta = 0, 4, 8, ... (the EVEN class's Ms = 0, 2, 4, ...)
+  P.frac = sp.frac;
+  // sectors n_alpha - n_beta = 0, 4, 8, ... (the EVEN class's Ms = 0, 2, 4,
+  // ...); with an odd electron count 1, -3, 5, ... (one determinant per SEF;
+  // negated where alpha and beta are swapped)
   std::vector<std::pair<int, int>> secs;
-  for (int dn = 0; dn <= N; dn += 4) secs.push_back({(N + dn) / 2, (N - dn) / 2});
+  if (sp.frac) {
+    if (N + 1 > 2 * (kRasMaxN / 4 + 1)) return fail("more than 9 spin sectors");
+    for (int x = 1; x <= N; x += 2) {
+      const int dn = ((x % 4 == 1) != sp.flag0) ? x : -x;
+      secs.push_back({(N + dn) / 2, (N - dn) / 2});
+    }
+  } else {
+    for (int dn = 0; dn <= N; dn += 4) secs.push_back({(N + dn) / 2, (N - dn) / 2});
+  }
+  if (general && !all && (P.fill < 1.0 || P.frac) &&
+      !strings_pay(rk.nI, rk.nE, m, secs, !sp.frac && sp.mult > 0, P.fill))
+    return fail("the configuration records are cheaper for this list");
   // levels: strings of n electrons with at most m external electrons
   std::vector<bool> need(N + 1, false);
   for (auto& s : secs)
@@ -477,8 +545,13 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two)
       const uint64_t ao = deposit(pt, s);
       const uint64_t am = d | ao, bm = d | (s & ~ao);
       const int dn = popc(am) - popc(bm);
-      if (dn < 0) return false;
-      sec = dn / 4;
+      if (sp.frac) {
+        sec = std::abs(dn) / 2;
+        if (P.sec[sec].na != popc(am)) return false;
+      } else {
+        if (dn < 0) return false;
+        sec = dn / 4;
+      }
       int ca, cb;
       int64_t ra, rb;
       rk.rank(am, ca, ra);
@@ -492,8 +565,9 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two)
       std::memset(&e, 0, sizeof(e));
       int sc;
       int32_t ga, gb;
-      if (no == 0) {
-        locate(pat[0], sc, ga, gb);
+      if (no == 0 || sp.frac) {
+        const bool ok = locate(pat[t], sc, ga, gb);
+        PSOCI_CHECK(ok, PSOCI_ERR_STATE, "SEF map: determinant outside the evaluated sectors");
         e.a[0] = ga;
         e.b[0] = gb;
         e.sec[0] = (int8_t)sc;

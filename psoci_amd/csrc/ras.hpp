@@ -558,6 +558,10 @@ struct RasPlan {
   // the compact layout: per block, its totals (per column) and flops
   std::vector<RasCmp> cmp;
   int64_t cwunit = 0, cdunit = 0, cgunit = 0;
+  // the list's share of the space's configurations (below 1: the others'
+  // determinants are zeros), and whether its SEFs are single determinants
+  double fill = 1.0;
+  bool frac = false;
   double cflops_per_col = 0.0;
 };
 
@@ -573,9 +577,13 @@ inline void ras_cmp_groups(const RasCmp& C, F&& f) {
 }
 
 // Builds the plan for the space and integrals; plan.ok = false (with a
-// reason) when the space is not a complete RAS space of the supported kind.
+// reason) when the space is not a complete RAS space of the EVEN class.
+// general: also a list that is part of a RAS space (its H is that space's
+// with the other determinants projected out) and odd electron counts, where
+// that costs less than the pair records (all: wherever it is possible).
 struct Space;
-void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two);
+void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two, bool general = false,
+              bool all = false);
 // A view of the plan's host tables (host pointers), e.g. for a host check.
 RasView ras_host_view(const RasPlan& P);
 

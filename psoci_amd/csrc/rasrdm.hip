@@ -270,7 +270,7 @@ void gram_blocks(Ctx& c, const std::vector<int64_t>& moff, const double* wk, Dev
     const RasSectorDev& S = P.sec[B.sector];
     // a sector n_alpha > n_beta stands for its spin flip, a product of a
     // symmetric sector for its mirror
-    double fac = S.na > S.nb ? 2.0 : 1.0;
+    double fac = S.na > S.nb && !P.frac ? 2.0 : 1.0;
     if (S.sym && (B.kind == 1 || B.cu < B.cw || B.tri)) fac *= 2.0;
     const int nt = (B.nq + kPT - 1) / kPT, ntp = nt * (nt + 1) / 2;
     constexpr int RC = kKK / KC;

@@ -99,11 +99,6 @@ __global__ __launch_bounds__(256) void k_ras_order(int64_t ndet, const int64_t* 
   const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (d < ndet && flag[d]) order[rank[d]] = sef[d];
 }
-__global__ __launch_bounds__(256) void k_ras_zero64(int64_t n, int64_t* __restrict__ p) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0;
-}
-
 // The signed rows of every SEF's determinant coefficients, in that order
 // (built once): rows.x = det + negative * ndet of its first determinant; rows.y the same for the second, or -1 (one determinant, coefficient
 // 1/sqrt(2)) or -2 (a closed shell, coefficient 1); -3 marks a determinant
@@ -153,6 +148,37 @@ __global__ __launch_bounds__(256) void k_ras_x2c(int64_t nsef, int64_t ndet, con
     c[(int64_t)r.y * KC + q] = y;
     c[(r.y < ndet ? r.y + ndet : r.y - ndet) * KC + q] = -y;
   }
+}
+
+// Determinants of a list that is only part of its space: flags of those that
+// belong to a SEF, the others' list, and their zeros (both signed rows)
+__global__ __launch_bounds__(256) void k_ras_present(const RasView* __restrict__ vp, int64_t* __restrict__ absent) {
+  const RasView& v = *vp;
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= v.nsef) return;
+  const RasSef e = v.sef[s];
+  for (int d = 0; d < e.n; ++d) {
+    const int64_t k = ras_sef_det(v, e, d);
+    if (k >= 0) absent[k] = 0;
+  }
+}
+__global__ __launch_bounds__(256) void k_ras_fill64(int64_t n, int64_t* __restrict__ p, int64_t x) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) p[t] = x;
+}
+__global__ __launch_bounds__(256) void k_ras_absent(int64_t ndet, const int64_t* __restrict__ absent,
+                                                    const int64_t* __restrict__ rank, int32_t* __restrict__ list) {
+  const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (d < ndet && absent[d]) list[rank[d]] = (int32_t)d;
+}
+template <typename T, int KC>
+__global__ __launch_bounds__(256) void k_ras_blank(int64_t n, int64_t ndet, const int32_t* __restrict__ list,
+                                                   T* __restrict__ c) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * KC) return;
+  const int64_t d = list[t / KC];
+  c[d * KC + t % KC] = (T)0;
+  c[(d + ndet) * KC + t % KC] = (T)0;
 }
 
 // Pair table of the compact products (built once): per block and variant the
@@ -779,6 +805,12 @@ void ras_chunk(Ctx& c, const TIO* X, int ldx, TIO* Y, int ldy, int col0, int kw,
   hipLaunchKernelGGL((k_ras_x2c<T, KC, TIO>), dim3(8 * nblk(nsef * KC, 8 * 256)), dim3(256), 0, c.stream, nsef, P.ndet,
                      c.d_rasorder.p, c.d_rasrows.p, X, ldx, col0, kw, cv);
   PSOCI_HIP(hipGetLastError());
+  if (c.d_rasabsent.n) {
+    const int64_t na = (int64_t)c.d_rasabsent.n;
+    hipLaunchKernelGGL((k_ras_blank<T, KC>), dim3(nblk(na * KC, 256)), dim3(256), 0, c.stream, na, P.ndet,
+                       c.d_rasabsent.p, cv);
+    PSOCI_HIP(hipGetLastError());
+  }
   if (tm) tm->mark(c.stream, 0);
   constexpr int ki = KC == 16 ? 0 : KC == 8 ? 1 : KC == 4 ? 2 : 3;
   const std::vector<RasLaunch>& L = c.ras_launch[ki];
@@ -899,7 +931,10 @@ bool build_ras(Ctx& c) {
   c.d_one.download(one.data(), one.size(), c.stream);
   c.d_two.download(two.data(), two.size(), c.stream);
   c.sync();
-  ras_plan(c.ras, sp, one.data(), two.data());
+  // engine 2 on request takes complete EVEN-class spaces only; the automatic
+  // choice also odd electron counts and parts of a space, where that is
+  // cheaper than the pair records
+  ras_plan(c.ras, sp, one.data(), two.data(), c.direct_engine_req == 0);
   if (!c.ras.ok) {
     c.ras_why = c.ras.why;
     return false;
@@ -1009,7 +1044,8 @@ bool build_ras(Ctx& c) {
     rank.alloc(P.ndet + 1);
     sef.alloc(P.ndet);
     c.d_rasorder.alloc(nsef);
-    hipLaunchKernelGGL(k_ras_zero64, dim3(nblk(P.ndet + 1, 256)), dim3(256), 0, c.stream, P.ndet + 1, flag.p);
+    hipLaunchKernelGGL(k_ras_fill64, dim3(nblk(P.ndet + 1, 256)), dim3(256), 0, c.stream, P.ndet + 1, flag.p,
+                       (int64_t)0);
     PSOCI_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_ras_mark, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p, flag.p, sef.p);
     PSOCI_HIP(hipGetLastError());
@@ -1020,6 +1056,27 @@ bool build_ras(Ctx& c) {
     PSOCI_CHECK(found == nsef, PSOCI_ERR_STATE, "string-driven sigma: inconsistent determinant map");
     hipLaunchKernelGGL(k_ras_order, dim3(nblk(P.ndet, 256)), dim3(256), 0, c.stream, P.ndet, flag.p, rank.p, sef.p,
                        c.d_rasorder.p);
+    PSOCI_HIP(hipGetLastError());
+    c.sync();
+  }
+  // the determinants of no SEF
+  c.d_rasabsent.release();
+  if (P.fill < 1.0) {
+    DevBuf<int64_t> absent, rank;
+    absent.alloc(P.ndet + 1);
+    rank.alloc(P.ndet + 1);
+    const int64_t nsef = (int64_t)P.sef.size();
+    hipLaunchKernelGGL(k_ras_fill64, dim3(nblk(P.ndet, 256)), dim3(256), 0, c.stream, P.ndet, absent.p, (int64_t)1);
+    hipLaunchKernelGGL(k_ras_fill64, dim3(1), dim3(256), 0, c.stream, (int64_t)1, absent.p + P.ndet, (int64_t)0);
+    hipLaunchKernelGGL(k_ras_present, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p, absent.p);
+    PSOCI_HIP(hipGetLastError());
+    c.scan(absent.p, rank.p, P.ndet + 1);
+    int64_t na = 0;
+    PSOCI_HIP(hipMemcpyAsync(&na, rank.p + P.ndet, sizeof(int64_t), hipMemcpyDeviceToHost, c.stream));
+    c.sync();
+    c.d_rasabsent.alloc(na);
+    hipLaunchKernelGGL(k_ras_absent, dim3(nblk(P.ndet, 256)), dim3(256), 0, c.stream, P.ndet, absent.p, rank.p,
+                       c.d_rasabsent.p);
     PSOCI_HIP(hipGetLastError());
     c.sync();
   }
@@ -1067,8 +1124,9 @@ void build_direct(Ctx& c) {
     c.ras_tried = true;
     if (build_ras(c)) return;
   }
-  PSOCI_CHECK(c.direct_engine_req != 2 || c.have_ras, PSOCI_ERR_UNSUPPORTED,
-              "the string-driven direct sigma does not apply to this space: " + c.ras_why);
+  PSOCI_CHECK(c.direct_engine_req != 2 || direct_engine(c) == 2, PSOCI_ERR_UNSUPPORTED,
+              c.have_ras ? "the string-driven direct sigma on request takes complete EVEN-class spaces only"
+                         : "the string-driven direct sigma does not apply to this space: " + c.ras_why);
   if (!direct_engine(c)) build_pairs(c);
 }
 
@@ -1107,11 +1165,15 @@ int ras_scatter64(Ctx& c, const double* X, int ldx, int col0, int kw) {
   double* cv = reinterpret_cast<double*>(c.d_rasc.p);
   const int kc = kw > 8 ? 16 : kw > 4 ? 8 : kw > 2 ? 4 : 2;
   const dim3 grid(8 * nblk(nsef * kc, 8 * 256));
+  const int64_t na = (int64_t)c.d_rasabsent.n;
   switch (kc) {
 #define PSOCI_RAS_SCATTER(KCV)                                                                                   \
   case KCV:                                                                                                      \
     hipLaunchKernelGGL((k_ras_x2c<double, KCV, double>), grid, dim3(256), 0, c.stream, nsef, c.ras.ndet,         \
                        c.d_rasorder.p, c.d_rasrows.p, X, ldx, col0, kw, cv);                                     \
+    if (na)                                                                                                      \
+      hipLaunchKernelGGL((k_ras_blank<double, KCV>), dim3(nblk(na * KCV, 256)), dim3(256), 0, c.stream, na,      \
+                         c.ras.ndet, c.d_rasabsent.p, cv);                                                       \
     break;
     PSOCI_RAS_SCATTER(16)
     PSOCI_RAS_SCATTER(8)

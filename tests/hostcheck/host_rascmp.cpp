@@ -11,14 +11,16 @@ using namespace psoci;
 
 // Y[n][k] = H X[n][k] through the compact products; info[0..2] = blocks
 // per level, info[3..4] =
-// full and compact multiply-adds.  0 on success.
+// full and compact multiply-adds, info[5] = the list's share of the space.  0
+// on success.
 extern "C" int hrc_sigma(int nbf, int nelec, int ksym, int64_t ncfg, const uint8_t* occ, const int32_t* jsym,
-                         const double* one, const double* two, int k, const double* X, double* Y, double* info) {
+                         const double* one, const double* two, int k, const double* X, double* Y, double* info,
+                         int general) {
   Space sp;
   RasPlan P;
   try {
     build_space(sp, nbf, nelec, ksym, ncfg, occ, jsym);
-    ras_plan(P, sp, one, two);
+    ras_plan(P, sp, one, two, general != 0, true);
   } catch (const Error&) {
     return -1;
   }
@@ -42,6 +44,7 @@ extern "C" int hrc_sigma(int nbf, int nelec, int ksym, int64_t ncfg, const uint8
   info[0] = info[1] = info[2] = 0.0;
   info[3] = P.gemm_flops_per_col;
   info[4] = P.cflops_per_col;
+  info[5] = P.fill;
   for (int bi = 0; bi < v.nblk; ++bi) {
     const RasBlockDev& B = v.blk[bi];
     const RasCmp& C = P.cmp[bi];

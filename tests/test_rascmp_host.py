@@ -30,7 +30,7 @@ def lib():
     L = ctypes.CDLL(OUT)
     P = ctypes.c_void_p
     L.hrc_sigma.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, P, P, P, P, ctypes.c_int, P, P,
-                            P]
+                            P, ctypes.c_int]
     return L
 
 
@@ -68,23 +68,64 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("name,make,levels", CASES, ids=[c[0] for c in CASES])
-def test_compact_products_match_oracle(lib, name, make, levels):
-    cfg, ints = make()
+def _run(lib, cfg, ints, general):
     sp = oracle.OracleSpace(cfg, ints)
     sp.build_h()
     X = np.random.default_rng(3).standard_normal((sp.n, 2))
     ref = sp.sigma(X)
     Y = np.zeros_like(X)
-    info = np.zeros(5)
+    info = np.zeros(6)
     occ = np.ascontiguousarray(cfg.occ, np.uint8)
     js = np.ascontiguousarray(cfg.jsym, np.int32)
     ptr = [a.ctypes.data_as(ctypes.c_void_p) for a in (occ, js, ints.valone, ints.valtwo)]
     rc = lib.hrc_sigma(cfg.nbf, cfg.nelec, cfg.ksym, cfg.ncfg, *ptr, X.shape[1],
                        X.ctypes.data_as(ctypes.c_void_p), Y.ctypes.data_as(ctypes.c_void_p),
-                       info.ctypes.data_as(ctypes.c_void_p))
+                       info.ctypes.data_as(ctypes.c_void_p), general)
+    return rc, Y, ref, info
+
+
+@pytest.mark.parametrize("name,make,levels", CASES, ids=[c[0] for c in CASES])
+def test_compact_products_match_oracle(lib, name, make, levels):
+    rc, Y, ref, info = _run(lib, *make(), 0)
     assert rc == 0, rc
     np.testing.assert_allclose(Y, ref, rtol=0, atol=1e-12 * np.abs(ref).max())
     for lev in levels:
         assert info[lev] > 0, info
     assert info[4] <= info[3]
+    assert info[5] == 1.0
+
+
+def _part(cfg, ints, share, seed=9):
+    keep = np.random.default_rng(seed).random(cfg.ncfg) < share
+    return (inputs.Configs(nbf=cfg.nbf, nelec=cfg.nelec, ksym=cfg.ksym, occ=cfg.occ[keep].copy(),
+                           jsym=cfg.jsym[keep].copy()), ints)
+
+
+def _odd(cfg, ints, jsym):
+    return inputs.Configs(nbf=cfg.nbf, nelec=cfg.nelec, ksym=jsym, occ=cfg.occ,
+                          jsym=np.full(cfg.ncfg, jsym, np.int32)), ints
+
+
+GENERAL = [
+    ("part of fci 6/6", lambda: _part(*_fci(6, 6), 0.5)),
+    ("part of fci 6/6, mult -1", lambda: _part(*_fci(6, 6, ksym=2), 0.5)),
+    ("part of mrcisd 5+5/4", lambda: _part(*_mrci(5, 5, 4), 0.3)),
+    ("odd fci 6/5", lambda: _fci(6, 5)),
+    ("odd fci 6/7, alpha and beta swapped", lambda: _odd(*_fci(6, 7), 3)),
+    ("odd mrcisd 4+5/5", lambda: _mrci(4, 5, 5)),
+    ("odd mrcisd 6+8/5", lambda: _mrci(6, 8, 5)),
+    ("part of odd mrcisd 4+5/3", lambda: _part(*_mrci(4, 5, 3), 0.6)),
+]
+
+
+@pytest.mark.parametrize("name,make", GENERAL, ids=[c[0] for c in GENERAL])
+def test_general_plans_match_oracle(lib, name, make):
+    """Lists that are part of a space, and odd electron counts: refused
+    without `general`, the oracle's sigma with it."""
+    cfg, ints = make()
+    rc, _, _, _ = _run(lib, cfg, ints, 0)
+    assert rc == 1
+    rc, Y, ref, info = _run(lib, cfg, ints, 1)
+    assert rc == 0, rc
+    assert (info[5] < 1.0) == name.startswith("part")
+    np.testing.assert_allclose(Y, ref, rtol=0, atol=1e-12 * np.abs(ref).max())
