@@ -21,6 +21,11 @@ int guarded(psoci_ctx* ctx, F&& f) {
     psoci::set_ctxfree_error("null context");
     return PSOCI_ERR_ARG;
   }
+  struct SpareOf {
+    psoci::Spare* before = psoci::t_spare;
+    ~SpareOf() { psoci::t_spare = before; }
+  } spare_of;
+  psoci::t_spare = &ctx->c.spare;
   try {
     PSOCI_HIP(hipSetDevice(ctx->c.device));
     ctx->c.err.clear();

@@ -29,6 +29,10 @@ struct Error : std::runtime_error {
     if (!(cond)) throw ::psoci::Error(code, msg); \
   } while (0)
 
+// Frees the scratch memory that the calling thread's context keeps between
+// builds (ctx.hpp); false if there is none or it is in use.
+bool give_back_spare();
+
 // Device buffer owned by a context.
 template <class T>
 struct DevBuf {
@@ -48,6 +52,10 @@ struct DevBuf {
     release();
     if (count == 0) return;
     hipError_t e = hipMalloc(&p, count * sizeof(T));
+    if (e == hipErrorOutOfMemory && give_back_spare()) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, count * sizeof(T));
+    }
     if (e != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();

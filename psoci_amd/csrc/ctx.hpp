@@ -15,6 +15,22 @@ struct Staging {
   size_t bytes = 0;
 };
 
+// Scratch memory of the Hamiltonian build, kept for the next build of the same
+// context (new integrals at the next geometry) up to kSpareBytes: freeing it
+// every time cost 0.5 ms beside a 1.6 ms build (32,000 SEFs, 0.85 GB), and
+// 20 ms where several contexts built in turn.  Given back when an allocation
+// of the context fails, before the direct engine sizes its plan, and with the
+// context.
+constexpr size_t kSpareBytes = size_t(1) << 30;
+struct Spare {
+  DevBuf<char> buf[2];
+  bool busy = false;  // in use by a build
+  void give_back() {
+    for (auto& b : buf) b.release();
+  }
+};
+inline thread_local Spare* t_spare = nullptr;  // of the context whose entry point runs on this thread
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -174,6 +190,7 @@ struct Ctx {
 
   // scratch
   DevBuf<char> d_pad;  // zero-padded column staging for the direct sigma
+  Spare spare;
   void* scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
 

@@ -952,6 +952,7 @@ bool build_ras(Ctx& c) {
     const double need = (double)P.cwunit * 64 + (double)P.cdunit * 4 + (double)P.cgunit * 12 + (double)P.ndet * 128 +
                         (double)terms * 4 + (double)P.sef.size() * 9;
     size_t fr = 0, tot = 0;
+    c.spare.give_back();
     PSOCI_HIP(hipMemGetInfo(&fr, &tot));
     // FP64 in chunks of 16 columns (whole 128-byte W and c pieces) when W and
     // c fit twice over in 60 % of the free memory, else chunks of 8
