@@ -499,6 +499,7 @@ int psoci_project(psoci_ctx* ctx, int64_t n, int m, int b, const double* A, int 
                 "bad projection arguments");
     psoci::Linalg L;
     L.stream = c.stream;
+    L.host = &c.lin_host;
     L.gemm_tn_host(n, m, b, A, lda, B, ldb, out);
     return PSOCI_OK;
   });
@@ -511,6 +512,7 @@ int psoci_combine(psoci_ctx* ctx, int64_t n, int m, int k, const double* A, int 
                 "bad combine arguments");
     psoci::Linalg L;
     L.stream = c.stream;
+    L.host = &c.lin_host;
     L.gemm_nn(n, m, k, A, lda, Y, alpha, Out, ldo);
     c.sync();
     return PSOCI_OK;

@@ -1,6 +1,7 @@
 // Context state of the PSOCI MI355X library (one GPU).
 #pragma once
 #include "common.hpp"
+#include "linalg.hpp"
 #include "elem.hpp"
 #include "ras.hpp"
 
@@ -15,18 +16,52 @@ struct Staging {
   size_t bytes = 0;
 };
 
-// Scratch memory of the Hamiltonian build, kept for the next build of the same
-// context (new integrals at the next geometry) up to kSpareBytes: freeing it
-// every time cost 0.5 ms beside a 1.6 ms build (32,000 SEFs, 0.85 GB), and
-// 20 ms where several contexts built in turn.  Given back when an allocation
-// of the context fails, before the direct engine sizes its plan, and with the
-// context.
+// Scratch memory of the Hamiltonian build (buf 0, 1) and of the Davidson
+// solver (2), kept for the context's next one (new integrals at the next
+// geometry) up to kSpareBytes in all: allocating and freeing it every time cost
+// 0.5 ms beside a 1.6 ms build (32,000 SEFs, 0.85 GB), and 20 ms where several
+// contexts built in turn.  Given back when an allocation of the context
+// fails, before the direct engine sizes its plan, and with the context.
 constexpr size_t kSpareBytes = size_t(1) << 30;
 struct Spare {
-  DevBuf<char> buf[2];
-  bool busy = false;  // in use by a build
-  void give_back() {
-    for (auto& b : buf) b.release();
+  DevBuf<char> buf[3];
+  bool busy[3] = {false, false, false};
+  bool give_back() {
+    bool any = false;
+    for (int i = 0; i < 3; ++i)
+      if (!busy[i] && buf[i].p) {
+        buf[i].release();
+        any = true;
+      }
+    return any;
+  }
+};
+// The buffers first .. first + count - 1 in use by a scope; the stream is idle
+// where it ends normally.
+struct SpareUse {
+  Spare& s;
+  const int first, count;
+  SpareUse(Spare& s_, int first_, int count_) : s(s_), first(first_), count(count_) {
+    for (int i = first; i < first + count; ++i) s.busy[i] = true;
+  }
+  SpareUse(const SpareUse&) = delete;
+  SpareUse& operator=(const SpareUse&) = delete;
+  ~SpareUse() {
+    for (int i = first; i < first + count; ++i) s.busy[i] = false;
+    if (s.buf[0].n + s.buf[1].n + s.buf[2].n > kSpareBytes)
+      for (int i = first; i < first + count; ++i) s.buf[i].release();
+  }
+};
+// Arrays carved from one of the spare buffers.
+struct Scratch {
+  DevBuf<char>& buf;
+  size_t used = 0;
+  static constexpr size_t bytes(size_t count, size_t size) { return (count * size + 255) / 256 * 256; }
+  template <typename T>
+  T* take(size_t count) {
+    T* p = reinterpret_cast<T*>(buf.p + used);
+    used += bytes(count, sizeof(T));
+    return p;
   }
 };
 inline thread_local Spare* t_spare = nullptr;  // of the context whose entry point runs on this thread
@@ -191,6 +226,7 @@ struct Ctx {
   // scratch
   DevBuf<char> d_pad;  // zero-padded column staging for the direct sigma
   Spare spare;
+  LinalgHost lin_host;  // the Davidson's small matrices
   void* scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
 

@@ -44,6 +44,22 @@ struct Timer {
   double sec() const { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); }
 };
 
+// A device array of the solver: part of the context's spare memory, or its
+// own allocation where the solver needs more than is kept.
+template <typename T>
+struct Block {
+  DevBuf<T> own;
+  T* p = nullptr;
+  void alloc(size_t count, Scratch* from) {
+    if (from) {
+      p = from->take<T>(count);
+    } else {
+      own.alloc(count);
+      p = own.p;
+    }
+  }
+};
+
 }  // namespace
 
 int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, psoci_dav_stats* st) {
@@ -77,24 +93,38 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
 
   Linalg L;
   L.stream = c.stream;
+  L.host = &c.lin_host;
+  // V^T HV of a step, in host memory (at a fixed place: captured launches
+  // write to it)
+  double* const proj = L.results((size_t)mmax * std::max(k0, kc));
   // the basis V and its sigma HV: FP64 for the FP64 phase, FP32 (V32,
   // HV32) for the FP32 phase; a mixed solve holds both
-  DevBuf<double> V, HV, R, T;
+  Block<double> V, HV, R, T;
   // R32: the FP32 phase's residual block (Olsen's correction keeps FP64 R)
-  DevBuf<float> V32, HV32, X32, Y32, R32;
+  Block<float> V32, HV32, X32, Y32, R32;
   const bool want32 = p.prec != PSOCI_FP64;
-  if (p.prec != PSOCI_FP32) {
-    V.alloc((size_t)n * mmax);
-    HV.alloc((size_t)n * mmax);
+  const size_t nv = (size_t)n * mmax, nk = (size_t)n * k0, nt = (size_t)n * std::max(kc, k0);
+  const size_t nv64 = p.prec != PSOCI_FP32 ? nv : 0, nv32 = want32 ? nv : 0, nk32 = want32 ? nk : 0;
+  const size_t nr32 = want32 && !olsen ? nk : 0;
+  SpareUse spare_use(c.spare, 2, 1);
+  Scratch arena{c.spare.buf[2]};
+  const size_t need = 2 * Scratch::bytes(nv64, 8) + Scratch::bytes(nk, 8) + Scratch::bytes(nt, 8) +
+                      2 * Scratch::bytes(nv32, 4) + 2 * Scratch::bytes(nk32, 4) + Scratch::bytes(nr32, 4);
+  Scratch* from = need <= kSpareBytes ? &arena : nullptr;
+  if (from) arena.buf.reserve(need);
+  else arena.buf.release();
+  if (nv64) {
+    V.alloc(nv64, from);
+    HV.alloc(nv64, from);
   }
-  R.alloc((size_t)n * k0);
-  T.alloc((size_t)n * std::max(kc, k0));
+  R.alloc(nk, from);
+  T.alloc(nt, from);
   if (want32) {
-    V32.alloc((size_t)n * mmax);
-    HV32.alloc((size_t)n * mmax);
-    X32.alloc((size_t)n * k0);
-    Y32.alloc((size_t)n * k0);
-    if (!olsen) R32.alloc((size_t)n * k0);
+    V32.alloc(nv32, from);
+    HV32.alloc(nv32, from);
+    X32.alloc(nk32, from);
+    Y32.alloc(nk32, from);
+    if (nr32) R32.alloc(nr32, from);
   }
   psoci_dav_stats S{};
   S.switch_iter = -1;
@@ -119,7 +149,7 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
   };
   if (p.guess == 2) {
     PSOCI_CHECK(evecs, PSOCI_ERR_ARG, "guess 2 needs the starting vectors in evecs");
-    R.upload(evecs, (size_t)n * k, c.stream);
+    PSOCI_HIP(hipMemcpyAsync(R.p, evecs, (size_t)n * k * sizeof(double), hipMemcpyHostToDevice, c.stream));
     if (phase32) L.to_f32(n, k, R.p, k, V32.p, mmax);
     else L.copy_cols(n, k, R.p, k, V.p, mmax);
   } else {
@@ -128,7 +158,7 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
 
   const double switch_tol = p.switch_tol > 0 ? p.switch_tol : 1e-4;
   // The device work of one step -- sigma of the new block V[:, c0:c0+nb)
-  // into HV and its projection V^T HV[:, c0:c0+nb) into L.small -- has no
+  // into HV and its projection V^T HV[:, c0:c0+nb) into proj -- has no
   // host decision inside, so on the stored sigma (launch- and
   // latency-bound: about 0.1 ms per sigma on 31,650 SEFs) it runs as one
   // captured hipGraph per (c0, nb, precision), instantiated on first use
@@ -150,7 +180,6 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
   } segs_guard{segs};
   if (graphs) {
     L.reserve_tn(n, mmax, k0);
-    L.small.reserve((size_t)mmax * k0);
     const size_t es = phase32 ? 4 : 8;
     c.d_pad.reserve((size_t)2 * n * 32 * std::max<size_t>(es, 8));
   }
@@ -167,8 +196,7 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
       if (p.sigma_mode == PSOCI_SIGMA_STORED) sigma_stored(c, PSOCI_FP64, nb, V.p + c0, mmax, HV.p + c0, mmax);
       else sigma_direct(c, PSOCI_FP64, nb, V.p + c0, mmax, HV.p + c0, mmax);
     }
-    L.small.reserve((size_t)(c0 + nb) * nb);
-    on_basis([&](auto* Vb, auto* HVb) { L.gemm_tn(n, c0 + nb, nb, Vb, mmax, HVb + c0, mmax, L.small.p); });
+    on_basis([&](auto* Vb, auto* HVb) { L.gemm_tn(n, c0 + nb, nb, Vb, mmax, HVb + c0, mmax, proj); });
   };
   auto run_step = [&](int c0, int nb) {
     if (!graphs) {
@@ -200,7 +228,7 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
     S.graph_launches += 1;
   };
 
-  std::vector<double> A((size_t)mmax * mmax, 0.0), tmp;
+  std::vector<double> A((size_t)mmax * mmax, 0.0);
   // sigma of V[:, c0:c0+nb) and the new columns of A = V^T H V
   auto sigma_update = [&](int c0, int nb) {
     Timer ts;
@@ -210,11 +238,8 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
     S.sigma_calls += 1;
     S.sigma_vectors += nb;
     int m = c0 + nb;
-    tmp.resize((size_t)m * nb);
-    L.small.download(tmp.data(), (size_t)m * nb, c.stream);
-    c.sync();
     for (int i = 0; i < m; ++i)
-      for (int j = 0; j < nb; ++j) A[(size_t)i * mmax + c0 + j] = tmp[(size_t)i * nb + j];
+      for (int j = 0; j < nb; ++j) A[(size_t)i * mmax + c0 + j] = proj[(size_t)i * nb + j];
     for (int i = c0; i < m; ++i)
       for (int j = c0; j < i; ++j) {
         double s = 0.5 * (A[(size_t)i * mmax + j] + A[(size_t)j * mmax + i]);
@@ -522,7 +547,7 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
   if (evecs) {
     cols_of(m, 0, kw, Yk);
     on_basis([&](auto* Vb, auto*) { L.gemm_nn(n, m, kw, Vb, mmax, Yk.data(), 0.0, R.p, kw); });
-    R.download(evecs, (size_t)n * kw, c.stream);
+    PSOCI_HIP(hipMemcpyAsync(evecs, R.p, (size_t)n * kw * sizeof(double), hipMemcpyDeviceToHost, c.stream));
     c.sync();
   }
   S.seconds = total.sec();

@@ -545,11 +545,7 @@ inline unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1)
 
 }  // namespace
 
-bool give_back_spare() {
-  if (!t_spare || t_spare->busy || !(t_spare->buf[0].p || t_spare->buf[1].p)) return false;
-  t_spare->give_back();
-  return true;
-}
+bool give_back_spare() { return t_spare && t_spare->give_back(); }
 
 void exclusive_scan_i64(const int64_t* in, int64_t* out, int64_t n, hipStream_t s, void*& tmp, size_t& tmp_bytes) {
   if (n <= 0) return;
@@ -582,36 +578,11 @@ void upload_space(Ctx& c) {
   c.sync();
 }
 
-namespace {
-
-// Scratch arrays carved from one of the context's spare buffers.
-struct Scratch {
-  DevBuf<char>& buf;
-  size_t used = 0;
-  static constexpr size_t bytes(size_t count, size_t size) { return (count * size + 255) / 256 * 256; }
-  template <typename T>
-  T* take(size_t count) {
-    T* p = reinterpret_cast<T*>(buf.p + used);
-    used += bytes(count, sizeof(T));
-    return p;
-  }
-};
-
-}  // namespace
-
 void build_h(Ctx& c) {
   const Space& sp = c.sp;
   const int64_t ncfg = sp.ncfg, n = sp.nsef_total;
   const auto t0 = std::chrono::steady_clock::now();
-  // the stream is idle wherever this scope is left normally
-  struct SpareUse {
-    Spare& s;
-    explicit SpareUse(Spare& sp_) : s(sp_) { s.busy = true; }
-    ~SpareUse() {
-      s.busy = false;
-      if (s.buf[0].n + s.buf[1].n > kSpareBytes) s.give_back();
-    }
-  } spare_use(c.spare);
+  SpareUse spare_use(c.spare, 0, 2);
   // connected pairs: lower (J <= I per I), then upper (J > I)
   DevBuf<int64_t> cnt, off;
   cnt.alloc(std::max(2 * ncfg, n) + 1);

@@ -43,20 +43,27 @@ constexpr int tn_cols() {
 // (i = 4*t + l/16, j = l%16).  With CP = 2 lane i carries A columns
 // 32 tm + 2i and 32 tm + 2i + 1, one per tile.  TA: the element type of A
 // and B (float columns are widened on load).
+//
+// A workgroup has wt tiles and, of each, up to 8 / wt wavefronts with a part
+// of the chunk's rows each, summed through LDS: one partial result per
+// workgroup and not per wavefront, which left the reduction below 5 MB to read
+// (10 us; with the partials of one workgroup and whole lines read, 5 us).
 template <typename TA, int CP = tn_cols<TA>()>
-__global__ __launch_bounds__(256) void k_gemm_tn_mfma(int64_t n, int m, int b, const TA* __restrict__ A, int lda,
-                                                      const TA* __restrict__ B, int ldb, int64_t rows_per_chunk,
+__global__ __launch_bounds__(512) void k_gemm_tn_mfma(int64_t n, int m, int b, const TA* __restrict__ A, int lda,
+                                                      const TA* __restrict__ B, int ldb, int wt, int64_t rows_per_sub,
                                                       double* __restrict__ partial) {
   constexpr int NCH = 4 / CP;  // accumulation chains per tile
+  __shared__ double sh[(8 - 1) * CP * 4 * kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int tiles_m = (m + 16 * CP - 1) / (16 * CP), tiles_b = (b + 15) / 16;
-  const int tile = blockIdx.x * (blockDim.x / kWave) + wave;
-  if (tile >= tiles_m * tiles_b) return;
+  const int sub = wave / wt, wtile = wave - sub * wt, nsub = blockDim.x / kWave / wt;
+  const int tile = blockIdx.x * wt + wtile;
   const int tm = tile / tiles_b, tb = tile - tm * tiles_b;
+  const bool valid = tile < tiles_m * tiles_b;  // else only the barrier below
   const int64_t chunk = blockIdx.y;
-  const int64_t r0 = chunk * rows_per_chunk;
-  const int64_t r1 = (r0 + rows_per_chunk < n) ? r0 + rows_per_chunk : n;
+  const int64_t r0 = valid ? (chunk * nsub + sub) * rows_per_sub : n;
+  const int64_t r1 = (r0 + rows_per_sub < n) ? r0 + rows_per_sub : n;
   const int ci = tm * 16 * CP + CP * (lane & 15);
   const int cj = tb * 16 + (lane & 15);
   const int kk = lane >> 4;
@@ -121,63 +128,91 @@ __global__ __launch_bounds__(256) void k_gemm_tn_mfma(int64_t n, int m, int b, c
         q[3] += (double)p[3];
       }
     }
-    // accumulator t of lane l holds output row 4 (l / 16) + t (FP32 layout)
-    double* out = partial + chunk * (int64_t)m * b;
+  } else {
+    for (int64_t r = r0; r < r1; r += 16) {
+      double a[CP][4], bb[4];
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+      for (int u = 0; u < 4; ++u) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int i = tm * 32 + 2 * (4 * (lane >> 4) + t) + c;
-        const int j = tb * 16 + (lane & 15);
-        if (i < m && j < b) out[(int64_t)i * b + j] = acc[c][0][t];
+        for (int c = 0; c < CP; ++c) a[c][u] = (double)ra[c][u];
+        bb[u] = (double)rb[u];
       }
-    return;
-  }
-  for (int64_t r = r0; r < r1; r += 16) {
-    double a[CP][4], bb[4];
+      if (r + 16 < r1) load(r + 16);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int c = 0; c < CP; ++c) a[c][u] = (double)ra[c][u];
-      bb[u] = (double)rb[u];
+        for (int c = 0; c < CP; ++c)
+          acc[c][u % NCH] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[c][u], bb[u], acc[c][u % NCH], 0, 0, 0);
     }
-    if (r + 16 < r1) load(r + 16);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int c = 0; c < CP; ++c)
-        acc[c][u % NCH] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[c][u], bb[u], acc[c][u % NCH], 0, 0, 0);
   }
-  double* out = partial + chunk * (int64_t)m * b;
+  double4_t sum[CP];
 #pragma unroll
   for (int c = 0; c < CP; ++c) {
-    double4_t sum = acc[c][0];
+    sum[c] = acc[c][0];
+    if (!(CP == 2 && kTnF32Mfma))
 #pragma unroll
-    for (int h = 1; h < NCH; ++h) sum += acc[c][h];
+      for (int h = 1; h < NCH; ++h) sum[c] += acc[c][h];
+  }
+  if (nsub > 1) {
+    // parts 1.. of each tile into LDS, added in order by the tile's part 0
+    if (sub > 0)
+#pragma unroll
+      for (int c = 0; c < CP; ++c)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) sh[(((wave - wt) * CP + c) * 4 + t) * kWave + lane] = sum[c][t];
+    __syncthreads();
+    if (sub > 0) return;
+    for (int q = 1; q < nsub; ++q)
+#pragma unroll
+      for (int c = 0; c < CP; ++c)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) sum[c][t] += sh[((((q - 1) * wt + wtile) * CP + c) * 4 + t) * kWave + lane];
+  }
+  if (!valid) return;
+  double* out = partial + chunk * (int64_t)m * b;
+#pragma unroll
+  for (int c = 0; c < CP; ++c)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const int i = tm * 16 * CP + CP * (4 * t + (lane >> 4)) + c;
+      // the FP32 instruction's accumulator t of lane l is row 4 (l / 16) + t
+      const int it = (CP == 2 && kTnF32Mfma) ? 4 * (lane >> 4) + t : 4 * t + (lane >> 4);
+      const int i = tm * 16 * CP + CP * it + c;
       const int j = tb * 16 + (lane & 15);
-      if (i < m && j < b) out[(int64_t)i * b + j] = sum[t];
+      if (i < m && j < b) out[(int64_t)i * b + j] = sum[c][t];
     }
-  }
 }
 
-// out[e] = sum over chunks of partial[c][e]: one workgroup per output entry,
-// strided partial sums then a fixed-order tree (deterministic)
-__global__ __launch_bounds__(256) void k_reduce_chunks(int64_t nchunks, int mb, const double* __restrict__ partial,
-                                                       double* __restrict__ out) {
-  __shared__ double sh[256];
-  const int e = blockIdx.x;
-  double s = 0.0;
-  for (int64_t c = threadIdx.x; c < nchunks; c += 256) s += partial[c * mb + e];
-  sh[threadIdx.x] = s;
+// out[e] = sum over chunks of partial[c][e] (deterministic): 16 entries per
+// workgroup, a 128-byte line of a chunk, and 32 threads per entry whose sums
+// are added in a fixed order.  out may be host memory.
+constexpr int kRedEntries = 16, kRedGroups = 32;
+__global__ __launch_bounds__(kRedEntries* kRedGroups) void k_reduce_chunks(int64_t nchunks, int mb,
+                                                                           const double* __restrict__ partial,
+                                                                           double* __restrict__ out) {
+  __shared__ double sh[kRedGroups][kRedEntries + 1];
+  const int x = threadIdx.x % kRedEntries, g = threadIdx.x / kRedEntries;
+  const int e = blockIdx.x * kRedEntries + x;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  if (e < mb) {
+    int64_t c = g;
+    for (; c + 3 * kRedGroups < nchunks; c += 4 * kRedGroups)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s[u] += partial[(c + u * kRedGroups) * mb + e];
+    for (; c < nchunks; c += kRedGroups) s[0] += partial[c * mb + e];
+  }
+  sh[g][x] = (s[0] + s[1]) + (s[2] + s[3]);
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+  for (int w = kRedGroups / 2; w > 0; w >>= 1) {
+    if (g < w) sh[g][x] += sh[g + w][x];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[e] = sh[0];
+  if (g == 0 && e < mb) out[e] = sh[0][x];
+}
+
+// dst = src (host memory), 8-byte words
+__global__ void k_put(int64_t words, const uint64_t* __restrict__ src, uint64_t* __restrict__ dst) {
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < words) dst[g] = src[g];
 }
 
 // Out[r][c] = alpha Out[r][c] + sum_t A[r][t] Y1[t][c] (+ sum_t B[r][t] Y2[t][c]
@@ -510,51 +545,99 @@ int tn_waves(int tiles) {
   return (tiles + groups - 1) / groups;
 }
 
-// Workgroups of k_gemm_tn_mfma with w wavefronts that the current device
-// holds at once (compute units x resident workgroups per unit), queried once
-// per device, width and columns per lane.
-int64_t tn_resident(int w, int cp) {
-  static int64_t cache[64][5][3] = {};
+// Workgroups of k_gemm_tn_mfma with w wavefronts that the current device holds
+// at once (compute units x resident workgroups per unit; *units: the compute
+// units), queried once per device, width and columns per lane.
+int64_t tn_resident(int w, int cp, int* units) {
+  static int64_t cache[64][9][3] = {};
+  static int cu_cache[64] = {};
   int dev = 0;
   PSOCI_HIP(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) dev = 0;
   if (cache[dev][w][cp] == 0) {
     int per_cu = 0, cus = 0;
+    const int threads = kWave * w;
     if (cp == 2)
-      PSOCI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gemm_tn_mfma<float>, kWave * w, 0));
+      PSOCI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gemm_tn_mfma<float>, threads, 0));
     else
-      PSOCI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gemm_tn_mfma<double>, kWave * w, 0));
+      PSOCI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gemm_tn_mfma<double>, threads, 0));
     PSOCI_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    cu_cache[dev] = cus;
     cache[dev][w][cp] = std::max<int64_t>(1, (int64_t)per_cu * cus);
   }
+  *units = cu_cache[dev];
   return cache[dev][w][cp];
 }
 
 // Output tiles of the projection's wavefronts (cp columns of A per lane).
 int tn_tiles(int m, int b, int cp) { return ((m + 16 * cp - 1) / (16 * cp)) * ((b + 15) / 16); }
 
-// Row chunks of the projection: one chunk per group of workgroups covering
-// the output tiles, as many groups as the device holds at once (a single
-// round of workgroups, no partly filled second round).
-void tn_chunks(int64_t n, int m, int b, int cp, int64_t& rows_per_chunk, int64_t& nchunks) {
+// Shape of the projection: wt tiles and subs row parts of a chunk per
+// workgroup, rows_per_sub rows per part (at least 64), nchunks chunks.  As many
+// chunks as the device holds workgroups at once (a single round, no partly
+// filled second one).  The most parts that 8 wavefronts allow, since each
+// chunk's partial result is written and read again, but fewer where the rows
+// then leave compute units idle (31,650 rows, one tile: 6.5 us with 8 parts
+// on 62 of 256 units, 5.3 us with one part).
+struct TnShape {
+  int wt, subs;
+  int64_t rows_per_sub, nchunks;
+};
+TnShape tn_shape(int64_t n, int m, int b, int cp) {
+  TnShape s;
   const int tiles = tn_tiles(m, b, cp);
-  const int w = tn_waves(tiles);
-  const int64_t blocks_per_chunk = (tiles + w - 1) / w;
-  int64_t want = std::max<int64_t>(1, tn_resident(w, cp) / blocks_per_chunk);
-  want = std::min<int64_t>(want, 65535);
-  rows_per_chunk = (n + want - 1) / want;
-  rows_per_chunk = std::max<int64_t>(64, (rows_per_chunk + 15) / 16 * 16);
-  nchunks = (n + rows_per_chunk - 1) / rows_per_chunk;
+  s.wt = tn_waves(tiles);
+  const int64_t blocks_per_chunk = (tiles + s.wt - 1) / s.wt;
+  for (s.subs = 8 / s.wt;; --s.subs) {
+    int units = 0;
+    int64_t want = std::max<int64_t>(1, tn_resident(s.wt * s.subs, cp, &units) / blocks_per_chunk);
+    want = std::min<int64_t>(want, 65535);
+    s.rows_per_sub = (n + want * s.subs - 1) / (want * s.subs);
+    s.rows_per_sub = std::max<int64_t>(64, (s.rows_per_sub + 15) / 16 * 16);
+    s.nchunks = (n + s.rows_per_sub * s.subs - 1) / (s.rows_per_sub * s.subs);
+    if (s.subs == 1 || s.nchunks * blocks_per_chunk >= units) return s;
+  }
 }
 
 }  // namespace
 
+char* Linalg::stage(size_t bytes) {
+  HostBuf& b = host->in;
+  bytes = (bytes + 63) / 64 * 64;
+  if (b.used + bytes > b.n) {
+    PSOCI_HIP(hipStreamSynchronize(stream));
+    b.reserve(std::max(bytes, (size_t)256 << 10));
+    b.used = 0;
+  }
+  char* p = b.p + b.used;
+  b.used += bytes;
+  return p;
+}
+
+void Linalg::put(void* dst, const char* staged, size_t bytes) {
+  const int64_t words = (int64_t)((bytes + 7) / 8);
+  hipLaunchKernelGGL(k_put, dim3(nblk(words, 256)), dim3(256), 0, stream, words,
+                     reinterpret_cast<const uint64_t*>(staged), static_cast<uint64_t*>(dst));
+  PSOCI_HIP(hipGetLastError());
+}
+
+void Linalg::put_y(const double* y, size_t count) {
+  char* st = stage(count * sizeof(double));
+  std::copy(y, y + count, reinterpret_cast<double*>(st));
+  put(ysmall.p, st, count * sizeof(double));
+}
+
+double* Linalg::results(size_t count) {
+  if (count * sizeof(double) > host->out.n) {
+    PSOCI_HIP(hipStreamSynchronize(stream));
+    host->out.reserve(std::max(count * sizeof(double), (size_t)64 << 10));
+  }
+  return reinterpret_cast<double*>(host->out.p);
+}
+
 size_t Linalg::tn_part_size(int64_t n, int m, int b) {
   // the larger of the FP64 and FP32 kernels' needs
-  int64_t rpc, nch1, nch2;
-  tn_chunks(n, m, b, 1, rpc, nch1);
-  tn_chunks(n, m, b, 2, rpc, nch2);
-  return (size_t)std::max(nch1, nch2) * m * b;
+  return (size_t)std::max(tn_shape(n, m, b, 1).nchunks, tn_shape(n, m, b, 2).nchunks) * m * b;
 }
 
 void Linalg::reserve_tn(int64_t n, int mmax, int bmax) {
@@ -568,25 +651,24 @@ template <typename TA>
 void Linalg::gemm_tn(int64_t n, int m, int b, const TA* A, int lda, const TA* B, int ldb, double* out_dev) {
   if (m == 0 || b == 0) return;
   constexpr int cp = tn_cols<TA>();
-  int64_t rows_per_chunk, nchunks;
-  tn_chunks(n, m, b, cp, rows_per_chunk, nchunks);
-  part.reserve((size_t)nchunks * m * b);
-  const int tiles = tn_tiles(m, b, cp);
-  const int w = tn_waves(tiles);
-  dim3 grid(nblk(tiles, w), (unsigned)nchunks);
-  hipLaunchKernelGGL(k_gemm_tn_mfma<TA>, grid, dim3(kWave * w), 0, stream, n, m, b, A, lda, B, ldb, rows_per_chunk,
-                     part.p);
+  const TnShape t = tn_shape(n, m, b, cp);
+  part.reserve((size_t)t.nchunks * m * b);
+  dim3 grid(nblk(tn_tiles(m, b, cp), t.wt), (unsigned)t.nchunks);
+  hipLaunchKernelGGL(k_gemm_tn_mfma<TA>, grid, dim3(kWave * t.wt * t.subs), 0, stream, n, m, b, A, lda, B, ldb, t.wt,
+                     t.rows_per_sub, part.p);
   PSOCI_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce_chunks, dim3((unsigned)(m * b)), dim3(256), 0, stream, nchunks, m * b, part.p, out_dev);
+  hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk((int64_t)m * b, kRedEntries)), dim3(kRedEntries * kRedGroups), 0,
+                     stream, t.nchunks, m * b, part.p, out_dev);
   PSOCI_HIP(hipGetLastError());
 }
 
 template <typename TA>
 void Linalg::gemm_tn_host(int64_t n, int m, int b, const TA* A, int lda, const TA* B, int ldb, double* out_host) {
-  small.reserve((size_t)m * b);
-  gemm_tn(n, m, b, A, lda, B, ldb, small.p);
-  PSOCI_HIP(hipMemcpyAsync(out_host, small.p, (size_t)m * b * sizeof(double), hipMemcpyDeviceToHost, stream));
+  double* res = results((size_t)m * b);
+  gemm_tn(n, m, b, A, lda, B, ldb, res);
   PSOCI_HIP(hipStreamSynchronize(stream));
+  host->in.used = 0;  // everything staged has been consumed
+  std::copy(res, res + (size_t)m * b, out_host);
 }
 
 namespace {
@@ -623,7 +705,7 @@ void Linalg::gemm_nn(int64_t n, int m, int k, const TA* A, int lda, const double
                      int ldo) {
   if (k == 0 || n == 0) return;
   ysmall.reserve((size_t)m * k);
-  PSOCI_HIP(hipMemcpyAsync(ysmall.p, Y1_host, (size_t)m * k * sizeof(double), hipMemcpyHostToDevice, stream));
+  put_y(Y1_host, (size_t)m * k);
   launch_nn<false, false, false, TA, TO>(stream, n, m, k, A, lda, nullptr, 0, ysmall.p, nullptr, alpha, Out, ldo,
                                          nullptr, 0);
 }
@@ -633,7 +715,7 @@ void Linalg::gemm_nn_rows(int64_t n, int m, int k, const T* A, int lda, const do
   if (k == 0 || n == 0) return;
   PSOCI_CHECK(k <= 128, PSOCI_ERR_ARG, "row-aliased product: at most 128 output columns");
   ysmall.reserve((size_t)m * k);
-  PSOCI_HIP(hipMemcpyAsync(ysmall.p, Y1_host, (size_t)m * k * sizeof(double), hipMemcpyHostToDevice, stream));
+  put_y(Y1_host, (size_t)m * k);
   launch_nn<false, false, false, T, T>(stream, n, m, k, A, lda, nullptr, 0, ysmall.p, nullptr, 0.0, Out, ldo, nullptr,
                                        0);
 }
@@ -643,7 +725,7 @@ void Linalg::gemm_nn_inplace(int64_t n, int m, int k, const double* Y1_host, T* 
   if (k == 0 || n == 0) return;
   PSOCI_CHECK(k <= 128 && k <= m, PSOCI_ERR_ARG, "in-place product: at most 128 and at most m output columns");
   ysmall.reserve((size_t)m * k);
-  PSOCI_HIP(hipMemcpyAsync(ysmall.p, Y1_host, (size_t)m * k * sizeof(double), hipMemcpyHostToDevice, stream));
+  put_y(Y1_host, (size_t)m * k);
   launch_nn<false, false, true, T, T>(stream, n, m, k, nullptr, 0, nullptr, 0, ysmall.p, nullptr, 0.0, Out, ldo,
                                       nullptr, 0);
 }
@@ -653,24 +735,27 @@ void Linalg::gemm_nn2(int64_t n, int m, int k, const TA* A, int lda, const doubl
                       const double* Y2_host, TO* Out, int ldo, double* X, int ldx) {
   if (k == 0 || n == 0) return;
   ysmall.reserve((size_t)2 * m * k);
-  yneg.assign(Y2_host, Y2_host + (size_t)m * k);
-  for (auto& v : yneg) v = -v;
-  PSOCI_HIP(hipMemcpyAsync(ysmall.p, Y1_host, (size_t)m * k * sizeof(double), hipMemcpyHostToDevice, stream));
-  PSOCI_HIP(hipMemcpyAsync(ysmall.p + (size_t)m * k, yneg.data(), (size_t)m * k * sizeof(double),
-                           hipMemcpyHostToDevice, stream));
+  const size_t mk = (size_t)m * k;
+  char* st = stage(2 * mk * sizeof(double));
+  double* y = reinterpret_cast<double*>(st);
+  for (size_t e = 0; e < mk; ++e) {
+    y[e] = Y1_host[e];
+    y[mk + e] = -Y2_host[e];
+  }
+  put(ysmall.p, st, 2 * mk * sizeof(double));
   if (X)
     launch_nn<true, true, false, TA, TO>(stream, n, m, k, A, lda, B, ldb, ysmall.p, ysmall.p + (size_t)m * k, 0.0,
                                          Out, ldo, X, ldx);
   else
     launch_nn<true, false, false, TA, TO>(stream, n, m, k, A, lda, B, ldb, ysmall.p, ysmall.p + (size_t)m * k, 0.0,
                                           Out, ldo, nullptr, 0);
-  // yneg is read by the copy above: keep it until the stream has consumed it
-  PSOCI_HIP(hipStreamSynchronize(stream));
 }
 
 void Linalg::precondition(int64_t n, int k, const double* D, const double* theta_host, double dmin, double* R, int ldr) {
   theta.reserve(k);
-  PSOCI_HIP(hipMemcpyAsync(theta.p, theta_host, k * sizeof(double), hipMemcpyHostToDevice, stream));
+  char* st = stage(k * sizeof(double));
+  std::copy(theta_host, theta_host + k, reinterpret_cast<double*>(st));
+  put(theta.p, st, k * sizeof(double));
   hipLaunchKernelGGL(k_precondition, dim3(nblk(n * k, 256)), dim3(256), 0, stream, n, k, D, theta.p, dmin, R, ldr);
   PSOCI_HIP(hipGetLastError());
 }
@@ -679,25 +764,29 @@ template <typename TR, typename TO>
 void Linalg::precondition_select(int64_t n, int k, const double* D, const double* theta_host, double dmin,
                                  const TR* R, int ldr, const int* sel_host, int ns, TO* Out, int ldo) {
   if (ns == 0 || n == 0) return;
-  std::vector<double> ts(ns);
-  for (int j = 0; j < ns; ++j) ts[j] = theta_host[sel_host[j]];
   (void)k;
-  theta.reserve(ns);
-  isel.reserve(ns);
-  PSOCI_HIP(hipMemcpyAsync(theta.p, ts.data(), ns * sizeof(double), hipMemcpyHostToDevice, stream));
-  PSOCI_HIP(hipMemcpyAsync(isel.p, sel_host, ns * sizeof(int), hipMemcpyHostToDevice, stream));
+  // the roots' values, then their columns
+  const size_t bytes = ns * (sizeof(double) + sizeof(int));
+  theta.reserve(bytes / sizeof(double) + 1);
+  char* st = stage(bytes);
+  int* sel = reinterpret_cast<int*>(st + ns * sizeof(double));
+  for (int j = 0; j < ns; ++j) {
+    reinterpret_cast<double*>(st)[j] = theta_host[sel_host[j]];
+    sel[j] = sel_host[j];
+  }
+  put(theta.p, st, bytes);
   hipLaunchKernelGGL((k_precondition_select<TR, TO>), dim3(nblk(n * ns, 256)), dim3(256), 0, stream, n, ns, D, theta.p,
-                     isel.p, dmin, R, ldr, Out, ldo);
+                     reinterpret_cast<const int*>(theta.p + ns), dmin, R, ldr, Out, ldo);
   PSOCI_HIP(hipGetLastError());
-  // ts is read by the copy above: keep it until the stream has consumed it
-  PSOCI_HIP(hipStreamSynchronize(stream));
 }
 
 void Linalg::precondition_olsen(int64_t n, int k, const double* D, const double* theta_host, double dmin, double* R,
                                 int ldr, const double* X, int ldx) {
   if (k == 0 || n == 0) return;
   theta.reserve(k);
-  PSOCI_HIP(hipMemcpyAsync(theta.p, theta_host, k * sizeof(double), hipMemcpyHostToDevice, stream));
+  char* st = stage(k * sizeof(double));
+  std::copy(theta_host, theta_host + k, reinterpret_cast<double*>(st));
+  put(theta.p, st, k * sizeof(double));
   const int64_t rows_per_blk = 4096;
   const int64_t nb = (n + rows_per_blk - 1) / rows_per_blk;
   part.reserve((size_t)nb * 2 * k);
@@ -705,7 +794,8 @@ void Linalg::precondition_olsen(int64_t n, int k, const double* D, const double*
   hipLaunchKernelGGL(k_olsen_dots, dim3((unsigned)nb), dim3(256), 0, stream, n, k, D, theta.p, dmin, R, ldr, X, ldx,
                      rows_per_blk, part.p);
   PSOCI_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_reduce_chunks, dim3((unsigned)(2 * k)), dim3(256), 0, stream, nb, 2 * k, part.p, small.p);
+  hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(2 * k, kRedEntries)), dim3(kRedEntries * kRedGroups), 0, stream, nb,
+                     2 * k, part.p, small.p);
   PSOCI_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_olsen_apply, dim3(nblk(n * k, 256)), dim3(256), 0, stream, n, k, D, theta.p, dmin, small.p, R,
                      ldr, X, ldx);

@@ -4,12 +4,49 @@
 
 namespace psoci {
 
+// Host memory that kernels read and write in place (pinned, coherent).
+struct HostBuf {
+  char* p = nullptr;
+  size_t n = 0, used = 0;
+  HostBuf() = default;
+  HostBuf(const HostBuf&) = delete;
+  HostBuf& operator=(const HostBuf&) = delete;
+  ~HostBuf() {
+    if (p) (void)hipHostFree(p);
+  }
+  // grow only; the caller has made sure that no kernel uses the memory
+  void reserve(size_t bytes) {
+    if (bytes <= n) return;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = used = 0;
+    PSOCI_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), bytes, hipHostMallocDefault));
+    n = bytes;
+  }
+};
+
+// The small matrices of the block Davidson pass between host and device
+// through pinned memory: a kernel copies them in (put), and the reduction of
+// a projection writes its result into host memory.  hipMemcpyAsync on the
+// caller's pageable arrays waits for each copy on the host, 12 to 20 us of
+// idle GPU per product.
+struct LinalgHost {
+  HostBuf in, out;
+};
+
 struct Linalg {
   hipStream_t stream = nullptr;
+  LinalgHost* host = nullptr;
   DevBuf<double> part, small, ysmall, theta;
-  DevBuf<int> isel;
   DevBuf<int64_t> ipart;
-  std::vector<double> yneg;
+
+  // bytes of staged host memory, valid until the stream has consumed them
+  char* stage(size_t bytes);
+  // device dst = the staged words (enqueued)
+  void put(void* dst, const char* staged, size_t bytes);
+  void put_y(const double* y, size_t count);  // into ysmall
+  // the projections' results in host memory: room for count doubles
+  double* results(size_t count);
 
   // partial-sum buffer of gemm_tn for (n, m, b); reserve_tn: for every
   // m <= mmax, b <= bmax (so captured launches allocate nothing)
