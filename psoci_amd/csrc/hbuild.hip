@@ -147,29 +147,47 @@ __device__ __forceinline__ bool connected(uint64_t a, uint64_t b, uint64_t sx) {
   return popc(x) + popc(x ^ sx) <= 4 && popc(a) == popc(b);
 }
 
+// The pairs of a wavefront's steps of 64 elements: the lanes mark the block
+// boundaries among the step's elements (mark: a wavefront's 64 words of LDS),
+// a ballot and a count give each lane its pair.
+struct PairWalk {
+  int64_t p0, next;  // the step's first pair and its end
+  __device__ __forceinline__ PairWalk(int64_t p, const int64_t* __restrict__ blk_off) : p0(p), next(blk_off[p + 1]) {}
+  __device__ __forceinline__ int64_t step(int64_t es, int lane, uint32_t* mark, int64_t npairs,
+                                          const int64_t* __restrict__ blk_off) {
+    if (next - es > kWave) return p0;
+    // boundaries past p0's first element (all at 1 or later)
+    mark[lane] = 0;
+    lds_order();
+    const int64_t pb = p0 + 1 + lane;
+    const int64_t left = pb <= npairs ? blk_off[pb] - es : kWave + 1;
+    if (left < kWave) mark[left] = 1;
+    lds_order();
+    const int64_t p = p0 + popc(__ballot(mark[lane] != 0) & ((2ull << lane) - 1ull));
+    p0 += popc(__ballot(left <= kWave));
+    if (p0 < npairs) next = blk_off[p0 + 1];
+    return p;
+  }
+};
+
 // Elements of the blocks, in block order: element (i, j) of pair p is number
 // blk_off[p] + i * nsef_J + j.  Kept ones (|h| >= 1e-8, and the diagonal; of
 // a diagonal block its lower triangle) get their bit; their values stand
 // together at the start of each batch of kBatch elements (staging), and
 // rank[w] counts those of the batch before word w of the bits.  Values left at
-// their own elements cost the rows' gather a memory line each.  tbits holds
-// the same bits with each block transposed (zeroed before; element (i, j) is
-// bit blk_off[p] + j * nsef_I + i).
+// their own elements cost the rows' gather a memory line each.
 //
 // One wavefront per 512 elements.  Bound by vector instructions: a
 // determinant pair's evaluation is some 150 and about one element in ten is
 // connected at all, so each 64-element step only tests its elements (the XOR
 // of two 64-bit masks and its counts) and appends the connected ones to a
 // queue in LDS; the queue is then evaluated 64 at a time, every lane with
-// work.  The pairs of a step are found from the first one: lanes mark the
-// block boundaries among its 64 elements, a ballot and a count give each
-// lane its pair.  Of an even-electron element's four determinant pairs two
-// are evaluated: flipping every open spin on both sides leaves a determinant
+// work.  Of an even-electron element's four determinant pairs two are
+// evaluated: flipping every open spin on both sides leaves a determinant
 // pair's element as it is, bit for bit (spin-orbit pairs take all four).
 // Measured on full CI of 10 orbitals and 8 electrons (31,650 SEFs, 78 M
-// elements): 0.64 ms, a third of it the transposed bits' atomics; a thread
-// per element, with its own search for its pair and four evaluations, took
-// 2.24 ms.
+// elements): 0.44 ms; a thread per element, with its own search for its pair
+// and four evaluations, took 2.24 ms.
 template <bool FRAC>
 __global__ __launch_bounds__(256) void k_block_elems(
     int64_t total, int64_t npairs, const int64_t* __restrict__ blk_off, const int64_t* __restrict__ first,
@@ -177,7 +195,7 @@ __global__ __launch_bounds__(256) void k_block_elems(
     const int8_t* __restrict__ nopen, const uint8_t* __restrict__ cph, const double* __restrict__ cmult,
     const int32_t* __restrict__ nsef, const int64_t* __restrict__ sefoff, const uint64_t* __restrict__ amask,
     const double* __restrict__ two, double* __restrict__ staging, uint64_t* __restrict__ bits,
-    uint64_t* __restrict__ tbits, uint16_t* __restrict__ rank) {
+    uint16_t* __restrict__ rank) {
   __shared__ uint32_t sh_mark[4][kWave];
   __shared__ uint32_t sh_queue[4][kBatch];
   __shared__ uint32_t sh_bits[4][kBatch / 32];
@@ -190,7 +208,7 @@ __global__ __launch_bounds__(256) void k_block_elems(
   uint32_t* queue = sh_queue[wv];
   uint32_t* wb = sh_bits[wv];
   const int64_t pf = first[batch];
-  int64_t p0 = pf, next = blk_off[pf + 1];  // the step's first pair and its end
+  PairWalk walk(pf, blk_off);
   int nq = 0;
   if (lane < kBatch / 32) wb[lane] = 0;
   // the lane's pair: kept while its elements stay in it (a block of more than
@@ -203,19 +221,7 @@ __global__ __launch_bounds__(256) void k_block_elems(
   for (int c = 0; c < kBatch / kWave; ++c) {
     const int64_t es = e0 + c * kWave;
     if (es >= total) break;
-    int64_t p = p0;
-    if (next - es <= kWave) {
-      // block boundaries past p0's first element (all at 1 or later)
-      mark[lane] = 0;
-      lds_order();
-      const int64_t pb = p0 + 1 + lane;
-      const int64_t left = pb <= npairs ? blk_off[pb] - es : kWave + 1;
-      if (left < kWave) mark[left] = 1;
-      lds_order();
-      p += popc(__ballot(mark[lane] != 0) & ((2ull << lane) - 1ull));
-      p0 += popc(__ballot(left <= kWave));
-      if (p0 < npairs) next = blk_off[p0 + 1];
-    }
+    const int64_t p = walk.step(es, lane, mark, npairs, blk_off);
     const int64_t e = es + lane;
     bool ok = false;
     if (e < total) {
@@ -246,7 +252,6 @@ __global__ __launch_bounds__(256) void k_block_elems(
   for (int k0 = 0; k0 < nq; k0 += kWave) {
     double v = 0.0;
     unsigned rel = 0;
-    int64_t tpos = 0;
     bool keep = false;
     if (k0 + lane < nq) {
       const uint32_t ent = queue[k0 + lane];
@@ -265,14 +270,12 @@ __global__ __launch_bounds__(256) void k_block_elems(
       else
         v = sef_elem_flip(P, A, B, a0, b0, cmult[P.I], cmult[P.J], two);
       keep = fabs(v) >= kThresh || (P.I == P.J && i == j);
-      tpos = blk_off[p] + (int64_t)j * nsef[P.I] + i;
     }
     // the queue is in element order, and so are the values
     const uint64_t mk = __ballot(keep);
     if (keep) {
       staging[e0 + kept + popc(mk & ((1ull << lane) - 1ull))] = v;
       atomicOr(&wb[rel >> 5], 1u << (rel & 31));
-      atomicOr(reinterpret_cast<uint32_t*>(tbits) + (tpos >> 5), 1u << (tpos & 31));
     }
     kept += popc(mk);
   }
@@ -286,6 +289,60 @@ __global__ __launch_bounds__(256) void k_block_elems(
       rank[w] = (uint16_t)before;
     }
   }
+}
+
+// The same bits with each block transposed: element (i, j) of pair p is bit
+// blk_off[p] + j * nsef_I + i.  One wavefront per 512 bits, a lane fetches
+// the source bit of one of a step's 64; bound by the latency of the
+// walk over the blocks (0.15 ms for 78 M bits; set one by one with atomics
+// where the elements are evaluated they took 0.21 ms).
+__global__ __launch_bounds__(256) void k_transpose_bits(int64_t total, int64_t npairs,
+                                                        const int64_t* __restrict__ blk_off,
+                                                        const int64_t* __restrict__ first,
+                                                        const PairInfo* __restrict__ pairs,
+                                                        const int32_t* __restrict__ nsef,
+                                                        const uint64_t* __restrict__ bits,
+                                                        uint64_t* __restrict__ tbits) {
+  __shared__ uint32_t sh_mark[4][kWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t batch = (int64_t)blockIdx.x * (blockDim.x / kWave) + wv;
+  const int64_t e0 = batch * kBatch;
+  if (e0 >= total) return;  // uniform per wavefront; no workgroup barrier below
+  PairWalk walk(first[batch], blk_off);
+  int64_t pc = -1, off = 0;
+  int shi = 0, shj = 0;
+  // all source words are fetched before the first is used
+  uint64_t word[kBatch / kWave];
+  int at[kBatch / kWave];
+#pragma unroll
+  for (int c = 0; c < kBatch / kWave; ++c) {
+    const int64_t es = e0 + c * kWave, e = es + lane;
+    word[c] = 0;
+    at[c] = 0;
+    if (es < total) {
+      const int64_t p = walk.step(es, lane, sh_mark[wv], npairs, blk_off);
+      if (e < total) {
+        if (p != pc) {
+          pc = p;
+          off = blk_off[p];
+          shi = popc((uint64_t)(nsef[pairs[p].I] - 1));
+          shj = popc((uint64_t)(nsef[pairs[p].J] - 1));
+        }
+        const unsigned loc = (unsigned)(e - off), j = loc >> shi, i = loc - (j << shi);
+        const int64_t src = off + ((i << shj) | j);
+        at[c] = (int)(src & 63);
+        word[c] = bits[src >> 6];
+      }
+    }
+  }
+  uint64_t out = 0;  // lane c's word of the batch
+#pragma unroll
+  for (int c = 0; c < kBatch / kWave; ++c) {
+    const uint64_t m = __ballot(word[c] >> at[c] & 1ull);
+    if (lane == c) out = m;
+  }
+  if (lane < kBatch / 64 && e0 + lane * 64 < total) tbits[e0 / 64 + lane] = out;
 }
 
 // One segment of a configuration's rows: the block that holds it.  Row j's
@@ -630,7 +687,6 @@ void build_h(Ctx& c) {
   int64_t* first = sb.take<int64_t>(nbatch);
   uint64_t* amask = sb.take<uint64_t>(n);
   int32_t* cfg = sb.take<int32_t>(n);
-  PSOCI_HIP(hipMemsetAsync(tbits, 0, (nwords + 2) * sizeof(uint64_t), c.stream));
   hipLaunchKernelGGL(k_sef_masks, dim3(per_cfg), dim3(256), 0, c.stream, ncfg, c.d_dm.p, c.d_sm.p, c.d_nopen.p,
                      c.d_pat.p, c.d_patoff.p, c.d_cls.p, c.d_nsef.p, c.d_sefoff.p, sp.frac ? 1 : 0, amask, cfg);
   PSOCI_HIP(hipGetLastError());
@@ -639,7 +695,10 @@ void build_h(Ctx& c) {
   // a wavefront per batch
   hipLaunchKernelGGL(sp.frac ? k_block_elems<true> : k_block_elems<false>, dim3(blocks_for(nbatch, 4)), dim3(256), 0,
                      c.stream, nstage, np, boff, first, info, c.d_dm.p, c.d_sm.p, c.d_nopen.p, c.d_cph.p, c.d_cmult.p,
-                     c.d_nsef.p, c.d_sefoff.p, amask, c.d_two.p, staging, bits, tbits, rank);
+                     c.d_nsef.p, c.d_sefoff.p, amask, c.d_two.p, staging, bits, rank);
+  PSOCI_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_transpose_bits, dim3(blocks_for(nbatch, 4)), dim3(256), 0, c.stream, nstage, np, boff, first,
+                     info, c.d_nsef.p, bits, tbits);
   PSOCI_HIP(hipGetLastError());
   // the rows: counts, offsets, elements
   hipLaunchKernelGGL(k_segs, dim3((unsigned)ncfg), dim3(256), 0, c.stream, ncfg, off.p, list, info, boff, c.d_nsef.p,
