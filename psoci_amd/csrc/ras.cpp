@@ -170,7 +170,8 @@ bool strings_pay(int nI, int nE, int m, const std::vector<std::pair<int, int>>& 
 // 28).  Sigma of 16 columns: FP32 48.7 -> 31.4 ms, FP64 86.0 -> 52.1 ms; on
 // 8 + 24 orbitals, 6 electrons (5.8e9 -> 4.2e9 flops) FP64 8 columns 1.36 ->
 // 1.02 ms.
-RasCmp compact(RasPlan& P, const RasBlockDev& B, int nI, int nE) {
+// full: level 0 throughout.
+RasCmp compact(RasPlan& P, const RasBlockDev& B, int nI, int nE, bool full) {
   const Binom& Bn = binom();
   RasCmp C;
   std::memset(&C, 0, sizeof(C));
@@ -198,7 +199,7 @@ RasCmp compact(RasPlan& P, const RasBlockDev& B, int nI, int nE) {
     return a * (a - 1) / 2 + (b >= 1 ? a * nE : 0) + (b >= 2 ? nE * (nE - 1) / 2 : 0);
   };
   double best = 0.0;
-  for (int level = 0; level <= (C.kind == 0 ? 2 : 1); ++level) {
+  for (int level = 0; level <= (full ? 0 : C.kind == 0 ? 2 : 1); ++level) {
     RasCmp T = C;
     T.level = level;
     const double nqp = (live(level) + 15) / 16 * 16;
@@ -227,6 +228,14 @@ RasCmp compact(RasPlan& P, const RasBlockDev& B, int nI, int nE) {
 }
 
 }  // namespace
+
+void ras_compact(RasPlan& P, bool full) {
+  const int nE = __builtin_popcountll(P.emask);
+  P.cmp.clear();
+  P.cwunit = P.cdunit = P.cgunit = 0;
+  P.cflops_per_col = 0.0;
+  for (const RasBlockDev& B : P.blk) P.cmp.push_back(compact(P, B, P.nbf - nE, nE, full));
+}
 
 void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two, bool general, bool all) {
   P = RasPlan();
@@ -525,7 +534,7 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
     }
   }
   (void)nb2;
-  for (const RasBlockDev& B : P.blk) P.cmp.push_back(compact(P, B, rk.nI, rk.nE));
+  ras_compact(P, false);
   if (wunit >= ((int64_t)1 << 31)) return fail("more than 2^31 W elements per column");
   if (dunit >= ((int64_t)1 << 31)) return fail("more than 2^31 D index entries");
   P.wunit = wunit;

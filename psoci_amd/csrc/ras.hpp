@@ -584,6 +584,9 @@ inline void ras_cmp_groups(const RasCmp& C, F&& f) {
 struct Space;
 void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two, bool general = false,
               bool all = false);
+// The plan's compact layouts; full: none dropped (level 0), whose one matrix
+// per product takes the least memory for matrices.
+void ras_compact(RasPlan& P, bool full);
 // A view of the plan's host tables (host pointers), e.g. for a host check.
 RasView ras_host_view(const RasPlan& P);
 

@@ -955,11 +955,18 @@ bool build_ras(Ctx& c) {
         const RasSectorDev& S = P.sec[e.sec[d]];
         terms += (int64_t)S.na * S.nb + (int64_t)S.na * (S.na - 1) / 2 + (int64_t)S.nb * (S.nb - 1) / 2;
       }
-    const double need = (double)P.cwunit * 64 + (double)P.cdunit * 4 + (double)P.cgunit * 12 + (double)P.ndet * 128 +
-                        (double)terms * 4 + (double)P.sef.size() * 9;
+    auto needs = [&] {
+      return (double)P.cwunit * 64 + (double)P.cdunit * 4 + (double)P.cgunit * 12 + (double)P.ndet * 128 +
+             (double)terms * 4 + (double)P.sef.size() * 9;
+    };
     size_t fr = 0, tot = 0;
     c.spare.give_back();
     PSOCI_HIP(hipMemGetInfo(&fr, &tot));
+    // the matrices per row group can take more than the W elements they save
+    // (10 + 24 orbitals: 18.8 GB against 17 GB): where that is too much, one
+    // matrix per product
+    if (needs() > 0.6 * (double)fr) ras_compact(c.ras, true);
+    const double need = needs();
     // FP64 in chunks of 16 columns (whole 128-byte W and c pieces) when W and
     // c fit twice over in 60 % of the free memory, else chunks of 8
     c.ras_kc64 = need + (double)P.cwunit * 64 + (double)P.ndet * 128 <= 0.6 * (double)fr ? 16 : 8;

@@ -11,7 +11,8 @@ using namespace psoci;
 
 // Y[n][k] = H X[n][k] through the compact products; info[0..2] = blocks
 // per level, info[3..4] =
-// full and compact multiply-adds, info[5] = the list's share of the space.  0
+// full and compact multiply-adds, info[5] = the list's share of the space.
+// general: bit 0 general plans, bit 1 the layouts without dropped pairs.  0
 // on success.
 extern "C" int hrc_sigma(int nbf, int nelec, int ksym, int64_t ncfg, const uint8_t* occ, const int32_t* jsym,
                          const double* one, const double* two, int k, const double* X, double* Y, double* info,
@@ -20,7 +21,8 @@ extern "C" int hrc_sigma(int nbf, int nelec, int ksym, int64_t ncfg, const uint8
   RasPlan P;
   try {
     build_space(sp, nbf, nelec, ksym, ncfg, occ, jsym);
-    ras_plan(P, sp, one, two, general != 0, true);
+    ras_plan(P, sp, one, two, (general & 1) != 0, true);
+    if (P.ok && (general & 2)) ras_compact(P, true);
   } catch (const Error&) {
     return -1;
   }

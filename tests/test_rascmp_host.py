@@ -95,6 +95,14 @@ def test_compact_products_match_oracle(lib, name, make, levels):
     assert info[5] == 1.0
 
 
+@pytest.mark.parametrize("name,make,levels", [c for c in CASES if c[2]], ids=[c[0] for c in CASES if c[2]])
+def test_layouts_without_dropped_pairs(lib, name, make, levels):
+    rc, Y, ref, info = _run(lib, *make(), 2)
+    assert rc == 0, rc
+    np.testing.assert_allclose(Y, ref, rtol=0, atol=1e-12 * np.abs(ref).max())
+    assert info[1] == info[2] == 0 and info[4] == info[3]
+
+
 def _part(cfg, ints, share, seed=9):
     keep = np.random.default_rng(seed).random(cfg.ncfg) < share
     return (inputs.Configs(nbf=cfg.nbf, nelec=cfg.nelec, ksym=cfg.ksym, occ=cfg.occ[keep].copy(),
