@@ -180,7 +180,7 @@ int psoci_get_h(psoci_ctx* ctx, int64_t* rowptr, int32_t* col, double* val, doub
  * --hamiltonian_restart).  The
  * file holds the lower triangle + diagonal in the reference's row layout
  * (as psoci_get_h returns it), fingerprints of the configuration list and
- * the integrals, the tuned stored-sigma shapes and a payload checksum.
+ * the integrals, the stored-sigma shapes and a payload checksum.
  * psoci_h_load needs psoci_set_configs and psoci_set_integrals with the same
  * inputs as the writer (PSOCI_ERR_ARG otherwise, and for a truncated or
  * corrupted file; such failures leave the context as it was) and then
