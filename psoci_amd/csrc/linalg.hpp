@@ -20,7 +20,7 @@ struct HostBuf {
     if (p) (void)hipHostFree(p);
     p = nullptr;
     n = used = 0;
-    PSOCI_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), bytes, hipHostMallocDefault));
+    PSOCI_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), bytes, hipHostMallocCoherent));
     n = bytes;
   }
 };
