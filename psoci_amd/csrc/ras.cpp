@@ -605,6 +605,42 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
   P.ok = true;
 }
 
+RasGrad ras_grad(const RasPlan& P) {
+  RasGrad R;
+  R.of.assign(P.blk.size(), -1);
+  std::vector<const RasBlockDev*> first;  // a block of each matrix
+  for (size_t bi = 0; bi < P.blk.size(); ++bi) {
+    const RasBlockDev& B = P.blk[bi];
+    // (an orbital that every configuration fills leaves same-spin products
+    // without a pair; the next matrix starts at the same G)
+    if (B.nq == 0) continue;
+    size_t x = 0;
+    while (x < first.size() &&
+           (first[x]->sector != B.sector || first[x]->kind != B.kind || first[x]->budget != B.budget))
+      ++x;
+    if (x == first.size()) {
+      const RasSectorDev& S = P.sec[B.sector];
+      RasGradMat G;
+      G.kind = B.kind;
+      G.nq = B.nq;
+      G.id = (B.kind ? 1 : 0) * (P.m + 1) + B.budget;
+      G.hr = G.hp = 0.0;
+      if (B.kind == 0) {
+        G.hr = 1.0 / S.nb;
+        G.hp = 1.0 / S.na;
+      } else if (S.na == 0 || S.nb == 0) {
+        G.hr = G.hp = 1.0 / ((B.kind == 1 ? S.na : S.nb) - 1);
+      }
+      G.moff = R.total;
+      R.total += (int64_t)B.nq * B.nq;
+      first.push_back(&B);
+      R.mat.push_back(G);
+    }
+    R.of[bi] = (int)x;
+  }
+  return R;
+}
+
 RasView ras_host_view(const RasPlan& P) {
   RasView v;
   std::memset(&v, 0, sizeof(v));

@@ -587,6 +587,19 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
 // The plan's compact layouts; full: none dropped (level 0), whose one matrix
 // per product takes the least memory for matrices.
 void ras_compact(RasPlan& P, bool full);
+// The adjoint's matrices: M = sum over rows and roots of w D D^T, one per
+// integral matrix (sector, kind, budget) and in its full pair layout.
+struct RasGradMat {
+  int kind, nq, id;  // id: row of the pair position table (shape and budget)
+  double hr, hp;     // factors of h_pq (r == s) and h_rs (p == q); same spin: of all four
+  int64_t moff;      // nq x nq elements from here
+};
+struct RasGrad {
+  std::vector<RasGradMat> mat;
+  std::vector<int> of;  // a block's matrix; -1: it has no pairs
+  int64_t total = 0;    // elements of all
+};
+RasGrad ras_grad(const RasPlan& P);
 // A view of the plan's host tables (host pointers), e.g. for a host check.
 RasView ras_host_view(const RasPlan& P);
 

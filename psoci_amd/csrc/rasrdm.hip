@@ -162,14 +162,7 @@ __global__ __launch_bounds__(256) void k_ras_fill0(int64_t n, double* __restrict
   if (t < n) p[t] = 0.0;
 }
 
-// One distinct integral matrix of the plan and its M.
-struct GradMat {
-  int kind, nq, id;  // id: row of the pair position table (shape and budget)
-  double hr, hp;     // factors of h_pq (r == s) and h_rs (p == q); same spin: of all four
-  int64_t moff;
-};
-
-__device__ __forceinline__ double gram_at(const GradMat& G, const double* __restrict__ M,
+__device__ __forceinline__ double gram_at(const RasGradMat& G, const double* __restrict__ M,
                                           const int16_t* __restrict__ px, int nbf, int p, int r, int q, int s) {
   const int i = px[p * nbf + r], j = px[q * nbf + s];
   if (i < 0 || j < 0) return 0.0;
@@ -180,7 +173,7 @@ __device__ __forceinline__ double gram_at(const GradMat& G, const double* __rest
 // dE/d(ij|kl): M over the distinct index orders of the packed integral.  An
 // alpha-beta entry [(p,r)][(q,s)] reads (pq|rs); a same-spin one (p > r, q >
 // s) reads (pq|rs) - (ps|rq).
-__global__ __launch_bounds__(256) void k_ras_grad2(int nbf, int64_t n2, int nmat, const GradMat* __restrict__ mat,
+__global__ __launch_bounds__(256) void k_ras_grad2(int nbf, int64_t n2, int nmat, const RasGradMat* __restrict__ mat,
                                                    const int16_t* __restrict__ pidx, const double* __restrict__ M,
                                                    double* __restrict__ g2) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -213,7 +206,7 @@ __global__ __launch_bounds__(256) void k_ras_grad2(int nbf, int64_t n2, int nmat
       d = x;
     }
     for (int m = 0; m < nmat; ++m) {
-      const GradMat G = mat[m];
+      const RasGradMat G = mat[m];
       const int16_t* __restrict__ px = pidx + (int64_t)G.id * nbf * nbf;
       if (G.kind == 0) {
         s += gram_at(G, M, px, nbf, a, c, b, d);
@@ -227,7 +220,7 @@ __global__ __launch_bounds__(256) void k_ras_grad2(int nbf, int64_t n2, int nmat
 }
 
 // dE/dh_xy: the one-electron integrals folded into the matrices (ras_plan)
-__global__ __launch_bounds__(64) void k_ras_grad1(int nbf, int n1, int nmat, const GradMat* __restrict__ mat,
+__global__ __launch_bounds__(64) void k_ras_grad1(int nbf, int n1, int nmat, const RasGradMat* __restrict__ mat,
                                                   const int16_t* __restrict__ pidx, const double* __restrict__ M,
                                                   double* __restrict__ g1) {
   const int e = (int)blockIdx.x;
@@ -241,7 +234,7 @@ __global__ __launch_bounds__(64) void k_ras_grad1(int nbf, int n1, int nmat, con
     for (int o = 0; o < (hi == lo ? 1 : 2); ++o) {
       const int x = o ? lo : hi, y = o ? hi : lo;
       for (int m = 0; m < nmat; ++m) {
-        const GradMat G = mat[m];
+        const RasGradMat G = mat[m];
         const int16_t* __restrict__ px = pidx + (int64_t)G.id * nbf * nbf;
         if (G.kind == 0) {
           if (G.hr != 0.0) s += G.hr * gram_at(G, M, px, nbf, x, z, y, z);
@@ -262,10 +255,11 @@ __global__ __launch_bounds__(64) void k_ras_grad1(int nbf, int n1, int nmat, con
 }
 
 template <int KC>
-void gram_blocks(Ctx& c, const std::vector<int64_t>& moff, const double* wk, DevBuf<double>& part, double* M) {
+void gram_blocks(Ctx& c, const RasGrad& R, const double* wk, DevBuf<double>& part, double* M) {
   const RasPlan& P = c.ras;
   const double* cv = reinterpret_cast<const double*>(c.d_rasc.p);
   for (int bi = 0; bi < (int)P.blk.size(); ++bi) {
+    if (R.of[bi] < 0) continue;
     const RasBlockDev& B = P.blk[bi];
     const RasSectorDev& S = P.sec[B.sector];
     // a sector n_alpha > n_beta stands for its spin flip, a product of a
@@ -286,7 +280,7 @@ void gram_blocks(Ctx& c, const std::vector<int64_t>& moff, const double* wk, Dev
                        c.d_rasview.p, bi, fac, cv, wk, per, part.p);
     PSOCI_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_ras_gram_sum, dim3(nblk((int64_t)ntp * kPT * kPT, 256)), dim3(256), 0, c.stream, ntp,
-                       (int)nsplit, part.p, B.nq, M + moff[bi]);
+                       (int)nsplit, part.p, B.nq, M + R.mat[R.of[bi]].moff);
     PSOCI_HIP(hipGetLastError());
   }
 }
@@ -298,40 +292,14 @@ void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1
   const RasPlan& P = c.ras;
   const int nbf = P.nbf;
   const int64_t n1 = (int64_t)nbf * (nbf + 1) / 2, n2 = n1 * (n1 + 1) / 2;
-  // one M per distinct integral matrix (sector, kind, budget)
-  std::vector<GradMat> mat;
-  std::vector<int64_t> moff(P.blk.size()), gof;
-  int64_t tot = 0;
-  for (size_t bi = 0; bi < P.blk.size(); ++bi) {
-    const RasBlockDev& B = P.blk[bi];
-    size_t x = 0;
-    while (x < gof.size() && gof[x] != B.goff) ++x;
-    if (x == gof.size()) {
-      const RasSectorDev& S = P.sec[B.sector];
-      GradMat G;
-      G.kind = B.kind;
-      G.nq = B.nq;
-      G.id = (B.kind ? 1 : 0) * (P.m + 1) + B.budget;
-      G.hr = G.hp = 0.0;
-      if (B.kind == 0) {
-        G.hr = 1.0 / S.nb;
-        G.hp = 1.0 / S.na;
-      } else if (S.na == 0 || S.nb == 0) {
-        G.hr = G.hp = 1.0 / ((B.kind == 1 ? S.na : S.nb) - 1);
-      }
-      G.moff = tot;
-      tot += (int64_t)B.nq * B.nq;
-      gof.push_back(B.goff);
-      mat.push_back(G);
-    }
-    moff[bi] = mat[x].moff;
-  }
+  const RasGrad R = ras_grad(P);
+  const std::vector<RasGradMat>& mat = R.mat;
   DevBuf<double>&M = c.d_rdmm, &part = c.d_rdmpart, &wk = c.d_rdmw;
-  M.reserve(tot);
-  c.d_rdmmat.reserve(mat.size() * sizeof(GradMat));
-  PSOCI_HIP(hipMemcpyAsync(c.d_rdmmat.p, mat.data(), mat.size() * sizeof(GradMat), hipMemcpyHostToDevice, c.stream));
-  const GradMat* dm = reinterpret_cast<const GradMat*>(c.d_rdmmat.p);
-  hipLaunchKernelGGL(k_ras_fill0, dim3(nblk(tot, 256)), dim3(256), 0, c.stream, tot, M.p);
+  M.reserve(R.total);
+  c.d_rdmmat.reserve(mat.size() * sizeof(RasGradMat));
+  PSOCI_HIP(hipMemcpyAsync(c.d_rdmmat.p, mat.data(), mat.size() * sizeof(RasGradMat), hipMemcpyHostToDevice, c.stream));
+  const RasGradMat* dm = reinterpret_cast<const RasGradMat*>(c.d_rdmmat.p);
+  hipLaunchKernelGGL(k_ras_fill0, dim3(nblk(R.total, 256)), dim3(256), 0, c.stream, R.total, M.p);
   PSOCI_HIP(hipGetLastError());
   // the roots in chunks of 16, 8, 4 or 2, their weights padded with zeros
   std::vector<double> hw((size_t)k + 16, 0.0);
@@ -342,10 +310,10 @@ void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1
     const int kw = std::min(c.ras_kc64, k - c0);
     const int kc = ras_scatter64(c, dC, k, c0, kw);
     const double* wc = wk.p + c0;
-    if (kc == 16) gram_blocks<16>(c, moff, wc, part, M.p);
-    else if (kc == 8) gram_blocks<8>(c, moff, wc, part, M.p);
-    else if (kc == 4) gram_blocks<4>(c, moff, wc, part, M.p);
-    else gram_blocks<2>(c, moff, wc, part, M.p);
+    if (kc == 16) gram_blocks<16>(c, R, wc, part, M.p);
+    else if (kc == 8) gram_blocks<8>(c, R, wc, part, M.p);
+    else if (kc == 4) gram_blocks<4>(c, R, wc, part, M.p);
+    else gram_blocks<2>(c, R, wc, part, M.p);
   }
   hipLaunchKernelGGL(k_ras_grad2, dim3(nblk(n2, 256)), dim3(256), 0, c.stream, nbf, n2, (int)mat.size(), dm,
                      c.d_raspidx.p, M.p, d_g2);

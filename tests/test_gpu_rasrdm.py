@@ -66,3 +66,28 @@ def test_zero_integrals_keep_the_pair_walk():
     np.testing.assert_allclose(b2, a2, rtol=0, atol=1e-12 * np.abs(a2).max())
     A.close()
     B.close()
+
+
+@pytest.mark.parametrize("ksym", [1, 2])
+@pytest.mark.parametrize("nelec", [4, 6])
+def test_always_filled_orbital(nelec, ksym):
+    """A core orbital that every configuration fills: same-spin products
+    without a pair among the plan's blocks."""
+    c = inputs.fci_configs(6, nelec, ksym=ksym)
+    keep = c.occ[:, 0] == 2
+    cfg = inputs.Configs(nbf=6, nelec=nelec, ksym=ksym, occ=c.occ[keep].copy(), jsym=c.jsym[keep].copy())
+    ints = inputs.make_integrals(6, 5)
+    A = api.Hamiltonian(cfg, ints)
+    B = api.Hamiltonian(cfg, ints)
+    A.direct_engine(1)
+    assert B.direct_engine(2) == 2
+    rng = np.random.default_rng(5)
+    for k in (1, 3, 9):
+        C = rng.standard_normal((A.n, k))
+        a1, a2, _ = A.rdm(C)
+        b1, b2, _ = B.rdm(C)
+        scale = max(np.abs(a1).max(), np.abs(a2).max())
+        assert np.abs(b1 - a1).max() <= 1e-12 * scale, k
+        assert np.abs(b2 - a2).max() <= 1e-12 * scale, k
+    A.close()
+    B.close()
