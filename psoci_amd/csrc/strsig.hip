@@ -307,13 +307,15 @@ struct IntC {
 // stages apart, does not wait for every copy in flight before each LDS read:
 // the kernel waits for its copies itself (vmcnt(0) before the barrier that
 // publishes a stage).  M0 carries the LDS address; nothing else in the
-// kernels that use this keeps a value in M0.
+// kernels that use this keeps a value in M0.  A copy may not issue in the
+// instruction after the one that writes M0 (one wait state: the s_nop, which
+// the compiler does not add inside asm).
 __device__ __forceinline__ void lds_copy16(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
 }
 // the same from a uniform base plus this lane's byte offset
 __device__ __forceinline__ void lds_copy16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
                : "memory", "m0");
 }
 // LDS byte address of a __shared__ location, uniform over the wavefront
