@@ -1,6 +1,7 @@
 // extern "C" boundary of the PSOCI MI355X library (declared in include/psoci.h).
 // Every entry point catches psoci::Error and HIP failures and returns a
 // status code; the message is kept on the context for psoci_last_error().
+#include <algorithm>
 #include <cstring>
 
 #include "ctx.hpp"
@@ -36,6 +37,18 @@ int guarded(psoci_ctx* ctx, F&& f) {
   } catch (const std::exception& e) {
     ctx->c.err = e.what();
     return PSOCI_ERR_ARG;
+  }
+}
+
+// whether f ran; false where it found no device memory
+template <class F>
+bool fits(F&& f) {
+  try {
+    f();
+    return true;
+  } catch (const Error& e) {
+    if (e.code != PSOCI_ERR_NOMEM) throw;
+    return false;
   }
 }
 
@@ -102,6 +115,7 @@ int psoci_set_integrals(psoci_ctx* ctx, int nbf, const double* valone, const dou
                                     psoci::hash_bytes(valone, nndaf(nbf) * sizeof(double), (uint64_t)nbf));
     c.nbf_ints = nbf;
     c.ecore = ecore;
+    c.zero_integral = std::find(valtwo, valtwo + nndaf(nndaf(nbf)), 0.0) != valtwo + nndaf(nndaf(nbf));
     c.have_ints = true;
     c.have_h = c.have_diag = c.have_pairs = c.have_trans = false;
     c.drop_ras();
@@ -241,11 +255,12 @@ int psoci_direct_engine(psoci_ctx* ctx, int request, int* engine) {
   return guarded(ctx, [&](Ctx& c) {
     PSOCI_CHECK(request >= -1 && request <= 2, PSOCI_ERR_ARG, "request must be -1, 0, 1 or 2");
     const int before = c.direct_engine_req;
-    const bool tried = c.ras_tried;
+    const bool tried = c.ras_tried, tried_strings = c.strings_tried;
     if (request >= 0) {
       c.direct_engine_req = request;
-      if (request == 1 && c.have_ras) c.drop_ras();
+      if (request == 1 && c.have_strings) c.drop_ras();
       if (request == 2 && !c.have_ras) c.ras_tried = false;
+      if (request == 2 && !c.have_strings) c.strings_tried = false;
     }
     if (engine) {
       PSOCI_CHECK(c.have_space && c.have_ints, PSOCI_ERR_STATE, "configurations and integrals are required");
@@ -254,6 +269,7 @@ int psoci_direct_engine(psoci_ctx* ctx, int request, int* engine) {
       } catch (...) {
         c.direct_engine_req = before;  // a request that cannot be met leaves the choice as it was
         if (!c.have_ras) c.ras_tried = tried;
+        if (!c.have_strings) c.strings_tried = tried_strings;
         throw;
       }
       *engine = psoci::direct_engine(c);
@@ -453,20 +469,24 @@ int psoci_rdm(psoci_ctx* ctx, int k, const double* C, const double* w, double* g
     PSOCI_CHECK(k >= 1 && C, PSOCI_ERR_ARG, "bad RDM arguments");
     const int64_t n = c.sp.nsef_total;
     const int64_t n1 = nndaf(c.sp.nbf), n2 = nndaf(n1);
-    // complete RAS spaces: the string plan (kept from the direct sigma, or
-    // built for this call unless the pair records are there already)
-    if (c.direct_engine_req != 1 && !c.have_ras && !c.ras_tried && !c.have_pairs) {
-      c.ras_tried = true;
-      psoci::build_ras(c);
-    }
-    const bool strings = c.direct_engine_req != 1 && c.have_ras && c.ras_rdm;
-    if (!strings && !c.have_pairs) psoci::build_pairs(c);
+    // the strings where they serve (those of the direct sigma, or built for
+    // this call unless the pair records are there already), without the
+    // sigma's products; the pair records where they do not or memory is short
+    const bool may = c.direct_engine_req != 1 && !c.zero_integral;
+    if (may && !c.have_pairs) fits([&] { psoci::build_strings(c, true); });
     psoci::DevBuf<double> dC, g1, g2;
     dC.upload(C, (size_t)n * k, c.stream);
     g1.alloc(n1);
     g2.alloc(n2);
-    if (strings) psoci::ras_rdm_grad(c, k, dC.p, w, g1.p, g2.p);
-    else psoci::rdm_grad(c, k, dC.p, w, g1.p, g2.p);
+    bool done = false;
+    if (may && c.have_strings && c.ras_rdm) {
+      done = fits([&] { psoci::ras_rdm_grad(c, k, dC.p, w, g1.p, g2.p); });
+      if (!done) c.have_ras ? c.drop_adjoint() : c.drop_plan();
+    }
+    if (!done) {
+      if (!c.have_pairs) psoci::build_pairs(c);
+      psoci::rdm_grad(c, k, dC.p, w, g1.p, g2.p);
+    }
     if (grad_one) g1.download(grad_one, n1, c.stream);
     if (grad_two) g2.download(grad_two, n2, c.stream);
     c.sync();

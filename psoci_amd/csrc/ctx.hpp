@@ -150,8 +150,12 @@ struct Ctx {
   // space qualifies, else the configuration records; 1 configuration
   // records; 2 string-driven only) and the string-driven plan (strsig.hip)
   int direct_engine_req = 0;
+  // (two parts, each tried once: the strings, which the adjoint needs too,
+  // and the products)
+  bool have_strings = false, strings_tried = false;
   bool have_ras = false, ras_tried = false;
   std::string ras_why;
+  bool zero_integral = false;  // a two-electron integral is exactly zero
   RasPlan ras;
   DevBuf<uint64_t> d_rasmask;
   DevBuf<int8_t> d_rascls;
@@ -181,38 +185,50 @@ struct Ctx {
   bool ras_rdm = false;
   DevBuf<double> d_rdmm, d_rdmpart, d_rdmw;
   DevBuf<char> d_rdmmat;
-  void drop_ras() {
-    have_ras = ras_tried = ras_rdm = false;
+  void drop_products() {
+    have_ras = false;
+    d_rascmp.release();
+    for (int k = 0; k < 4; ++k) {
+      d_rastile[k].release();
+      ras_launch[k].clear();
+    }
+    d_rasg64.release();
+    d_rasg32.release();
+    d_rasw.release();
+    d_rasdidx.release();
+    d_rastoff.release();
+    d_rasterm.release();
+    d_rasscl.release();
+  }
+  void drop_adjoint() {
     d_rdmm.release();
     d_rdmpart.release();
     d_rdmw.release();
     d_rdmmat.release();
+  }
+  // everything built; what has been tried stays so
+  void drop_plan() {
+    drop_products();
+    drop_adjoint();
+    have_strings = ras_rdm = false;
     ras = RasPlan();
     d_rasmask.release();
     d_rascls.release();
     d_rasadd.release();
     d_rasrem.release();
     d_rasblk.release();
-    d_rascmp.release();
     d_rasq.release();
     d_raspidx.release();
-    for (int k = 0; k < 4; ++k) {
-      d_rastile[k].release();
-      ras_launch[k].clear();
-    }
     d_rassef.release();
-    d_rasg64.release();
-    d_rasg32.release();
     d_rasview.release();
     d_rasc.release();
-    d_rasw.release();
-    d_rasdidx.release();
-    d_rastoff.release();
-    d_rasterm.release();
-    d_rasscl.release();
     d_rasrows.release();
     d_rasorder.release();
     d_rasabsent.release();
+  }
+  void drop_ras() {
+    drop_plan();
+    strings_tried = ras_tried = false;
   }
 
   // transition Hamiltonian (rows: this list's SEFs; columns: a second
@@ -255,14 +271,16 @@ void block_on_device(Ctx& c, int64_t I, int64_t J, double* host_out, int* status
 void sigma_stored(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy, const Staging& st = Staging{});
 void sigma_direct(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy, const Staging& st = Staging{});
 int64_t direct_det_pairs(Ctx& c);
-// string-driven direct sigma (strsig.hip): the plan and its device tables
-// (false when the space does not qualify; c.ras_why says why), and the sigma
+// string-driven direct sigma (strsig.hip): the plan's strings (adjoint: only
+// where they serve the adjoint) and its products (false when the space does
+// not qualify; c.ras_why says why), and the sigma
+bool build_strings(Ctx& c, bool adjoint);
 bool build_ras(Ctx& c);
 void sigma_ras(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy);
 // columns [col0, col0 + kw) of X [n][ldx] as FP64 determinant vectors in
 // c.d_rasc; returns their padded width (16, 8, 4 or 2)
 int ras_scatter64(Ctx& c, const double* X, int ldx, int col0, int kw);
-// the adjoint through the string plan (needs have_ras and ras_rdm)
+// the adjoint through the string plan (needs have_strings and ras_rdm)
 void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1, double* d_g2);
 // one timed sigma of k columns on internal buffers, averaged over reps: ms[5]
 // per launch group (scatter, products by kind, gather), flops[3] per kind

@@ -288,7 +288,7 @@ void gram_blocks(Ctx& c, const RasGrad& R, const double* wk, DevBuf<double>& par
 }  // namespace
 
 void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1, double* d_g2) {
-  PSOCI_CHECK(c.have_ras && c.ras_rdm, PSOCI_ERR_STATE, "the string-driven adjoint is not set up");
+  PSOCI_CHECK(c.have_strings && c.ras_rdm, PSOCI_ERR_STATE, "the string-driven adjoint is not set up");
   const RasPlan& P = c.ras;
   const int nbf = P.nbf;
   const int64_t n1 = (int64_t)nbf * (nbf + 1) / 2, n2 = n1 * (n1 + 1) / 2;

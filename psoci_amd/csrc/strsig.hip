@@ -930,11 +930,28 @@ static void ras_tile_tables(Ctx& c) {
   c.sync();
 }
 
-// Builds the string plan and its device tables; false (c.ras_why says why)
-// when the space does not qualify.
-bool build_ras(Ctx& c) {
+// the plan's tables as the kernels read them
+static void ras_upload_view(Ctx& c) {
+  RasView v = ras_host_view(c.ras);
+  v.mask = c.d_rasmask.p;
+  v.cls = c.d_rascls.p;
+  v.add = c.d_rasadd.p;
+  v.rem = c.d_rasrem.p;
+  v.blk = c.d_rasblk.p;
+  v.qlist = c.d_rasq.p;
+  v.cmp = c.d_rascmp.p;
+  v.wunit = c.ras.cwunit;
+  v.pidx = c.d_raspidx.p;
+  v.sef = c.d_rassef.p;
+  c.d_rasview.upload(&v, 1, c.stream);
+  c.sync();
+}
+
+// Builds the plan's strings: the tables, the SEFs' determinants and the
+// determinant vectors, which the adjoint works on as well as the sigma; false
+// (c.ras_why says why) when the space does not qualify.
+static bool make_strings(Ctx& c, bool adjoint) {
   const Space& sp = c.sp;
-  c.have_ras = false;
   std::vector<double> one(c.d_one.n), two(c.d_two.n);
   c.d_one.download(one.data(), one.size(), c.stream);
   c.d_two.download(two.data(), two.size(), c.stream);
@@ -949,37 +966,6 @@ bool build_ras(Ctx& c) {
   }
   const RasPlan& P = c.ras;
   {
-    // device memory: W and the determinant vectors (16 FP32 / 8 or 16 FP64
-    // columns), the term lists; leave room for the caller's vectors
-    int64_t terms = 0;
-    for (const RasSef& e : P.sef)
-      for (int d = 0; d < e.n; ++d) {
-        const RasSectorDev& S = P.sec[e.sec[d]];
-        terms += (int64_t)S.na * S.nb + (int64_t)S.na * (S.na - 1) / 2 + (int64_t)S.nb * (S.nb - 1) / 2;
-      }
-    auto needs = [&] {
-      return (double)P.cwunit * 64 + (double)P.cdunit * 4 + (double)P.cgunit * 12 + (double)P.ndet * 128 +
-             (double)terms * 4 + (double)P.sef.size() * 9;
-    };
-    size_t fr = 0, tot = 0;
-    c.spare.give_back();
-    PSOCI_HIP(hipMemGetInfo(&fr, &tot));
-    // the matrices per row group can take more than the W elements they save
-    // (10 + 24 orbitals: 18.8 GB against 17 GB): where that is too much, one
-    // matrix per product
-    if (needs() > 0.6 * (double)fr) ras_compact(c.ras, true);
-    const double need = needs();
-    // FP64 in chunks of 16 columns (whole 128-byte W and c pieces) when W and
-    // c fit twice over in 60 % of the free memory, else chunks of 8
-    c.ras_kc64 = need + (double)P.cwunit * 64 + (double)P.ndet * 128 <= 0.6 * (double)fr ? 16 : 8;
-    if (need > 0.6 * (double)fr) {
-      c.ras_why = "needs " + std::to_string((int64_t)(need / 1e9)) + " GB of device memory, " +
-                  std::to_string((int64_t)(fr / 1000000000)) + " GB free";
-      c.ras = RasPlan();
-      return false;
-    }
-  }
-  {
     DevBuf<int> flag;
     flag.alloc(1);
     PSOCI_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), c.stream));
@@ -992,65 +978,44 @@ bool build_ras(Ctx& c) {
     // the string-driven adjoint has no pairs that the reference leaves out
     // (a double excitation both of whose integrals are exactly zero, a single
     // one whose sum is)
-    c.ras_rdm = !(f & 2) && std::find(two.begin(), two.end(), 0.0) == two.end();
+    c.ras_rdm = !(f & 2) && !c.zero_integral;
     if (f & 1) {
       c.ras_rdm = false;
       c.ras_why = "a configuration pair one electron apart has vnt[0] exactly zero with nonzero exchange terms";
       c.ras = RasPlan();
       return false;
     }
+    if (adjoint && !c.ras_rdm) {
+      c.strings_tried = false;  // they may still serve the sigma
+      c.ras = RasPlan();
+      return false;
+    }
+  }
+  // determinant vectors of 16 FP64 columns where they take a small part of the
+  // free memory, else of 16 FP32 or 8 FP64 columns
+  {
+    size_t fr = 0, tot = 0;
+    c.spare.give_back();
+    PSOCI_HIP(hipMemGetInfo(&fr, &tot));
+    const double rows = 2.0 * (double)P.ndet + 2.0;
+    c.ras_kc64 = rows * 128 <= 0.2 * (double)fr ? 16 : 8;
+    if (c.ras_kc64 == 8 && rows * 64 > 0.6 * (double)fr) {
+      c.ras_why = "needs " + std::to_string((int64_t)(rows * 64 / 1e9)) + " GB of device memory, " +
+                  std::to_string((int64_t)(fr / 1000000000)) + " GB free";
+      c.ras = RasPlan();
+      return false;
+    }
+    c.d_rasc.alloc((size_t)(2 * P.ndet + 2) * 8 * c.ras_kc64);
   }
   c.d_rasmask.upload(P.mask, c.stream);
   c.d_rascls.upload(P.cls, c.stream);
   c.d_rasadd.upload(P.add, c.stream);
   c.d_rasrem.upload(P.rem, c.stream);
   c.d_rasblk.upload(P.blk, c.stream);
-  c.d_rascmp.upload(P.cmp, c.stream);
   c.d_rasq.upload(P.qlist, c.stream);
   c.d_raspidx.upload(P.pidx, c.stream);
   c.d_rassef.upload(P.sef, c.stream);
-  RasView v = ras_host_view(P);
-  v.mask = c.d_rasmask.p;
-  v.cls = c.d_rascls.p;
-  v.add = c.d_rasadd.p;
-  v.rem = c.d_rasrem.p;
-  v.blk = c.d_rasblk.p;
-  v.qlist = c.d_rasq.p;
-  v.cmp = c.d_rascmp.p;
-  v.wunit = P.cwunit;
-  v.pidx = c.d_raspidx.p;
-  v.sef = c.d_rassef.p;
-  c.d_rasview.upload(&v, 1, c.stream);
-  // determinant vectors and W: 16 FP32 or ras_kc64 FP64 columns per chunk
-  c.d_rasc.alloc((size_t)(2 * P.ndet + 2) * (c.ras_kc64 == 16 ? 16 * sizeof(double) : 16 * sizeof(float)));
-  // the compact products' matrices and the D entries' signed rows
-  c.d_rasg64.alloc(P.cgunit);
-  c.d_rasg32.alloc(P.cgunit);
-  c.d_rasdidx.alloc(P.cdunit);
-  {
-    DevBuf<double> full;
-    full.upload(P.G, c.stream);
-    int64_t most = 0;
-    for (const RasCmp& C : P.cmp) most = std::max(most, C.nvar * C.nqp);
-    DevBuf<int16_t> pr, pos;
-    pr.alloc(most);
-    pos.alloc(most);
-    for (int bi = 0; bi < (int)P.cmp.size(); ++bi) {
-      const RasCmp& C = P.cmp[bi];
-      if (C.nq == 0) continue;
-      hipLaunchKernelGGL(k_ras_pairs, dim3(nblk(C.nvar, 64)), dim3(64), 0, c.stream, c.d_rasview.p, bi, pr.p, pos.p);
-      PSOCI_HIP(hipGetLastError());
-      const int64_t ng = C.nvar * C.nqp * C.nqp;
-      hipLaunchKernelGGL(k_ras_gvar, dim3(nblk(ng, 256)), dim3(256), 0, c.stream, C.gbase, ng, C.nqp, P.blk[bi].nqp,
-                         pos.p, full.p + P.blk[bi].goff, c.d_rasg64.p, c.d_rasg32.p);
-      PSOCI_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_ras_didx, dim3(nblk(C.nrows * C.nqp, 256)), dim3(256), 0, c.stream, c.d_rasview.p, bi, pr.p,
-                         c.d_rasdidx.p);
-      PSOCI_HIP(hipGetLastError());
-    }
-    ras_tile_tables(c);
-    c.sync();
-  }
+  ras_upload_view(c);
   // the SEF order
   {
     const int64_t nsef = (int64_t)P.sef.size();
@@ -1096,6 +1061,102 @@ bool build_ras(Ctx& c) {
     PSOCI_HIP(hipGetLastError());
     c.sync();
   }
+  // their determinants' signed rows
+  {
+    const int64_t nsef = (int64_t)P.sef.size();
+    c.d_rasrows.alloc(nsef);
+    hipLaunchKernelGGL(k_ras_sefrows, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p,
+                       c.d_rasorder.p, c.d_rasrows.p);
+    PSOCI_HIP(hipGetLastError());
+    c.sync();
+  }
+  return true;
+}
+
+bool build_strings(Ctx& c, bool adjoint) {
+  if (c.strings_tried) return c.have_strings;
+  c.strings_tried = true;
+  try {
+    c.have_strings = make_strings(c, adjoint);
+  } catch (...) {
+    c.drop_plan();
+    throw;
+  }
+  return c.have_strings;
+}
+
+// The products of the plan: the compact layouts' matrices, the D entries' and
+// terms' tables, and W.
+static bool make_products(Ctx& c) {
+  const RasPlan& P = c.ras;
+  if (c.direct_engine_req == 2 && (P.frac || P.fill < 1.0)) {
+    c.ras_why = P.frac ? "odd electron count (one determinant per SEF)" : "not a complete RAS configuration space";
+    return false;
+  }
+  {
+    // device memory: W and the determinant vectors (16 FP32 / 8 or 16 FP64
+    // columns), the term lists; leave room for the caller's vectors
+    int64_t terms = 0;
+    for (const RasSef& e : P.sef)
+      for (int d = 0; d < e.n; ++d) {
+        const RasSectorDev& S = P.sec[e.sec[d]];
+        terms += (int64_t)S.na * S.nb + (int64_t)S.na * (S.na - 1) / 2 + (int64_t)S.nb * (S.nb - 1) / 2;
+      }
+    auto needs = [&] {
+      return (double)P.cwunit * 64 + (double)P.cdunit * 4 + (double)P.cgunit * 12 + (double)P.ndet * 128 +
+             (double)terms * 4 + (double)P.sef.size() * 9;
+    };
+    size_t fr = 0, tot = 0;
+    c.spare.give_back();
+    PSOCI_HIP(hipMemGetInfo(&fr, &tot));
+    fr += c.d_rasc.n;  // counted below
+    // the matrices per row group can take more than the W elements they save
+    // (10 + 24 orbitals: 18.8 GB against 17 GB): where that is too much, one
+    // matrix per product
+    if (needs() > 0.6 * (double)fr) ras_compact(c.ras, true);
+    const double need = needs();
+    // FP64 in chunks of 16 columns (whole 128-byte W and c pieces) when W and
+    // c fit twice over in 60 % of the free memory, else chunks of 8
+    c.ras_kc64 = need + (double)P.cwunit * 64 + (double)P.ndet * 128 <= 0.6 * (double)fr ? 16 : 8;
+    if (need > 0.6 * (double)fr) {
+      c.ras_why = "needs " + std::to_string((int64_t)(need / 1e9)) + " GB of device memory, " +
+                  std::to_string((int64_t)(fr / 1000000000)) + " GB free";
+      c.drop_plan();
+      return false;
+    }
+  }
+  c.d_rascmp.upload(P.cmp, c.stream);
+  ras_upload_view(c);
+  // determinant vectors and W: 16 FP32 or ras_kc64 FP64 columns per chunk
+  c.d_rasc.alloc((size_t)(2 * P.ndet + 2) * 8 * c.ras_kc64);
+  // the compact products' matrices and the D entries' signed rows
+  c.d_rasg64.alloc(P.cgunit);
+  c.d_rasg32.alloc(P.cgunit);
+  c.d_rasdidx.alloc(P.cdunit);
+  {
+    DevBuf<double> full;
+    full.upload(P.G, c.stream);
+    int64_t most = 0;
+    for (const RasCmp& C : P.cmp) most = std::max(most, C.nvar * C.nqp);
+    DevBuf<int16_t> pr, pos;
+    pr.alloc(most);
+    pos.alloc(most);
+    for (int bi = 0; bi < (int)P.cmp.size(); ++bi) {
+      const RasCmp& C = P.cmp[bi];
+      if (C.nq == 0) continue;
+      hipLaunchKernelGGL(k_ras_pairs, dim3(nblk(C.nvar, 64)), dim3(64), 0, c.stream, c.d_rasview.p, bi, pr.p, pos.p);
+      PSOCI_HIP(hipGetLastError());
+      const int64_t ng = C.nvar * C.nqp * C.nqp;
+      hipLaunchKernelGGL(k_ras_gvar, dim3(nblk(ng, 256)), dim3(256), 0, c.stream, C.gbase, ng, C.nqp, P.blk[bi].nqp,
+                         pos.p, full.p + P.blk[bi].goff, c.d_rasg64.p, c.d_rasg32.p);
+      PSOCI_HIP(hipGetLastError());
+      hipLaunchKernelGGL(k_ras_didx, dim3(nblk(C.nrows * C.nqp, 256)), dim3(256), 0, c.stream, c.d_rasview.p, bi, pr.p,
+                         c.d_rasdidx.p);
+      PSOCI_HIP(hipGetLastError());
+    }
+    ras_tile_tables(c);
+    c.sync();
+  }
   // the SEF term lists (merged where an SEF's two determinants read the
   // same W elements): count, scan, fill
   {
@@ -1116,10 +1177,6 @@ bool build_ras(Ctx& c) {
     c.sync();
     c.d_rasterm.alloc(nterm);
     c.d_rasscl.alloc(nsef);
-    c.d_rasrows.alloc(nsef);
-    hipLaunchKernelGGL(k_ras_sefrows, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p,
-                       c.d_rasorder.p, c.d_rasrows.p);
-    PSOCI_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_ras_terms<true>, dim3(nblk(nsef, 256)), dim3(256), 0, c.stream, c.d_rasview.p,
                        c.d_rasorder.p, nullptr, c.d_rastoff.p, c.d_rasterm.p, c.d_rasscl.p, bad.p);
     PSOCI_HIP(hipGetLastError());
@@ -1129,17 +1186,30 @@ bool build_ras(Ctx& c) {
     PSOCI_CHECK(!b, PSOCI_ERR_STATE, "string-driven sigma: inconsistent term lists");
     c.ras_nterm = nterm;
   }
-  c.d_rasw.alloc((size_t)P.cwunit * (c.ras_kc64 == 16 ? 16 * sizeof(double) : 16 * sizeof(float)));
+  c.d_rasw.alloc((size_t)P.cwunit * 8 * c.ras_kc64);
   c.sync();
-  c.have_ras = true;
   return true;
 }
 
-void build_direct(Ctx& c) {
-  if (c.direct_engine_req != 1 && !c.have_ras && !c.ras_tried) {
-    c.ras_tried = true;
-    if (build_ras(c)) return;
+bool build_ras(Ctx& c) {
+  c.ras_tried = true;
+  if (!build_strings(c, false)) return false;
+  try {
+    c.have_ras = make_products(c);
+  } catch (...) {
+    c.drop_plan();
+    throw;
   }
+  return c.have_ras;
+}
+
+void build_direct(Ctx& c) {
+  if (c.direct_engine_req != 1 && !c.have_ras && !c.ras_tried) try {
+      if (build_ras(c)) return;
+    } catch (const Error& e) {
+      // (the pair records may take less)
+      if (e.code != PSOCI_ERR_NOMEM || c.direct_engine_req == 2) throw;
+    }
   PSOCI_CHECK(c.direct_engine_req != 2 || direct_engine(c) == 2, PSOCI_ERR_UNSUPPORTED,
               c.have_ras ? "the string-driven direct sigma on request takes complete EVEN-class spaces only"
                          : "the string-driven direct sigma does not apply to this space: " + c.ras_why);

@@ -91,3 +91,63 @@ def test_always_filled_orbital(nelec, ksym):
         assert np.abs(b2 - a2).max() <= 1e-12 * scale, k
     A.close()
     B.close()
+
+
+def _has_products(H):
+    try:
+        H.direct_ras_info()
+        return True
+    except api.PsociError:
+        return False
+
+
+def test_densities_set_up_no_products():
+    """A density on a new context takes the strings and not the sigma's
+    products; a sigma afterwards, and densities after it, as ever."""
+    cfg, ints = _mrci(5, 7, 6)
+    A = api.Hamiltonian(cfg, ints)
+    B = api.Hamiltonian(cfg, ints)
+    assert B.direct_engine() == 2
+    rng = np.random.default_rng(7)
+    C = rng.standard_normal((A.n, 3))
+    a = A.rdm(C)
+    assert not _has_products(A)
+    b = B.rdm(C)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    assert np.array_equal(A.sigma(C, api.DIRECT), B.sigma(C, api.DIRECT))
+    assert A.direct_engine() == 2 and _has_products(A)
+    c = A.rdm(C)
+    assert np.array_equal(a[0], c[0]) and np.array_equal(a[1], c[1])
+    A.close()
+    B.close()
+
+
+@pytest.mark.parametrize("which", ["integral", "single"])
+def test_pair_walk_without_a_plan(which):
+    """Where exact zeros keep the pair walk (a two-electron integral, or the
+    sum of one-electron moves), a density sets up no string plan; the sigma
+    still takes the strings."""
+    cfg, ints = inputs.fci_configs(5, 4 if which == "integral" else 2), inputs.make_integrals(5, 8)
+    one, two = ints.valone.copy(), ints.valtwo.copy()
+    if which == "integral":
+        two[inputs.canonical_index(0, 2, 1, 3)] = 0.0
+    else:  # (2,0,0,0,0) -> (1,1,0,0,0): h_01 - (01|00) + 2 (01|00)
+        one[inputs.pair_index(0, 1)] = -two[inputs.canonical_index(0, 1, 0, 0)]
+    ints = inputs.Integrals(nbf=5, valone=one, valtwo=two)
+    A = api.Hamiltonian(cfg, ints)
+    B = api.Hamiltonian(cfg, ints)
+    A.direct_engine(1)
+    C = np.random.default_rng(1).standard_normal((A.n, 2))
+    b1, b2, _ = B.rdm(C)
+    assert not _has_products(B)
+    a1, a2, _ = A.rdm(C)
+    np.testing.assert_allclose(b1, a1, rtol=0, atol=1e-12 * np.abs(a1).max())
+    np.testing.assert_allclose(b2, a2, rtol=0, atol=1e-12 * np.abs(a2).max())
+    ref = A.sigma(C, api.DIRECT)
+    assert np.abs(B.sigma(C, api.DIRECT) - ref).max() <= 1e-12 * np.abs(ref).max()
+    assert B.direct_engine() == 2 and _has_products(B)
+    b1, b2, _ = B.rdm(C)
+    np.testing.assert_allclose(b1, a1, rtol=0, atol=1e-12 * np.abs(a1).max())
+    np.testing.assert_allclose(b2, a2, rtol=0, atol=1e-12 * np.abs(a2).max())
+    A.close()
+    B.close()
