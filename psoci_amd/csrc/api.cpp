@@ -259,8 +259,12 @@ int psoci_direct_engine(psoci_ctx* ctx, int request, int* engine) {
     if (request >= 0) {
       c.direct_engine_req = request;
       if (request == 1 && c.have_strings) c.drop_ras();
-      if (request == 2 && !c.have_ras) c.ras_tried = false;
-      if (request == 2 && !c.have_strings) c.strings_tried = false;
+      // another request takes other spaces: what the one before found
+      // impossible may be possible
+      if (request == 2 || request != before) {
+        if (!c.have_ras) c.ras_tried = false;
+        if (!c.have_strings) c.strings_tried = false;
+      }
     }
     if (engine) {
       PSOCI_CHECK(c.have_space && c.have_ints, PSOCI_ERR_STATE, "configurations and integrals are required");

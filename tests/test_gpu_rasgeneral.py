@@ -72,3 +72,22 @@ def test_small_or_thin_lists_stay_on_the_records():
             H.direct_engine(2)
         assert H.direct_engine() == 1
         H.close()
+
+
+@pytest.mark.parametrize("fails", ["sigma", "rdm"])
+def test_unmet_request_is_forgotten(fails):
+    """A request for engine 2 that a call finds impossible does not keep the
+    automatic choice, asked for again, from the strings."""
+    cfg, ints = SPACES[2][1]()
+    H = api.Hamiltonian(cfg, ints)
+    X = np.random.default_rng(2).standard_normal((H.n, 2))
+    assert H.direct_engine(2, build=False) is None
+    if fails == "sigma":
+        with pytest.raises(api.PsociError) as e:
+            H.sigma(X, api.DIRECT)
+        assert e.value.code == api.ERR_UNSUPPORTED
+    else:
+        H.rdm(X)  # the pair walk
+    H.direct_engine(0, build=False)
+    assert H.direct_engine() == 2
+    H.close()
