@@ -302,9 +302,8 @@ int psoci_direct_schedule_prec(psoci_ctx* ctx, int prec, int* order, int* chunk,
  * PSOCI_FP32) at 16 columns: lanes per nonzero (1, 2, 4) and rows per
  * wavefront (1, 2, 4, 8), by a rule on the width, the precision and the row
  * lengths or, for every width, as fixed by the PSOCI_SPMM_SHAPE environment
- * ("<lanes>x<rows>") or a checkpoint with other shapes; tune_ms: -1, or the
- * time a checkpoint's writer measured.  No reference counterpart; any output
- * may be NULL. */
+ * ("<lanes>x<rows>") here or where a loaded checkpoint was written; tune_ms:
+ * -1 (nothing is timed).  No reference counterpart; any output may be NULL. */
 int psoci_stored_shape(psoci_ctx* ctx, int prec, int* lanes_per_nz, int* rows_per_wave, double* tune_ms);
 
 /* The stored sigma's row-length buckets (full symmetric rows of length

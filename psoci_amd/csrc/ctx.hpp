@@ -102,9 +102,8 @@ struct Ctx {
   DevBuf<float> d_val32;      // full FP32
   DevBuf<int32_t> d_lowcnt;   // per row: entries of the lower part (incl. diagonal)
   // stored sigma shape per precision ([0] FP64, [1] FP32) at 16 columns:
-  // lanes per nonzero, rows per wavefront (spmm_fixed: for every width), and
-  // a tuner's time read from an older checkpoint (else -1)
-  bool spmm_fixed = false;
+  // lanes per nonzero, rows per wavefront (spmm_fixed: for every width)
+  bool spmm_fixed[2] = {false, false};
   int spmm_g[2] = {1, 1}, spmm_r[2] = {1, 1};
   double spmm_tune_ms[2] = {-1, -1};
   // row-length buckets (kSpmmBuckets length classes): the rows of each in
@@ -258,11 +257,12 @@ struct Ctx {
 void upload_space(Ctx& c);
 void build_pairs(Ctx& c);               // adjacency + determinant masks (direct sigma, adjoint)
 void build_h(Ctx& c);                   // stored Hamiltonian
-// a checkpoint's stored-sigma shapes
+// a checkpoint's stored-sigma choices per precision: whether rows are launched
+// by length class (chosen: the writer chose by the present rule), and the
+// shapes where the writer had fixed them
 struct SpmmSaved {
+  bool fixed[2], chosen[2], bucketed[2];
   int g[2], r[2], bg[2][kSpmmBuckets], br[2][kSpmmBuckets];
-  bool bucketed[2];
-  double tune_ms[2];
 };
 // the stored sigma's shapes and row-length buckets (after build_h or a load)
 void tune_stored(Ctx& c, const SpmmSaved* saved = nullptr);

@@ -21,12 +21,16 @@
 // Stored Hamiltonian checkpoint (replaces the DRA files of cimat / icicol /
 // number / diag of PsociConstructHamiltonian.C:56-700, whose layout is a
 // property of Global Arrays; this layout is the library's own):
-//   char magic[8] = "PSOCIHCK", int32 version = 1, int32 0,
+//   char magic[8] = "PSOCIHCK", int32 version = 3, int32 fixed,
 //   int64 n, int64 ncfg, int64 nnz (lower triangle + diagonal),
 //   uint64 configuration fingerprint, uint64 integral fingerprint,
 //   int32 lanes[2], int32 rows[2], double tune_ms[2]   (stored-sigma shapes),
+//   int32 used[2], int32 lanes[2][5], int32 rows[2][5] (by row-length class),
 //   int64 rowptr[n + 1], int32 col[nnz], double val[nnz], double diag[n],
 //   uint64 fingerprint of the four arrays.
+// fixed: bit p set where the shapes of precision p were fixed by the writer's
+// PSOCI_SPMM_SHAPE (the others follow from the matrix).  Version 2 files have
+// zero there, version 1 files have no shapes by row-length class.
 // Rows are the reference's (packSefsef, PsociGAhamiltonian.C:4077-4136):
 // columns ascending, the diagonal last.  Loading checks the fingerprints
 // against the context's inputs and the payload, validates the pattern, then
@@ -160,15 +164,14 @@ void civec_read(const char* path, int64_t n, int k, double* C, int* nread) {
 
 struct HHeader {
   char magic[8];
-  int32_t version, pad;
+  int32_t version, fixed;
   int64_t n, ncfg, nnz;
   uint64_t space_hash, ints_hash;
   int32_t lanes[2], rows[2];
   double tune_ms[2];
 };
 static_assert(sizeof(HHeader) == 88, "checkpoint header layout");
-// version 2 follows the header with the stored sigma's row-length bucket
-// shapes (version 1 files have none: one shape for all rows)
+// follows the header from version 2 on
 struct HBuckets {
   int32_t used[2];
   int32_t lanes[2][kSpmmBuckets], rows[2][kSpmmBuckets];
@@ -197,13 +200,14 @@ void save_h(Ctx& c, const char* path) {
   get_h_lower(c, nullptr, col.data(), val.data(), diag.data());
   HHeader h{};
   std::memcpy(h.magic, kMagic, 8);
-  h.version = 2;
+  h.version = 3;
   h.n = n;
   h.ncfg = c.sp.ncfg;
   h.nnz = nnz;
   h.space_hash = c.space_hash;
   h.ints_hash = c.ints_hash;
   for (int p = 0; p < 2; ++p) {
+    if (c.spmm_fixed[p]) h.fixed |= 1 << p;
     h.lanes[p] = c.spmm_g[p];
     h.rows[p] = c.spmm_r[p];
     h.tune_ms[p] = c.spmm_tune_ms[p];
@@ -233,10 +237,10 @@ void load_h(Ctx& c, const char* path) {
   File in(path, "rb");
   HHeader h{};
   in.get(&h, 1, "the header");
-  PSOCI_CHECK(std::memcmp(h.magic, kMagic, 8) == 0 && (h.version == 1 || h.version == 2), PSOCI_ERR_ARG,
+  PSOCI_CHECK(std::memcmp(h.magic, kMagic, 8) == 0 && h.version >= 1 && h.version <= 3, PSOCI_ERR_ARG,
               in.path + ": not a stored-Hamiltonian checkpoint");
   HBuckets hb{};
-  const int64_t hsize = (int64_t)sizeof(HHeader) + (h.version == 2 ? (int64_t)sizeof(HBuckets) : 0);
+  const int64_t hsize = (int64_t)sizeof(HHeader) + (h.version >= 2 ? (int64_t)sizeof(HBuckets) : 0);
   const int64_t n = c.sp.nsef_total;
   PSOCI_CHECK(h.n == n && h.ncfg == c.sp.ncfg && h.space_hash == c.space_hash, PSOCI_ERR_ARG,
               in.path + ": written for another configuration list");
@@ -246,7 +250,7 @@ void load_h(Ctx& c, const char* path) {
   PSOCI_CHECK(nnz >= n && nnz <= n * (n + 1) / 2 && nnz <= (int64_t(1) << 40) &&
                   in.size() == hsize + 8 * (n + 1) + 12 * nnz + 8 * n + 8,
               PSOCI_ERR_ARG, in.path + ": file size does not match its header");
-  if (h.version == 2) in.get(&hb, 1, "the bucket shapes");
+  if (h.version >= 2) in.get(&hb, 1, "the bucket shapes");
   std::vector<int64_t> rp(n + 1);
   std::vector<int32_t> col(nnz);
   std::vector<double> val(nnz), diag(n);
@@ -296,29 +300,34 @@ void load_h(Ctx& c, const char* path) {
   bool shapes_ok = true;
   for (int p = 0; p < 2; ++p) {
     shapes_ok = shapes_ok && lanes_ok(h.lanes[p]) && rows_ok(h.rows[p]);
-    if (h.version == 2 && hb.used[p]) {
+    if (h.version >= 2 && hb.used[p]) {
       shapes_ok = shapes_ok && hb.used[p] == 1;
       for (int b = 0; b < kSpmmBuckets; ++b) shapes_ok = shapes_ok && lanes_ok(hb.lanes[p][b]) && rows_ok(hb.rows[p][b]);
     }
   }
-  if (shapes_ok) {
-    // the writer's stored-sigma shapes (and row-length buckets, which depend
-    // on the matrix alone): the same kernels, bit for bit
-    SpmmSaved sv;
-    for (int p = 0; p < 2; ++p) {
-      sv.g[p] = h.lanes[p];
-      sv.r[p] = h.rows[p];
-      sv.tune_ms[p] = h.tune_ms[p];
-      sv.bucketed[p] = h.version == 2 && hb.used[p] == 1;
-      for (int b = 0; b < kSpmmBuckets; ++b) {
-        sv.bg[p][b] = h.version == 2 ? hb.lanes[p][b] : 1;
-        sv.br[p][b] = h.version == 2 ? hb.rows[p][b] : 1;
-      }
-    }
-    tune_stored(c, &sv);
-  } else {
+  // The writer's fixed shapes and choice of launches, so that the kernels and
+  // their sums are the writer's.  Files before version 3 do not say what was
+  // fixed: shapes with a time were timed for a kernel that is no longer there,
+  // and PSOCI_SPMM_SHAPE gave both precisions one shape, without a time.
+  SpmmSaved sv{};
+  const bool timed = h.tune_ms[0] >= 0.0 || h.tune_ms[1] >= 0.0;
+  bool fixed_before = false;
+  if (h.version < 3 && !timed && h.lanes[0] == h.lanes[1] && h.rows[0] == h.rows[1] && !hb.used[0] && !hb.used[1]) {
     tune_stored(c);
+    for (int p = 0; p < 2; ++p) fixed_before |= h.lanes[p] != c.spmm_g[p] || h.rows[p] != c.spmm_r[p];
   }
+  for (int p = 0; p < 2; ++p) {
+    sv.fixed[p] = h.version >= 3 ? (h.fixed >> p & 1) != 0 : fixed_before;
+    sv.chosen[p] = h.version >= 2 && !timed;
+    sv.bucketed[p] = hb.used[p] == 1;
+    sv.g[p] = h.lanes[p];
+    sv.r[p] = h.rows[p];
+    for (int b = 0; b < kSpmmBuckets; ++b) {
+      sv.bg[p][b] = h.version >= 2 ? hb.lanes[p][b] : 1;
+      sv.br[p][b] = h.version >= 2 ? hb.rows[p][b] : 1;
+    }
+  }
+  tune_stored(c, shapes_ok ? &sv : nullptr);
 }
 
 }  // namespace psoci

@@ -263,7 +263,7 @@ void launch_spmm(Ctx& c, const T* val, const T* X, int ldx, T* Y, int ldy) {
   if (!c.spmm_bucketed[pi]) {
     const int64_t n = c.sp.nsef_total;
     SpmmShape s = spmm_shape(sizeof(T), K, n, (double)c.nnz_full / (double)n);
-    if (c.spmm_fixed) s = {c.spmm_g[pi], c.spmm_r[pi]};
+    if (c.spmm_fixed[pi]) s = {c.spmm_g[pi], c.spmm_r[pi]};
     launch_shape<T, K>(c, s.g, s.r, val, X, ldx, Y, ldy, nullptr, n);
     return;
   }
@@ -271,7 +271,7 @@ void launch_spmm(Ctx& c, const T* val, const T* X, int ldx, T* Y, int ldy) {
     const int64_t lo = c.spmm_boff[b], cnt = c.spmm_boff[b + 1] - lo;
     if (cnt <= 0) continue;
     SpmmShape s = spmm_shape(sizeof(T), K, cnt, (double)c.spmm_bnnz[b] / (double)cnt);
-    if (c.spmm_fixed) s = {c.spmm_bg[pi][b], c.spmm_br[pi][b]};
+    if (c.spmm_fixed[pi]) s = {c.spmm_bg[pi][b], c.spmm_br[pi][b]};
     launch_shape<T, K>(c, s.g, s.r, val, X, ldx, Y, ldy, c.d_brows.p + lo, cnt);
   }
 }
@@ -358,13 +358,12 @@ static void list_buckets(Ctx& c) {
 // and whether the rows are launched by length class: where the classes of at
 // least a tenth of the nonzeros take another R than the mean row does.
 // PSOCI_SPMM_SHAPE=<G>x<R> fixes one shape for every width,
-// PSOCI_SPMM_BUCKETS=0 / 1 the other choice.  saved (a checkpoint's shapes):
-// kept, and fixed where they are not the rule's.
+// PSOCI_SPMM_BUCKETS=0 / 1 the other choice.  saved (a checkpoint's): its
+// fixed shapes and its choice of launches stand for that precision.
 void tune_stored(Ctx& c, const SpmmSaved* saved) {
   count_buckets(c);
   const int64_t n = c.sp.nsef_total;
   const double mean = n ? (double)c.nnz_full / (double)n : 0.0;
-  c.spmm_fixed = false;
   int eg = 0, er = 0;
   if (const char* env = std::getenv("PSOCI_SPMM_SHAPE")) {
     int g = 1, r = 1;
@@ -372,16 +371,25 @@ void tune_stored(Ctx& c, const SpmmSaved* saved) {
         (r == 1 || r == 2 || r == 4 || r == 8)) {
       eg = g;
       er = r;
-      c.spmm_fixed = true;
       saved = nullptr;
     }
   }
   for (int pi = 0; pi < 2; ++pi) {
+    c.spmm_tune_ms[pi] = c.spmm_bucket_ms[pi] = -1.0;
+    if (saved && saved->fixed[pi]) {
+      c.spmm_fixed[pi] = true;
+      c.spmm_g[pi] = saved->g[pi];
+      c.spmm_r[pi] = saved->r[pi];
+      c.spmm_bucketed[pi] = saved->bucketed[pi];
+      std::copy(saved->bg[pi], saved->bg[pi] + kSpmmBuckets, c.spmm_bg[pi]);
+      std::copy(saved->br[pi], saved->br[pi] + kSpmmBuckets, c.spmm_br[pi]);
+      continue;
+    }
     const size_t es = pi ? 4 : 8;
     const SpmmShape s = spmm_shape(es, 16, n, mean);
+    c.spmm_fixed[pi] = eg != 0;
     c.spmm_g[pi] = eg ? eg : s.g;
     c.spmm_r[pi] = er ? er : s.r;
-    c.spmm_tune_ms[pi] = c.spmm_bucket_ms[pi] = -1.0;
     int64_t other = 0;
     int nonempty = 0;
     for (int b = 0; b < kSpmmBuckets; ++b) {
@@ -401,24 +409,8 @@ void tune_stored(Ctx& c, const SpmmSaved* saved) {
     c.spmm_bucketed[pi] = nonempty > 1 && 10 * other >= c.nnz_full;
     if (const char* eb = std::getenv("PSOCI_SPMM_BUCKETS")) c.spmm_bucketed[pi] = nonempty > 1 && eb[0] == '1';
     if (eg) c.spmm_bucketed[pi] = false;
-    if (!saved) continue;
-    bool same = saved->g[pi] == c.spmm_g[pi] && saved->r[pi] == c.spmm_r[pi];
-    for (int b = 0; b < kSpmmBuckets; ++b)
-      if (saved->bucketed[pi])
-        same = same && saved->bg[pi][b] == c.spmm_bg[pi][b] && saved->br[pi][b] == c.spmm_br[pi][b];
-    if (!same) c.spmm_fixed = true;
+    if (saved && saved->chosen[pi]) c.spmm_bucketed[pi] = saved->bucketed[pi];
   }
-  if (saved)
-    for (int pi = 0; pi < 2; ++pi) {
-      c.spmm_g[pi] = saved->g[pi];
-      c.spmm_r[pi] = saved->r[pi];
-      c.spmm_tune_ms[pi] = saved->tune_ms[pi];
-      c.spmm_bucketed[pi] = saved->bucketed[pi];
-      for (int b = 0; b < kSpmmBuckets; ++b) {
-        c.spmm_bg[pi][b] = saved->bg[pi][b];
-        c.spmm_br[pi][b] = saved->br[pi][b];
-      }
-    }
   if (c.spmm_bucketed[0] || c.spmm_bucketed[1]) list_buckets(c);
 }
 

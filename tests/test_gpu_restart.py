@@ -109,3 +109,72 @@ def test_resume_from_vector_file(fci10, built, tmp_path):
     more = H.davidson(4, prec=api.FP64, tol=1e-8, restart=path)
     assert more["converged"]
     np.testing.assert_allclose(more["evals"], full["evals"], atol=1e-9, rtol=0)
+
+
+def _products(H):
+    rng = np.random.default_rng(6)
+    X = {k: rng.standard_normal((H.n, k)) for k in (1, 2, 4, 16)}
+    return [H.sigma(x.astype(t), api.STORED, p) for x in X.values()
+            for t, p in ((np.float64, api.FP64), (np.float32, api.FP32))]
+
+
+def _same(a, b):
+    return [np.array_equal(x, y) for x, y in zip(a, b)]
+
+
+def test_checkpoint_keeps_fixed_shapes(fci6, tmp_path, monkeypatch):
+    """Shapes that the writer had fixed stand at every width, also where they
+    are the rule's at 16 columns; a file from before the flag for that keeps
+    them where it can tell."""
+    cfg, ints, _ = fci6
+    for shape, version in (("4x1", 3), ("2x2", 3), ("2x2", 2)):
+        monkeypatch.setenv("PSOCI_SPMM_SHAPE", shape)
+        H = api.Hamiltonian(cfg, ints)
+        H.build()
+        path = tmp_path / f"{shape}.ck"
+        H.save_h(str(path))
+        monkeypatch.delenv("PSOCI_SPMM_SHAPE")
+        data = bytearray(path.read_bytes())
+        if version == 2:
+            data[8:16] = np.array([2, 0], np.int32).tobytes()
+            path.write_bytes(bytes(data))
+        G = api.Hamiltonian(cfg, ints)
+        G.load_h(str(path))
+        for p in (api.FP64, api.FP32):
+            assert G.stored_shape(p) == H.stored_shape(p)
+        assert all(_same(_products(G), _products(H))), (shape, version)
+        if version == 3:  # one precision fixed: the other follows the rule
+            data[12:16] = np.array([1], np.int32).tobytes()
+            path.write_bytes(bytes(data))
+            G.load_h(str(path))
+            R = api.Hamiltonian(cfg, ints)
+            R.build()
+            assert all(_same(_products(G)[0::2], _products(H)[0::2]))
+            assert all(_same(_products(G)[1::2], _products(R)[1::2]))
+            R.close()
+        G.close()
+        H.close()
+
+
+@pytest.mark.parametrize("version", [1, 2])
+def test_old_checkpoint_shapes_follow_the_rule(fci6, tmp_path, version):
+    """Files from before version 3 with timed shapes: the rule's instead."""
+    cfg, ints, _ = fci6
+    H = api.Hamiltonian(cfg, ints)
+    H.build()
+    path = tmp_path / "h.ck"
+    H.save_h(str(path))
+    data = bytearray(path.read_bytes())
+    data[8:16] = np.array([version, 0], np.int32).tobytes()
+    data[56:72] = np.array([1, 2, 8, 1], np.int32).tobytes()  # lanes, rows
+    data[72:88] = np.array([0.1, 0.2]).tobytes()  # their times
+    if version == 1:
+        del data[88:176]
+    path.write_bytes(bytes(data))
+    G = api.Hamiltonian(cfg, ints)
+    G.load_h(str(path))
+    for p in (api.FP64, api.FP32):
+        assert G.stored_shape(p) == H.stored_shape(p)
+    assert all(_same(_products(G), _products(H)))
+    G.close()
+    H.close()
