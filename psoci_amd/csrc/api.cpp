@@ -65,7 +65,7 @@ int psoci_ctx_create(int device, psoci_ctx** out) {
   if (hipGetDeviceCount(&count) != hipSuccess || count <= 0) return PSOCI_ERR_HIP;
   if (device < 0 || device >= count) return PSOCI_ERR_ARG;
   psoci_ctx* ctx = new psoci_ctx;
-  ctx->c.device = device;
+  ctx->c.device = ctx->c.spare.device = device;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking) != hipSuccess) {
     delete ctx;
     return PSOCI_ERR_HIP;
@@ -485,7 +485,7 @@ int psoci_rdm(psoci_ctx* ctx, int k, const double* C, const double* w, double* g
     bool done = false;
     if (may && c.have_strings && c.ras_rdm) {
       done = fits([&] { psoci::ras_rdm_grad(c, k, dC.p, w, g1.p, g2.p); });
-      if (!done) c.have_ras ? c.drop_adjoint() : c.drop_plan();
+      if (!done && !c.have_ras) c.drop_plan();
     }
     if (!done) {
       if (!c.have_pairs) psoci::build_pairs(c);

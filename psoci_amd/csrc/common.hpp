@@ -30,8 +30,21 @@ struct Error : std::runtime_error {
   } while (0)
 
 // Frees the scratch memory that the calling thread's context keeps between
-// builds (ctx.hpp); false if there is none or it is in use.
-bool give_back_spare();
+// calls (ctx.hpp), or what every context on the current device keeps, except
+// what is in use; false if there is none.
+bool give_back_spare(bool others);
+
+// hipMalloc, again without that memory where it fails: the calling context's
+// first, the others' if that is not enough.
+inline hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  for (int others = 0; others < 2 && e == hipErrorOutOfMemory; ++others)
+    if (give_back_spare(others != 0)) {
+      (void)hipGetLastError();
+      e = hipMalloc(p, bytes);
+    }
+  return e;
+}
 
 // Device buffer owned by a context.
 template <class T>
@@ -51,11 +64,7 @@ struct DevBuf {
     if (count == n && p) return;
     release();
     if (count == 0) return;
-    hipError_t e = hipMalloc(&p, count * sizeof(T));
-    if (e == hipErrorOutOfMemory && give_back_spare()) {
-      (void)hipGetLastError();
-      e = hipMalloc(&p, count * sizeof(T));
-    }
+    const hipError_t e = device_malloc(reinterpret_cast<void**>(&p), count * sizeof(T));
     if (e != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();

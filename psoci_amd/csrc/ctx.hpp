@@ -16,41 +16,38 @@ struct Staging {
   size_t bytes = 0;
 };
 
-// Scratch memory of the Hamiltonian build (buf 0, 1) and of the Davidson
-// solver (2), kept for the context's next one (new integrals at the next
-// geometry) up to kSpareBytes in all: allocating and freeing it every time cost
-// 0.5 ms beside a 1.6 ms build (32,000 SEFs, 0.85 GB), and 20 ms where several
-// contexts built in turn.  Given back when an allocation of the context
-// fails, before the direct engine sizes its plan, and with the context.
+// Scratch memory of the Hamiltonian build (buf 0, 1), of the Davidson solver (2)
+// and of the adjoint (3), kept for the context's next one (new integrals at the
+// next geometry): allocating and freeing it every time cost 0.5 ms beside a 1.6
+// ms build (32,000 SEFs, 0.85 GB), and 20 ms where several contexts built in
+// turn.  A context keeps up to kSpareBytes in all and, beyond a sixteenth of
+// that, no more than a sixteenth of the device memory that is free when it grows
+// (asking every time cost 10 us).  Given back when an allocation of any context
+// on the device fails, before the direct engine sizes its plan, and with the
+// context.
 constexpr size_t kSpareBytes = size_t(1) << 30;
 struct Spare {
-  DevBuf<char> buf[3];
-  bool busy[3] = {false, false, false};
-  bool give_back() {
-    bool any = false;
-    for (int i = 0; i < 3; ++i)
-      if (!busy[i] && buf[i].p) {
-        buf[i].release();
-        any = true;
-      }
-    return any;
-  }
+  DevBuf<char> buf[4];
+  int device = -1;  // of the context
+  size_t allowed = kSpareBytes / 16;  // what it may keep without asking
+  bool busy[4] = {false, false, false, false};  // in use by a scope of the context's thread
+  Spare();
+  ~Spare();
+  Spare(const Spare&) = delete;
+  Spare& operator=(const Spare&) = delete;
+  bool give_back();  // frees what no scope uses; whether there was any
+  void take(int first, int count);
+  void leave(int first, int count);
 };
 // The buffers first .. first + count - 1 in use by a scope; the stream is idle
 // where it ends normally.
 struct SpareUse {
   Spare& s;
   const int first, count;
-  SpareUse(Spare& s_, int first_, int count_) : s(s_), first(first_), count(count_) {
-    for (int i = first; i < first + count; ++i) s.busy[i] = true;
-  }
+  SpareUse(Spare& s_, int first_, int count_) : s(s_), first(first_), count(count_) { s.take(first, count); }
   SpareUse(const SpareUse&) = delete;
   SpareUse& operator=(const SpareUse&) = delete;
-  ~SpareUse() {
-    for (int i = first; i < first + count; ++i) s.busy[i] = false;
-    if (s.buf[0].n + s.buf[1].n + s.buf[2].n > kSpareBytes)
-      for (int i = first; i < first + count; ++i) s.buf[i].release();
-  }
+  ~SpareUse() { s.leave(first, count); }
 };
 // Arrays carved from one of the spare buffers.
 struct Scratch {
@@ -180,10 +177,8 @@ struct Ctx {
   DevBuf<int32_t> d_rasorder;   // the order the SEFs are walked in (d_rastoff, d_rasscl, d_rasrows follow it)
   DevBuf<int2> d_rasrows;       // per SEF: signed rows of its determinants' coefficients
   // the string-driven adjoint (rasrdm.hip): whether it equals the pair walk
-  // (no integral sum that the reference's blocks leave out), and its buffers
+  // (no integral sum that the reference's blocks leave out)
   bool ras_rdm = false;
-  DevBuf<double> d_rdmm, d_rdmpart, d_rdmw;
-  DevBuf<char> d_rdmmat;
   void drop_products() {
     have_ras = false;
     d_rascmp.release();
@@ -199,16 +194,9 @@ struct Ctx {
     d_rasterm.release();
     d_rasscl.release();
   }
-  void drop_adjoint() {
-    d_rdmm.release();
-    d_rdmpart.release();
-    d_rdmw.release();
-    d_rdmmat.release();
-  }
   // everything built; what has been tried stays so
   void drop_plan() {
     drop_products();
-    drop_adjoint();
     have_strings = ras_rdm = false;
     ras = RasPlan();
     d_rasmask.release();
@@ -278,7 +266,8 @@ bool build_strings(Ctx& c, bool adjoint);
 bool build_ras(Ctx& c);
 void sigma_ras(Ctx& c, int prec, int k, const void* X, int ldx, void* Y, int ldy);
 // columns [col0, col0 + kw) of X [n][ldx] as FP64 determinant vectors in
-// c.d_rasc; returns their padded width (16, 8, 4 or 2)
+// c.d_rasc; returns their padded width
+inline int ras_width64(int kw) { return kw > 8 ? 16 : kw > 4 ? 8 : kw > 2 ? 4 : 2; }
 int ras_scatter64(Ctx& c, const double* X, int ldx, int col0, int kw);
 // the adjoint through the string plan (needs have_strings and ras_rdm)
 void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1, double* d_g2);

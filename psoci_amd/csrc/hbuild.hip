@@ -602,8 +602,6 @@ inline unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1)
 
 }  // namespace
 
-bool give_back_spare() { return t_spare && t_spare->give_back(); }
-
 void exclusive_scan_i64(const int64_t* in, int64_t* out, int64_t n, hipStream_t s, void*& tmp, size_t& tmp_bytes) {
   if (n <= 0) return;
   size_t need = 0;
@@ -611,7 +609,7 @@ void exclusive_scan_i64(const int64_t* in, int64_t* out, int64_t n, hipStream_t 
   if (need > tmp_bytes) {
     if (tmp) PSOCI_HIP(hipFree(tmp));
     tmp = nullptr;
-    PSOCI_HIP(hipMalloc(&tmp, need));
+    PSOCI_HIP(device_malloc(&tmp, need));
     tmp_bytes = need;
   }
   PSOCI_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, in, out, n, s));

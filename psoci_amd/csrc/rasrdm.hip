@@ -254,8 +254,26 @@ __global__ __launch_bounds__(64) void k_ras_grad1(int nbf, int n1, int nmat, con
   if (threadIdx.x == 0) g1[e] = s;
 }
 
+// Ranges of a block's rows at kc roots: about four workgroups per CU in all, 8
+// chunks each at least, and at most 256 MB of partial tiles.
+struct GramSplit {
+  int ntp, nsplit;
+  int64_t per;
+  size_t part() const { return (size_t)nsplit * ntp * kPT * kPT; }
+};
+GramSplit gram_split(const RasBlockDev& B, int kc) {
+  const int nt = (B.nq + kPT - 1) / kPT, rc = kKK / kc;
+  GramSplit g;
+  g.ntp = nt * (nt + 1) / 2;
+  int64_t n = std::min<int64_t>((1024 + g.ntp - 1) / g.ntp, (B.nrows + 8 * rc - 1) / (8 * rc));
+  n = std::max<int64_t>(1, std::min<int64_t>(n, ((int64_t)1 << 25) / ((int64_t)g.ntp * kPT * kPT)));
+  g.per = ((B.nrows + n - 1) / n + rc - 1) / rc * rc;
+  g.nsplit = (int)((B.nrows + g.per - 1) / g.per);
+  return g;
+}
+
 template <int KC>
-void gram_blocks(Ctx& c, const RasGrad& R, const double* wk, DevBuf<double>& part, double* M) {
+void gram_blocks(Ctx& c, const RasGrad& R, const double* wk, double* part, double* M) {
   const RasPlan& P = c.ras;
   const double* cv = reinterpret_cast<const double*>(c.d_rasc.p);
   for (int bi = 0; bi < (int)P.blk.size(); ++bi) {
@@ -266,21 +284,12 @@ void gram_blocks(Ctx& c, const RasGrad& R, const double* wk, DevBuf<double>& par
     // symmetric sector for its mirror
     double fac = S.na > S.nb && !P.frac ? 2.0 : 1.0;
     if (S.sym && (B.kind == 1 || B.cu < B.cw || B.tri)) fac *= 2.0;
-    const int nt = (B.nq + kPT - 1) / kPT, ntp = nt * (nt + 1) / 2;
-    constexpr int RC = kKK / KC;
-    // ranges of rows: about four workgroups per CU in all, 8 chunks each at
-    // least, and at most 256 MB of partial tiles
-    int64_t nsplit = std::min<int64_t>((1024 + ntp - 1) / ntp, (B.nrows + 8 * RC - 1) / (8 * RC));
-    nsplit = std::max<int64_t>(1, std::min<int64_t>(nsplit, ((int64_t)1 << 25) / ((int64_t)ntp * kPT * kPT)));
-    int64_t per = (B.nrows + nsplit - 1) / nsplit;
-    per = (per + RC - 1) / RC * RC;
-    nsplit = (B.nrows + per - 1) / per;
-    part.reserve((size_t)nsplit * ntp * kPT * kPT);
-    hipLaunchKernelGGL((k_ras_gram<KC>), dim3((unsigned)ntp, (unsigned)nsplit), dim3(256), 0, c.stream,
-                       c.d_rasview.p, bi, fac, cv, wk, per, part.p);
+    const GramSplit g = gram_split(B, KC);
+    hipLaunchKernelGGL((k_ras_gram<KC>), dim3((unsigned)g.ntp, (unsigned)g.nsplit), dim3(256), 0, c.stream,
+                       c.d_rasview.p, bi, fac, cv, wk, g.per, part);
     PSOCI_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_ras_gram_sum, dim3(nblk((int64_t)ntp * kPT * kPT, 256)), dim3(256), 0, c.stream, ntp,
-                       (int)nsplit, part.p, B.nq, M + R.mat[R.of[bi]].moff);
+    hipLaunchKernelGGL(k_ras_gram_sum, dim3(nblk((int64_t)g.ntp * kPT * kPT, 256)), dim3(256), 0, c.stream, g.ntp,
+                       g.nsplit, part, B.nq, M + R.mat[R.of[bi]].moff);
     PSOCI_HIP(hipGetLastError());
   }
 }
@@ -294,32 +303,39 @@ void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1
   const int64_t n1 = (int64_t)nbf * (nbf + 1) / 2, n2 = n1 * (n1 + 1) / 2;
   const RasGrad R = ras_grad(P);
   const std::vector<RasGradMat>& mat = R.mat;
-  DevBuf<double>&M = c.d_rdmm, &part = c.d_rdmpart, &wk = c.d_rdmw;
-  M.reserve(R.total);
-  c.d_rdmmat.reserve(mat.size() * sizeof(RasGradMat));
-  PSOCI_HIP(hipMemcpyAsync(c.d_rdmmat.p, mat.data(), mat.size() * sizeof(RasGradMat), hipMemcpyHostToDevice, c.stream));
-  const RasGradMat* dm = reinterpret_cast<const RasGradMat*>(c.d_rdmmat.p);
-  hipLaunchKernelGGL(k_ras_fill0, dim3(nblk(R.total, 256)), dim3(256), 0, c.stream, R.total, M.p);
-  PSOCI_HIP(hipGetLastError());
   // the roots in chunks of 16, 8, 4 or 2, their weights padded with zeros
   std::vector<double> hw((size_t)k + 16, 0.0);
   for (int x = 0; x < k; ++x) hw[x] = w ? w[x] : 1.0;
-  wk.reserve(hw.size());
-  PSOCI_HIP(hipMemcpyAsync(wk.p, hw.data(), hw.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
+  size_t npart = 0;
+  for (int c0 = 0; c0 < k; c0 += c.ras_kc64)
+    for (size_t bi = 0; bi < P.blk.size(); ++bi)
+      if (R.of[bi] >= 0) npart = std::max(npart, gram_split(P.blk[bi], ras_width64(std::min(c.ras_kc64, k - c0))).part());
+  SpareUse spare_use(c.spare, 3, 1);
+  Scratch arena{c.spare.buf[3]};
+  arena.buf.reserve(arena.bytes(npart, 8) + arena.bytes(R.total, 8) + arena.bytes(hw.size(), 8) +
+                    arena.bytes(mat.size(), sizeof(RasGradMat)));
+  double* part = arena.take<double>(npart);
+  double* M = arena.take<double>(R.total);
+  double* wk = arena.take<double>(hw.size());
+  RasGradMat* dm = arena.take<RasGradMat>(mat.size());
+  PSOCI_HIP(hipMemcpyAsync(dm, mat.data(), mat.size() * sizeof(RasGradMat), hipMemcpyHostToDevice, c.stream));
+  hipLaunchKernelGGL(k_ras_fill0, dim3(nblk(R.total, 256)), dim3(256), 0, c.stream, R.total, M);
+  PSOCI_HIP(hipGetLastError());
+  PSOCI_HIP(hipMemcpyAsync(wk, hw.data(), hw.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
   for (int c0 = 0; c0 < k; c0 += c.ras_kc64) {
     const int kw = std::min(c.ras_kc64, k - c0);
     const int kc = ras_scatter64(c, dC, k, c0, kw);
-    const double* wc = wk.p + c0;
-    if (kc == 16) gram_blocks<16>(c, R, wc, part, M.p);
-    else if (kc == 8) gram_blocks<8>(c, R, wc, part, M.p);
-    else if (kc == 4) gram_blocks<4>(c, R, wc, part, M.p);
-    else gram_blocks<2>(c, R, wc, part, M.p);
+    const double* wc = wk + c0;
+    if (kc == 16) gram_blocks<16>(c, R, wc, part, M);
+    else if (kc == 8) gram_blocks<8>(c, R, wc, part, M);
+    else if (kc == 4) gram_blocks<4>(c, R, wc, part, M);
+    else gram_blocks<2>(c, R, wc, part, M);
   }
   hipLaunchKernelGGL(k_ras_grad2, dim3(nblk(n2, 256)), dim3(256), 0, c.stream, nbf, n2, (int)mat.size(), dm,
-                     c.d_raspidx.p, M.p, d_g2);
+                     c.d_raspidx.p, M, d_g2);
   PSOCI_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_ras_grad1, dim3((unsigned)n1), dim3(64), 0, c.stream, nbf, (int)n1, (int)mat.size(), dm,
-                     c.d_raspidx.p, M.p, d_g1);
+                     c.d_raspidx.p, M, d_g1);
   PSOCI_HIP(hipGetLastError());
   c.sync();
 }

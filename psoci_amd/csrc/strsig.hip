@@ -1249,7 +1249,7 @@ void ras_timing(Ctx& c, int prec, int k, int reps, double* ms, double* flops) {
 int ras_scatter64(Ctx& c, const double* X, int ldx, int col0, int kw) {
   const int64_t nsef = (int64_t)c.ras.sef.size();
   double* cv = reinterpret_cast<double*>(c.d_rasc.p);
-  const int kc = kw > 8 ? 16 : kw > 4 ? 8 : kw > 2 ? 4 : 2;
+  const int kc = ras_width64(kw);
   const dim3 grid(8 * nblk(nsef * kc, 8 * 256));
   const int64_t na = (int64_t)c.d_rasabsent.n;
   switch (kc) {
