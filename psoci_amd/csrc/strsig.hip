@@ -211,17 +211,20 @@ __global__ __launch_bounds__(64) void k_ras_pairs(const RasView* __restrict__ vp
 }
 
 // The variants' integral matrices, gathered from the block's full matrix
-// (np x np); zero rows and columns for padding.
+// (np x np); zero rows and columns for padding.  (A grid of at most kGvarGrid
+// workgroups: a block's variants can hold more than the 2^32 elements that one
+// launch may have threads, 52 GB of matrices.)
+constexpr unsigned kGvarGrid = 1u << 20;
 __global__ __launch_bounds__(256) void k_ras_gvar(int64_t gbase, int64_t n, int nqp, int np,
                                                   const int16_t* __restrict__ pos, const double* __restrict__ full,
                                                   double* __restrict__ g64, float* __restrict__ g32) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const int64_t row = e / nqp;  // variant * nqp + p-pair
-  const int i = pos[row], j = pos[row / nqp * nqp + e % nqp];
-  const double x = (i < 0 || j < 0) ? 0.0 : full[(int64_t)i * np + j];
-  g64[gbase + e] = x;
-  g32[gbase + e] = (float)x;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t row = e / nqp;  // variant * nqp + p-pair
+    const int i = pos[row], j = pos[row / nqp * nqp + e % nqp];
+    const double x = (i < 0 || j < 0) ? 0.0 : full[(int64_t)i * np + j];
+    g64[gbase + e] = x;
+    g32[gbase + e] = (float)x;
+  }
 }
 
 // Signed vector row of every D entry (built once): didx[dbase + row * nqp +
@@ -1147,8 +1150,9 @@ static bool make_products(Ctx& c) {
       hipLaunchKernelGGL(k_ras_pairs, dim3(nblk(C.nvar, 64)), dim3(64), 0, c.stream, c.d_rasview.p, bi, pr.p, pos.p);
       PSOCI_HIP(hipGetLastError());
       const int64_t ng = C.nvar * C.nqp * C.nqp;
-      hipLaunchKernelGGL(k_ras_gvar, dim3(nblk(ng, 256)), dim3(256), 0, c.stream, C.gbase, ng, C.nqp, P.blk[bi].nqp,
-                         pos.p, full.p + P.blk[bi].goff, c.d_rasg64.p, c.d_rasg32.p);
+      hipLaunchKernelGGL(k_ras_gvar, dim3((unsigned)std::min<int64_t>((ng + 255) / 256, kGvarGrid)), dim3(256), 0,
+                         c.stream, C.gbase, ng, C.nqp, P.blk[bi].nqp, pos.p, full.p + P.blk[bi].goff, c.d_rasg64.p,
+                         c.d_rasg32.p);
       PSOCI_HIP(hipGetLastError());
       hipLaunchKernelGGL(k_ras_didx, dim3(nblk(C.nrows * C.nqp, 256)), dim3(256), 0, c.stream, c.d_rasview.p, bi, pr.p,
                          c.d_rasdidx.p);
