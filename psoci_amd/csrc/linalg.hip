@@ -547,10 +547,11 @@ int tn_waves(int tiles) {
 
 // Workgroups of k_gemm_tn_mfma with w wavefronts that the current device holds
 // at once (compute units x resident workgroups per unit; *units: the compute
-// units), queried once per device, width and columns per lane.
+// units), queried once per thread, device, width and columns per lane (solves
+// of several threads ask at the same time).
 int64_t tn_resident(int w, int cp, int* units) {
-  static int64_t cache[64][9][3] = {};
-  static int cu_cache[64] = {};
+  static thread_local int64_t cache[64][9][3] = {};
+  static thread_local int cu_cache[64] = {};
   int dev = 0;
   PSOCI_HIP(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) dev = 0;
