@@ -300,8 +300,8 @@ int psoci_direct_schedule_prec(psoci_ctx* ctx, int prec, int* order, int* chunk,
 
 /* The stored sigma's kernel shape for precision prec (PSOCI_FP64 or
  * PSOCI_FP32) at 16 columns: lanes per nonzero (1, 2, 4) and rows per
- * wavefront (1, 2, 4, 8), by a rule on the width, the precision and the row
- * lengths or, for every width, as fixed by the PSOCI_SPMM_SHAPE environment
+ * wavefront (1, 2, 4, 8), by a rule on the width, the precision and the rows
+ * or, for every width, as fixed by the PSOCI_SPMM_SHAPE environment
  * ("<lanes>x<rows>") here or where a loaded checkpoint was written; tune_ms:
  * -1 (nothing is timed).  No reference counterpart; any output may be NULL. */
 int psoci_stored_shape(psoci_ctx* ctx, int prec, int* lanes_per_nz, int* rows_per_wave, double* tune_ms);
@@ -310,8 +310,8 @@ int psoci_stored_shape(psoci_ctx* ctx, int prec, int* lanes_per_nz, int* rows_pe
  * < 64, 64-255, 256-1023, 1024-4095, >= 4096): rows[5] per bucket, the
  * 16-column shape of each (lanes_per_nz[5], rows_per_wave[5]), whether
  * per-bucket launches replace the single launch of psoci_stored_shape for
- * precision prec (*used: when classes of a tenth of the nonzeros take
- * another shape, or as PSOCI_SPMM_BUCKETS=0 / 1 fixes it), and bucketed_ms:
+ * precision prec (*used: only where PSOCI_SPMM_BUCKETS=1 asks for it here or
+ * where a loaded checkpoint was written), and bucketed_ms:
  * -1 (nothing is timed).  The reference splits rows by length into its ELL
  * table and the supplemental overflow (PsociGAhamiltonian.C:4223-4312,
  * 9325-9580); no other counterpart.  Any output may be NULL. */

@@ -101,14 +101,15 @@ struct Ctx {
   // stored sigma shape per precision ([0] FP64, [1] FP32) at 16 columns:
   // lanes per nonzero, rows per wavefront (spmm_fixed: for every width)
   bool spmm_fixed[2] = {false, false};
+  int units = 0;  // compute units of the device
   int spmm_g[2] = {1, 1}, spmm_r[2] = {1, 1};
   double spmm_tune_ms[2] = {-1, -1};
   // row-length buckets (kSpmmBuckets length classes): the rows of each in
   // d_brows[spmm_boff[b] .. spmm_boff[b + 1]), a shape per bucket and
   // precision, and whether the bucketed launches are used (count_buckets and
-  // the tuner in sigma.hip)
+  // tune_stored in sigma.hip)
   DevBuf<int32_t> d_brows;
-  int64_t spmm_boff[kSpmmBuckets + 1] = {0}, spmm_bnnz[kSpmmBuckets] = {0};  // rows before, nonzeros of each
+  int64_t spmm_boff[kSpmmBuckets + 1] = {0};  // rows before each
   int spmm_bg[2][kSpmmBuckets] = {}, spmm_br[2][kSpmmBuckets] = {};
   bool spmm_bucketed[2] = {false, false};
   double hbuild_seconds[2] = {-1.0, -1.0};  // last build_h: build proper, shape tuner

@@ -9,6 +9,7 @@
 // reduces one row for all k vectors at once: the row's values and columns
 // stream from HBM once per launch, X rows are gathered from L2/MALL.
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <type_traits>
@@ -233,25 +234,39 @@ void launch_shape(Ctx& c, int g0, int r, const T* val, const T* X, int ldx, T* Y
 }
 
 // Shape rule of a launch of K columns: each lane reads 16 bytes of an x row
-// (G = K sizeof / 16 lanes, at most 4), eight rows share a wavefront (64
-// nonzeros of each are in flight per turn), four where FP32 sums would get
-// longer chains (G = 4), one for rows that fill a wavefront many times over,
-// fewer where the launch would not fill the GPU.  us per call on that matrix
-// (G x R): FP32 1 / 4 / 8 / 16 / 32 columns 1x8 70 / 1x8 89 / 2x8 102 / 4x4 125
-// / 4x4 172, against 1x4 76 / 96 / 140 / 210 / 413; FP64 1x8 91 / 2x8 114 / 4x8
-// 134 / 4x8 185 / 4x8 479, against 1x4 98 / 149 / 220 / 440 / 805.
+// (G = K sizeof / 16 lanes, at most 4).  More rows per wavefront waste less of a
+// row's last turn and of its reduction (gain), if there are wavefronts enough
+// to hide the loads behind; fewer spread the rows more evenly over the compute
+// units.  FP32 sums of G = 4 take at most four rows, whose chains are no longer
+// than those of one lane per nonzero.  us per call over R = 1, 2, 4, 8:
+//   rows (nonzeros each)   FP32 1 column            FP64 16 columns
+//   2,044 (266)            18.2 18.5 19.4 20.1      22.5 22.9 24.4 28.7
+//   9,080 (870)            32.0 32.6 33.8 35.6      62.8 66.9 73.4 88.4
+//   18,354 (650, uneven)   43.4 42.3 43.6 45.2       106   97   99  127
+//   31,650 (715)           64.5 65.1 60.9 54.8       190  186  179  170
+//   122,235 (3,508)        1301 1203 1076  946      3802 3309 3155 2826
+//   257,670 (5,179)        4227 3915 3466 3014     13161 11555 10845 9278
+// and over K on 31,650 rows: FP32 1 / 4 / 8 / 16 / 32 columns 55 / 68 / 81 / 106
+// / 152, FP64 81 / 105 / 125 / 169 against one lane per nonzero at its best R
+// 55 / 68 / 103 / 175 / 397, 85 / 125 / 193 / 392.
 struct SpmmShape {
   int g, r;
 };
-inline int spmm_rows_of_len(size_t es, int g, double len) {
-  if (len > 4096.0) return 1;
-  return es == 4 && g == 4 ? 4 : 8;
-}
-inline SpmmShape spmm_shape(size_t es, int K, int64_t rows, double len) {
+inline SpmmShape spmm_shape(size_t es, int K, int64_t rows, int units) {
   SpmmShape s;
   s.g = std::max(1, std::min(4, (int)(K * es) / 16));
-  s.r = spmm_rows_of_len(es, s.g, len);
-  while (s.r > 1 && rows < (int64_t)2048 * s.r) s.r >>= 1;
+  s.r = 1;
+  double best = 0.0;
+  for (int r = 1, i = 0; r <= (es == 4 && s.g == 4 ? 4 : 8); r *= 2, ++i) {
+    const double gain[4] = {0.0, 0.08, 0.18, 0.30};
+    const double load = std::ceil((double)rows / (4 * r)) / units;  // workgroups per unit
+    if (r > 1 && load <= 1.0) break;
+    const double score = load / std::ceil(load) * (1.0 + gain[i] * std::min(1.0, (load - 1.0) / 3.0));
+    if (score > best) {
+      best = score;
+      s.r = r;
+    }
+  }
   return s;
 }
 
@@ -262,7 +277,7 @@ void launch_spmm(Ctx& c, const T* val, const T* X, int ldx, T* Y, int ldy) {
   const int pi = sizeof(T) == 4 ? 1 : 0;
   if (!c.spmm_bucketed[pi]) {
     const int64_t n = c.sp.nsef_total;
-    SpmmShape s = spmm_shape(sizeof(T), K, n, (double)c.nnz_full / (double)n);
+    SpmmShape s = spmm_shape(sizeof(T), K, n, c.units);
     if (c.spmm_fixed[pi]) s = {c.spmm_g[pi], c.spmm_r[pi]};
     launch_shape<T, K>(c, s.g, s.r, val, X, ldx, Y, ldy, nullptr, n);
     return;
@@ -270,7 +285,7 @@ void launch_spmm(Ctx& c, const T* val, const T* X, int ldx, T* Y, int ldy) {
   for (int b = 0; b < kSpmmBuckets; ++b) {
     const int64_t lo = c.spmm_boff[b], cnt = c.spmm_boff[b + 1] - lo;
     if (cnt <= 0) continue;
-    SpmmShape s = spmm_shape(sizeof(T), K, cnt, (double)c.spmm_bnnz[b] / (double)cnt);
+    SpmmShape s = spmm_shape(sizeof(T), K, cnt, c.units);
     if (c.spmm_fixed[pi]) s = {c.spmm_bg[pi][b], c.spmm_br[pi][b]};
     launch_shape<T, K>(c, s.g, s.r, val, X, ldx, Y, ldy, c.d_brows.p + lo, cnt);
   }
@@ -280,7 +295,16 @@ template <typename T>
 void spmm_any_k(Ctx& c, const T* val, int k, const T* X, int ldx, T* Y, int ldy, const Staging& st) {
   pad::blocks<T>(c, c.sp.nsef_total, k, 32, X, ldx, Y, ldy, [&](int K, const T* x, int lx, T* y, int ly) {
     switch (K) {
-      case 32: launch_spmm<T, 32>(c, val, x, lx, y, ly); break;
+      case 32:
+        // FP64: 32 columns' sums and x pieces leave too few wavefronts (18,354
+        // rows: 368 us, 31,650 rows: 459 us, against twice 97 and 170 us)
+        if constexpr (sizeof(T) == 8) {
+          launch_spmm<T, 16>(c, val, x, lx, y, ly);
+          launch_spmm<T, 16>(c, val, x + 16, lx, y + 16, ly);
+        } else {
+          launch_spmm<T, 32>(c, val, x, lx, y, ly);
+        }
+        break;
       case 16: launch_spmm<T, 16>(c, val, x, lx, y, ly); break;
       case 8: launch_spmm<T, 8>(c, val, x, lx, y, ly); break;
       case 4: launch_spmm<T, 4>(c, val, x, lx, y, ly); break;
@@ -295,23 +319,22 @@ void spmm_any_k(Ctx& c, const T* val, int k, const T* X, int ldx, T* Y, int ldy,
 namespace {
 const int64_t kBucketLim[kSpmmBuckets] = {64, 256, 1024, 4096, INT64_MAX};
 
-// rows (out[b]) and nonzeros (out[kSpmmBuckets + b]) per row-length class
+// rows per row-length class
 __global__ __launch_bounds__(256) void k_bucket_count(int64_t n, const int64_t* __restrict__ rowptr,
                                                       unsigned long long* __restrict__ out) {
-  __shared__ unsigned long long cnt[2 * kSpmmBuckets];
-  if (threadIdx.x < 2 * kSpmmBuckets) cnt[threadIdx.x] = 0;
+  __shared__ unsigned long long cnt[kSpmmBuckets];
+  if (threadIdx.x < kSpmmBuckets) cnt[threadIdx.x] = 0;
   __syncthreads();
   for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x) {
     const int64_t len = rowptr[r + 1] - rowptr[r];
     const int b = len < 64 ? 0 : len < 256 ? 1 : len < 1024 ? 2 : len < 4096 ? 3 : 4;
     atomicAdd(&cnt[b], 1ull);
-    atomicAdd(&cnt[kSpmmBuckets + b], (unsigned long long)len);
   }
   __syncthreads();
-  if (threadIdx.x < 2 * kSpmmBuckets && cnt[threadIdx.x]) atomicAdd(&out[threadIdx.x], cnt[threadIdx.x]);
+  if (threadIdx.x < kSpmmBuckets && cnt[threadIdx.x]) atomicAdd(&out[threadIdx.x], cnt[threadIdx.x]);
 }
 __global__ void k_bucket_zero(unsigned long long* out) {
-  if (threadIdx.x < 2 * kSpmmBuckets) out[threadIdx.x] = 0;
+  if (threadIdx.x < kSpmmBuckets) out[threadIdx.x] = 0;
 }
 }  // namespace
 
@@ -322,19 +345,16 @@ __global__ void k_bucket_zero(unsigned long long* out) {
 static void count_buckets(Ctx& c) {
   const int64_t n = c.sp.nsef_total;
   DevBuf<unsigned long long> d;
-  d.alloc(2 * kSpmmBuckets);
+  d.alloc(kSpmmBuckets);
   hipLaunchKernelGGL(k_bucket_zero, dim3(1), dim3(64), 0, c.stream, d.p);
   hipLaunchKernelGGL(k_bucket_count, dim3((unsigned)std::min<int64_t>(256, (n + 255) / 256)), dim3(256), 0, c.stream, n,
                      c.d_rowptr.p, d.p);
   PSOCI_HIP(hipGetLastError());
-  unsigned long long h[2 * kSpmmBuckets];
-  d.download(h, 2 * kSpmmBuckets, c.stream);
+  unsigned long long h[kSpmmBuckets];
+  d.download(h, kSpmmBuckets, c.stream);
   c.sync();
   c.spmm_boff[0] = 0;
-  for (int b = 0; b < kSpmmBuckets; ++b) {
-    c.spmm_boff[b + 1] = c.spmm_boff[b] + (int64_t)h[b];
-    c.spmm_bnnz[b] = (int64_t)h[kSpmmBuckets + b];
-  }
+  for (int b = 0; b < kSpmmBuckets; ++b) c.spmm_boff[b + 1] = c.spmm_boff[b] + (int64_t)h[b];
 }
 static void list_buckets(Ctx& c) {
   const int64_t n = c.sp.nsef_total;
@@ -354,16 +374,17 @@ static void list_buckets(Ctx& c) {
   c.sync();
 }
 
-// The stored sigma's shapes (spmm_shape; those at 16 columns are reported)
-// and whether the rows are launched by length class: where the classes of at
-// least a tenth of the nonzeros take another R than the mean row does.
-// PSOCI_SPMM_SHAPE=<G>x<R> fixes one shape for every width,
-// PSOCI_SPMM_BUCKETS=0 / 1 the other choice.  saved (a checkpoint's): its
+// The stored sigma's shapes (spmm_shape; those at 16 columns are reported).
+// PSOCI_SPMM_SHAPE=<G>x<R> fixes one shape for every width.  All rows go in
+// one launch; PSOCI_SPMM_BUCKETS=1 launches them by length class, which took 3
+// to 8 % longer on 31,650 to 45,304 rows and 10 to 45 % on 17,022 and 18,354
+// (fewer rows per launch), the same on 48,852 and 263,004, and 8 to 17 % less on
+// 257,670 rows whose configurations mix two lengths (5,877 and 2,976).  saved (a checkpoint's): its
 // fixed shapes and its choice of launches stand for that precision.
 void tune_stored(Ctx& c, const SpmmSaved* saved) {
   count_buckets(c);
   const int64_t n = c.sp.nsef_total;
-  const double mean = n ? (double)c.nnz_full / (double)n : 0.0;
+  PSOCI_HIP(hipDeviceGetAttribute(&c.units, hipDeviceAttributeMultiprocessorCount, c.device));
   int eg = 0, er = 0;
   if (const char* env = std::getenv("PSOCI_SPMM_SHAPE")) {
     int g = 1, r = 1;
@@ -386,11 +407,10 @@ void tune_stored(Ctx& c, const SpmmSaved* saved) {
       continue;
     }
     const size_t es = pi ? 4 : 8;
-    const SpmmShape s = spmm_shape(es, 16, n, mean);
+    const SpmmShape s = spmm_shape(es, 16, n, c.units);
     c.spmm_fixed[pi] = eg != 0;
     c.spmm_g[pi] = eg ? eg : s.g;
     c.spmm_r[pi] = er ? er : s.r;
-    int64_t other = 0;
     int nonempty = 0;
     for (int b = 0; b < kSpmmBuckets; ++b) {
       const int64_t cnt = c.spmm_boff[b + 1] - c.spmm_boff[b];
@@ -398,15 +418,13 @@ void tune_stored(Ctx& c, const SpmmSaved* saved) {
       c.spmm_br[pi][b] = er ? er : 1;
       if (cnt <= 0) continue;
       ++nonempty;
-      const double len = (double)c.spmm_bnnz[b] / (double)cnt;
-      const SpmmShape t = spmm_shape(es, 16, cnt, len);
+      const SpmmShape t = spmm_shape(es, 16, cnt, c.units);
       if (!eg) {
         c.spmm_bg[pi][b] = t.g;
         c.spmm_br[pi][b] = t.r;
       }
-      if (spmm_rows_of_len(es, s.g, len) != spmm_rows_of_len(es, s.g, mean)) other += c.spmm_bnnz[b];
     }
-    c.spmm_bucketed[pi] = nonempty > 1 && 10 * other >= c.nnz_full;
+    c.spmm_bucketed[pi] = false;
     if (const char* eb = std::getenv("PSOCI_SPMM_BUCKETS")) c.spmm_bucketed[pi] = nonempty > 1 && eb[0] == '1';
     if (eg) c.spmm_bucketed[pi] = false;
     if (saved && saved->chosen[pi]) c.spmm_bucketed[pi] = saved->bucketed[pi];

@@ -38,3 +38,25 @@ def test_stored_sigma_widths(name, make, shape, monkeypatch):
         y32 = H.sigma(X.astype(np.float32), api.STORED, api.FP32).reshape(ref.shape)
         assert np.abs(y32 - ref).max() <= 2e-5 * scale, k
     H.close()
+
+
+RULE = [
+    # rows per wavefront of 16 columns, FP64 and FP32, by the number of rows
+    ("2,044 rows", lambda: (inputs.fci_configs(8, 6), inputs.make_integrals(8, 4)), 1, 1),
+    ("18,354 rows", SPACES[3][1], 2, 2),
+    ("31,650 rows", lambda: (inputs.fci_configs(10, 8), inputs.make_integrals(10, 4)), 8, 4),
+]
+
+
+@pytest.mark.parametrize("name,make,r64,r32", RULE, ids=[c[0] for c in RULE])
+def test_rows_per_wavefront(name, make, r64, r32):
+    """Whole rounds of workgroups over 256 compute units."""
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("another number of compute units")
+    cfg, ints = make()
+    H = api.Hamiltonian(cfg, ints)
+    H.build()
+    assert H.stored_shape(api.FP64)["rows_per_wave"] == r64
+    assert H.stored_shape(api.FP32)["rows_per_wave"] == r32
+    H.close()
