@@ -237,6 +237,10 @@ void ras_compact(RasPlan& P, bool full) {
   for (const RasBlockDev& B : P.blk) P.cmp.push_back(compact(P, B, P.nbf - nE, nE, full));
 }
 
+const char* ras_limit(const RasPlan& P) {
+  return P.cwunit >= kRasMaxW ? "more than 2^31 W elements per column" : nullptr;
+}
+
 void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two, bool general, bool all) {
   P = RasPlan();
   const int nbf = sp.nbf, N = sp.nelec;
@@ -396,8 +400,8 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
     P.sec.push_back(S);
   }
   P.ndet = det0;
-  // the D index table names signed vector rows 2 det + negative (and the zero
-  // rows 2 ndet, 2 ndet + 1) in 31 bits
+  // the D index table names signed vector rows det + negative * ndet (and the
+  // zero row 2 ndet) in 31 bits
   if (P.ndet >= ((int64_t)1 << 30) - 1) return fail("more than 2^30 determinants");
   // pair lists per (shape, budget): shape 0 ordered (q, s), shape 1 q > s;
   // q-major so that consecutive pairs reach determinants of one alpha string
@@ -416,7 +420,7 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
           ++cnt;
         }
       qn[id] = cnt;
-      qnp[id] = (cnt + 15) / 16 * 16;  // the products take chunks of 32 pairs and a last one of 16
+      qnp[id] = (cnt + 15) / 16 * 16;  // the products take chunks of 16 pairs
       for (int64_t t = cnt; t < qnp[id]; ++t) P.qlist.push_back((int16_t)-1);
     }
   // blocks
@@ -425,7 +429,7 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
   const int nb2 = nbf * nbf;
   auto g2d = [&](int p, int q, int r, int s) { return g2(two, p, q, r, s); };
   auto h1d = [&](int p, int q) { return h1(one, p, q); };
-  int64_t wunit = 0, dunit = 0;
+  int64_t wunit = 0;
   double flops = 0.0;
   for (size_t si = 0; si < nsec; ++si) {
     const RasSectorDev& S = P.sec[si];
@@ -481,8 +485,6 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
           B.qoff = qoff[id];
           B.wbase = wunit;
           wunit += B.nrows * B.nqp;
-          B.dbase = dunit;
-          dunit += (B.nrows + 15) / 16 * 16 * B.nqp;
           B.qmoff = (int64_t)P.qm.size();
           B.umoff = P.lev[lu].mask_off;
           for (int c0 = 0; c0 < B.nqp; c0 += 16) {
@@ -535,10 +537,8 @@ void ras_plan(RasPlan& P, const Space& sp, const double* one, const double* two,
   }
   (void)nb2;
   ras_compact(P, false);
-  if (wunit >= ((int64_t)1 << 31)) return fail("more than 2^31 W elements per column");
-  if (dunit >= ((int64_t)1 << 31)) return fail("more than 2^31 D index entries");
+  if (const char* why = ras_limit(P)) return fail(why);
   P.wunit = wunit;
-  P.dunit = dunit;
   P.gemm_flops_per_col = flops;
   // SEF -> determinants: SEF k of a configuration with open shells is
   // (D_2k + mult D_2k+1)/sqrt(2), each D = (-1)^phase times its canonical

@@ -49,6 +49,9 @@ namespace psoci {
 
 constexpr int kRasMaxCls = 7;    // external-electron classes 0..6
 constexpr int kRasMaxN = 32;     // electrons
+// W elements per column: a term is an offset and a sign in 32 bits (the D index
+// table has as many entries)
+constexpr int64_t kRasMaxW = (int64_t)1 << 31;
 constexpr uint32_t kRasNone = 0xffffffffu;
 
 // add-table entry: sign << 31 | class << 28 | rank within the class
@@ -93,8 +96,8 @@ struct RasBlockDev {
   int64_t qoff;   // first pair in qlist[]
   int64_t goff;   // first element of G (nqp x nqp, row-major [p-pair][q-pair])
   int64_t wbase;  // W offset per column: W element (wbase + row * nqp + pidx) * KC + v
-  int64_t dbase;  // first entry in the D index table (rows padded to a multiple of 16)
-  // per chunk of 16 pairs: the bits of the orbitals q the chunk adds first
+  // for the host check of the full layout alone (no kernel reads them), per
+  // chunk of 16 pairs: the bits of the orbitals q the chunk adds first
   // (qm[qmoff + chunk]); a chunk all of whose q the row string u already
   // holds has only zero D entries (kinds 0 and 1, where u is the row's
   // first string: mask[umoff + u])
@@ -553,7 +556,6 @@ struct RasPlan {
   std::vector<RasSef> sef;
   int64_t ndet = 0;   // evaluated determinants (all sectors with n_alpha >= n_beta)
   int64_t wunit = 0;  // W elements per column
-  int64_t dunit = 0;  // D index table entries
   double gemm_flops_per_col = 0.0;  // 2 * sum over blocks of rows * nq^2
   // the compact layout: per block, its totals (per column) and flops
   std::vector<RasCmp> cmp;
@@ -600,6 +602,9 @@ struct RasGrad {
   int64_t total = 0;    // elements of all
 };
 RasGrad ras_grad(const RasPlan& P);
+// Why the products' offsets cannot hold the plan's compact layouts; null: they
+// can.
+const char* ras_limit(const RasPlan& P);
 // A view of the plan's host tables (host pointers), e.g. for a host check.
 RasView ras_host_view(const RasPlan& P);
 

@@ -1116,7 +1116,8 @@ static bool make_products(Ctx& c) {
     // the matrices per row group can take more than the W elements they save
     // (10 + 24 orbitals: 18.8 GB against 17 GB): where that is too much, one
     // matrix per product
-    if (needs() > 0.6 * (double)fr) ras_compact(c.ras, true);
+    // (that of the full layouts, if its W offsets fit)
+    if (needs() > 0.6 * (double)fr && P.wunit < kRasMaxW) ras_compact(c.ras, true);
     const double need = needs();
     // FP64 in chunks of 16 columns (whole 128-byte W and c pieces) when W and
     // c fit twice over in 60 % of the free memory, else chunks of 8

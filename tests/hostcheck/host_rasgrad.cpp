@@ -46,3 +46,11 @@ extern "C" int hrg_check(int nbf, int nelec, int ksym, int64_t ncfg, const uint8
   }
   return at == R.total && at > 0 ? 0 : 8;
 }
+
+// ras_limit of a plan whose compact and full layouts have these W elements
+extern "C" int hrg_limited(int64_t cwunit, int64_t wunit) {
+  RasPlan P;
+  P.cwunit = P.cdunit = cwunit;
+  P.wunit = wunit;
+  return ras_limit(P) ? 1 : 0;
+}

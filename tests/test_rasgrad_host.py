@@ -59,3 +59,11 @@ def test_adjoint_matrices(lib, name, make, empty):
     assert lib.hrg_check(cfg.nbf, cfg.nelec, cfg.ksym, ctypes.c_int64(cfg.ncfg), *ptr) == 0
     assert (info[1] > 0) == empty
     assert 0 < info[2] <= info[0] - info[1]
+
+
+def test_limit_is_the_compact_layouts(lib):
+    """The products' 31-bit offsets are those of the compact layout; the full
+    one may be larger."""
+    lim = 1 << 31
+    for compact, full, limited in ((lim - 1, lim - 1, 0), (lim - 1, 2 * lim, 0), (lim, lim, 1), (lim, 2 * lim, 1)):
+        assert lib.hrg_limited(ctypes.c_int64(compact), ctypes.c_int64(full)) == limited
