@@ -228,8 +228,9 @@ int psoci_sigma(psoci_ctx* ctx, int mode, int prec, int k, const void* X, void* 
  * (held until the process ends) instead of context memory; a block needing
  * more (2 n K sizeof(element) bytes at launch width K) is refused with
  * PSOCI_ERR_ARG before anything runs.  The operator must exist already:
- * psoci_build_h (STORED) or the pair records of the direct sigma (built by
- * psoci_direct_info or a first psoci_sigma; DIRECT), else PSOCI_ERR_STATE.
+ * psoci_build_h (STORED) or the direct sigma's products or pair records
+ * (built by psoci_direct_engine, psoci_direct_info or a first psoci_sigma, not
+ * by psoci_rdm; DIRECT), else PSOCI_ERR_STATE.
  * Calls that overlap on one GPU share the array and race.  Same ordering
  * and results as psoci_sigma. */
 int psoci_sigma_noalloc(psoci_ctx* ctx, int mode, int prec, int k, const void* X, void* Y);
@@ -246,10 +247,12 @@ int psoci_direct_info(psoci_ctx* ctx, int64_t* npairs, int64_t* nelems);
  * configuration-driven one; 1 the configuration-driven engine (pair records
  * per connected configuration pair, elements regenerated per determinant
  * pair: the reference's scheme, PsociGAhamiltonian.C:7549-7823); 2 the
- * string-driven engine only.  The string-driven engine applies to spaces of
- * one jsym in the EVEN determinant class with an even electron count whose
- * configuration list is complete RAS: every occupation with at most m
- * electrons in a set of external orbitals (full CI, MR-CISD); it evaluates
+ * string-driven engine only, for spaces of one jsym in the EVEN determinant
+ * class with an even electron count whose configuration list is complete
+ * RAS: every occupation with at most m electrons in a set of external
+ * orbitals (full CI, MR-CISD).  The default choice also takes the strings for
+ * odd electron counts and for lists that are part of such a space, where an
+ * estimate finds them cheaper than the pair records.  The engine evaluates
  * the determinant Hamiltonian by resolutions of the identity over strings
  * with one and two electrons fewer, as dense products on MFMA, and agrees
  * with the configuration-driven sigma to rounding.  With engine != NULL the
@@ -426,6 +429,9 @@ int psoci_combine(psoci_ctx* ctx, int64_t n, int m, int k, const double* A, int 
  * grad_so[NNDAF(nbf)] is the spin-orbit gradient (identically zero: the
  * adjoint takes spaces of one jsym, where the reference never enters socig,
  * PsociHamiltonian.C:223-238; others return PSOCI_ERR_UNSUPPORTED).
+ * Evaluated over the string-driven engine's strings where its spaces and the
+ * integrals allow (no two-electron integral exactly zero), else over the pair
+ * records; neither sets up the direct sigma's products.
  * No reference counterpart for the 2-RDM; the 1-RDM part relates to
  * PsociNOpopulations::constructDensityMatrix (PsociNOpopulations.C:858-989)
  * as grad_one[pp] = D_pp and grad_one[pq] = 2 D_pq (p != q). */

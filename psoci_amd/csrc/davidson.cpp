@@ -346,7 +346,7 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
     const double* G0 = Q.data() + (size_t)c0 * nb;
     // V[:, 0:c0) is orthonormal, so after x -= V (V^T x) the block's Gram
     // matrix is G0 - P^T P; cancellation costs a factor 1 / keep in relative
-    // error
+    // error, and the orthonormalisation another 1 / indep
     for (int i = 0; i < nb; ++i)
       for (int j = 0; j < nb; ++j) {
         double g = G0[(size_t)i * nb + j];
@@ -519,10 +519,11 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
       // spaces stalled where two passes converge
       bool again = m > 0, fused = false;
       if (m > 0) {
-        // FP64: a first pass that keeps 1e-6 of the squared norms gives a
-        // Gram matrix good to 1e-10, which the second pass (held to the
-        // FP32 phase's test, which its nearly orthonormal block meets)
-        // makes good to rounding.  Projection and orthonormalisation in one
+        // FP64: a first pass held to 1e-6 of the squared norms and to 1e-6
+        // for the smallest eigenvalue leaves the block orthonormal to
+        // rounding / (1e-6 * 1e-6) = 1e-4 at worst; the second pass, whose
+        // own test (the FP32 phase's) such a block meets, makes it good to
+        // rounding, and a block that fails it takes the separate passes.  Projection and orthonormalisation in one
         // read of V each way: two projections and two updates instead of
         // five of each (31,650 SEFs, 4 roots: 0.18 to 0.10 ms an iteration
         // beside the sigma)

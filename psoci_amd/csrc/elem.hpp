@@ -392,10 +392,11 @@ PSOCI_HD double sef_elem_ao(const PairInfo& P, const ConfView& A, const ConfView
   return t;
 }
 
-// sef_elem_ao() of a pair of kind 1, 2 or 3, even electron count: flipping every open spin of both determinants exchanges
-// their alpha and beta sets, under which detval_ao() gives the same bits (the
-// same orbital sets, sign windows and canonical integral slots), so
-// D(2i+1, 2j+1) = D(2i, 2j) and D(2i+1, 2j) = D(2i, 2j+1).
+// sef_elem_ao() of a pair of kind 1, 2 or 3, even electron count: flipping every
+// open spin of both determinants exchanges their alpha and beta sets, under
+// which detval_ao() gives the same bits (the same orbital sets, sign windows
+// and canonical integral slots), so D(2i+1, 2j+1) = D(2i, 2j) and
+// D(2i+1, 2j) = D(2i, 2j+1).
 PSOCI_HD double sef_elem_flip(const PairInfo& P, const ConfView& A, const ConfView& B, uint64_t aI, uint64_t aJ,
                               double multi, double multj, const double* __restrict__ two) {
   const double d0 = detval_ao(P, A, B, aI, aJ, two);

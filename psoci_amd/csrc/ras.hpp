@@ -1,4 +1,4 @@
-// String-driven direct sigma for complete RAS spaces (host plan and the
+// String-driven direct sigma for RAS spaces (host plan and the
 // index arithmetic shared by the GPU kernels and the host check).
 //
 // A configuration list that holds every occupation of N electrons with at
@@ -33,11 +33,12 @@
 //
 // The reference keeps no such structure (it regenerates every block with
 // generateSOCIblocks, PsociHamiltonian.C:401-558); the plan is used only
-// where it is exact: EVEN-class spaces of one jsym with an even electron
-// count, and no configuration pair whose single-excitation sum vnt[0] is
-// exactly zero while its exchange terms are not (the reference skips such a
-// block, processSingleExcitation PsociHamiltonian.C:190-261; checked on the
-// GPU at setup).
+// where it is exact: spaces of one jsym, EVEN class or an odd electron count
+// (one determinant per SEF), and no configuration pair whose single-excitation
+// sum vnt[0] is exactly zero while its exchange terms are not (the reference
+// skips such a block, processSingleExcitation PsociHamiltonian.C:190-261;
+// checked on the GPU at setup).  A list that is only part of a RAS space runs
+// on the whole space, the coefficients of the others zero.
 #pragma once
 #include <cstdint>
 #include <string>

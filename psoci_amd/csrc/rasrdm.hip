@@ -1,6 +1,6 @@
-// Adjoint of the energies on the string plan (ras.hpp): for complete RAS
-// spaces the generalised 1- and 2-RDM that psoci_rdm returns are
-// contractions of Gram matrices.
+// Adjoint of the energies on the string plan (ras.hpp): for its spaces the
+// generalised 1- and 2-RDM that psoci_rdm returns are contractions of Gram
+// matrices.
 //
 // E = sum_k w_k c_k^T H c_k is, per product of the plan (RasBlockDev), the sum
 // over its rows of D^T G D with G the product's integral matrix, so
@@ -11,7 +11,7 @@
 // atomics: the results are reproducible.  Replaces, for these spaces, the
 // pair walk of rdm.hip, which generates every SEF element and adds to a few
 // integrals with atomics: four roots of the 10-orbital, 8-electron full CI
-// 22.5 -> 0.31 ms, and no pair records (56 ms of set-up) for a gradient.
+// 22.6 -> 0.43 ms a call, and no pair records (56 ms of set-up) for a gradient.
 //
 // The pair walk leaves out pairs whose integral sums are exactly zero (the
 // reference computes no block for them); the Gram matrices do not, so spaces
@@ -309,7 +309,8 @@ void ras_rdm_grad(Ctx& c, int k, const double* dC, const double* w, double* d_g1
   size_t npart = 0;
   for (int c0 = 0; c0 < k; c0 += c.ras_kc64)
     for (size_t bi = 0; bi < P.blk.size(); ++bi)
-      if (R.of[bi] >= 0) npart = std::max(npart, gram_split(P.blk[bi], ras_width64(std::min(c.ras_kc64, k - c0))).part());
+      if (R.of[bi] >= 0)
+        npart = std::max(npart, gram_split(P.blk[bi], ras_width64(std::min(c.ras_kc64, k - c0))).part());
   SpareUse spare_use(c.spare, 3, 1);
   Scratch arena{c.spare.buf[3]};
   arena.buf.reserve(arena.bytes(npart, 8) + arena.bytes(R.total, 8) + arena.bytes(hw.size(), 8) +

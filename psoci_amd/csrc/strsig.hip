@@ -1,7 +1,7 @@
 // String-driven direct sigma on the GPU (the plan and its index arithmetic
 // are in ras.hpp / ras.cpp).
 //
-// Replaces, for complete RAS spaces (full CI and MR-CISD lists), the direct
+// Replaces, for RAS spaces (full CI and MR-CISD lists) and parts of them, the direct
 // path of the reference (matrixVectorProductsScatterAccumulateLowLevel...
 // DirectFetch, PsociGAhamiltonian.C:7549-7823, with matrixVectorUpdate
 // :13036-13115), which regenerates every configuration-pair block.  One
@@ -100,9 +100,9 @@ __global__ __launch_bounds__(256) void k_ras_order(int64_t ndet, const int64_t* 
   if (d < ndet && flag[d]) order[rank[d]] = sef[d];
 }
 // The signed rows of every SEF's determinant coefficients, in that order
-// (built once): rows.x = det + negative * ndet of its first determinant; rows.y the same for the second, or -1 (one determinant, coefficient
-// 1/sqrt(2)) or -2 (a closed shell, coefficient 1); -3 marks a determinant
-// outside the plan.
+// (built once): rows.x = det + negative * ndet of its first determinant; rows.y
+// the same for the second, or -1 (one determinant, coefficient 1/sqrt(2)) or -2
+// (a closed shell, coefficient 1); -3 marks a determinant outside the plan.
 __global__ __launch_bounds__(256) void k_ras_sefrows(const RasView* __restrict__ vp,
                                                      const int32_t* __restrict__ order, int2* __restrict__ rows) {
   const RasView& v = *vp;
@@ -645,8 +645,8 @@ void k_ras_gemm_wide(const RasTile* __restrict__ tiles, int64_t ntiles, int sh, 
 #pragma unroll
       for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) 
-            ras_store(acc[i][j][t], &Wt[((int64_t)(ps + 16 * i + M::row(t, lane)) * tile.rows + row) * KC + m % KC]);
+        for (int t = 0; t < 4; ++t)
+          ras_store(acc[i][j][t], &Wt[((int64_t)(ps + 16 * i + M::row(t, lane)) * tile.rows + row) * KC + m % KC]);
     }
   };
   // the same number of barriers in every variant: nch
