@@ -485,7 +485,10 @@ int psoci_rdm(psoci_ctx* ctx, int k, const double* C, const double* w, double* g
     bool done = false;
     if (may && c.have_strings && c.ras_rdm) {
       done = fits([&] { psoci::ras_rdm_grad(c, k, dC.p, w, g1.p, g2.p); });
-      if (!done && !c.have_ras) c.drop_plan();
+      if (!done && !c.have_ras) {
+        c.drop_plan();
+        c.strings_tried = false;  // later ones may find the memory
+      }
     }
     if (!done) {
       if (!c.have_pairs) psoci::build_pairs(c);

@@ -1005,6 +1005,7 @@ static bool make_strings(Ctx& c, bool adjoint) {
     if (c.ras_kc64 == 8 && rows * 64 > 0.6 * (double)fr) {
       c.ras_why = "needs " + std::to_string((int64_t)(rows * 64 / 1e9)) + " GB of device memory, " +
                   std::to_string((int64_t)(fr / 1000000000)) + " GB free";
+      c.strings_tried = !adjoint;
       c.ras = RasPlan();
       return false;
     }
@@ -1083,6 +1084,7 @@ bool build_strings(Ctx& c, bool adjoint) {
     c.have_strings = make_strings(c, adjoint);
   } catch (...) {
     c.drop_plan();
+    c.strings_tried = !adjoint;  // a density's shortage of memory is not the sigma's
     throw;
   }
   return c.have_strings;
