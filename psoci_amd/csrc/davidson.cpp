@@ -94,6 +94,10 @@ int davidson(Ctx& c, const psoci_dav_params& p, double* evals, double* evecs, ps
   Linalg L;
   L.stream = c.stream;
   L.host = &c.lin_host;
+  struct TrimGuard {
+    Linalg& l;
+    ~TrimGuard() { l.trim(); }
+  } trim_guard{L};
   // V^T HV of a step, in host memory (at a fixed place: captured launches
   // write to it)
   double* const proj = L.results((size_t)mmax * std::max(k0, kc));

@@ -623,9 +623,22 @@ void Linalg::put(void* dst, const char* staged, size_t bytes) {
 }
 
 void Linalg::put_y(const double* y, size_t count) {
+  if (count * sizeof(double) > kPinnedBytes) {
+    PSOCI_HIP(hipMemcpyAsync(ysmall.p, y, count * sizeof(double), hipMemcpyHostToDevice, stream));
+    PSOCI_HIP(hipStreamSynchronize(stream));  // y is the caller's
+    return;
+  }
   char* st = stage(count * sizeof(double));
   std::copy(y, y + count, reinterpret_cast<double*>(st));
   put(ysmall.p, st, count * sizeof(double));
+}
+
+void Linalg::trim() {
+  for (HostBuf* b : {&host->in, &host->out})
+    if (b->n > kPinnedBytes) {
+      (void)hipStreamSynchronize(stream);
+      b->release();
+    }
 }
 
 double* Linalg::results(size_t count) {
@@ -665,6 +678,13 @@ void Linalg::gemm_tn(int64_t n, int m, int b, const TA* A, int lda, const TA* B,
 
 template <typename TA>
 void Linalg::gemm_tn_host(int64_t n, int m, int b, const TA* A, int lda, const TA* B, int ldb, double* out_host) {
+  if ((size_t)m * b * sizeof(double) > kPinnedBytes) {
+    small.reserve((size_t)m * b);
+    gemm_tn(n, m, b, A, lda, B, ldb, small.p);
+    PSOCI_HIP(hipMemcpyAsync(out_host, small.p, (size_t)m * b * sizeof(double), hipMemcpyDeviceToHost, stream));
+    PSOCI_HIP(hipStreamSynchronize(stream));
+    return;
+  }
   double* res = results((size_t)m * b);
   gemm_tn(n, m, b, A, lda, B, ldb, res);
   PSOCI_HIP(hipStreamSynchronize(stream));
@@ -737,13 +757,15 @@ void Linalg::gemm_nn2(int64_t n, int m, int k, const TA* A, int lda, const doubl
   if (k == 0 || n == 0) return;
   ysmall.reserve((size_t)2 * m * k);
   const size_t mk = (size_t)m * k;
-  char* st = stage(2 * mk * sizeof(double));
-  double* y = reinterpret_cast<double*>(st);
+  std::vector<double> large(2 * mk * sizeof(double) > kPinnedBytes ? 2 * mk : 0);
+  char* st = large.empty() ? stage(2 * mk * sizeof(double)) : nullptr;
+  double* y = large.empty() ? reinterpret_cast<double*>(st) : large.data();
   for (size_t e = 0; e < mk; ++e) {
     y[e] = Y1_host[e];
     y[mk + e] = -Y2_host[e];
   }
-  put(ysmall.p, st, 2 * mk * sizeof(double));
+  if (large.empty()) put(ysmall.p, st, 2 * mk * sizeof(double));
+  else put_y(y, 2 * mk);
   if (X)
     launch_nn<true, true, false, TA, TO>(stream, n, m, k, A, lda, B, ldb, ysmall.p, ysmall.p + (size_t)m * k, 0.0,
                                          Out, ldo, X, ldx);

@@ -11,15 +11,17 @@ struct HostBuf {
   HostBuf() = default;
   HostBuf(const HostBuf&) = delete;
   HostBuf& operator=(const HostBuf&) = delete;
-  ~HostBuf() {
-    if (p) (void)hipHostFree(p);
-  }
-  // grow only; the caller has made sure that no kernel uses the memory
-  void reserve(size_t bytes) {
-    if (bytes <= n) return;
+  ~HostBuf() { release(); }
+  // (the caller has made sure that no kernel uses the memory)
+  void release() {
     if (p) (void)hipHostFree(p);
     p = nullptr;
     n = used = 0;
+  }
+  // grow only
+  void reserve(size_t bytes) {
+    if (bytes <= n) return;
+    release();
     PSOCI_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), bytes, hipHostMallocCoherent));
     n = bytes;
   }
@@ -29,7 +31,10 @@ struct HostBuf {
 // through pinned memory: a kernel copies them in (put), and the reduction of
 // a projection writes its result into host memory.  hipMemcpyAsync on the
 // caller's pageable arrays waits for each copy on the host, 12 to 20 us of
-// idle GPU per product.
+// idle GPU per product.  Larger ones go the pageable way, whose wait no longer
+// counts there (60,000 rows x 2048 x 2048: combination 14.6 ms through pinned
+// memory, 13.7 ms so), and nothing larger stays pinned after a solve.
+constexpr size_t kPinnedBytes = size_t(4) << 20;
 struct LinalgHost {
   HostBuf in, out;
 };
@@ -47,6 +52,8 @@ struct Linalg {
   void put_y(const double* y, size_t count);  // into ysmall
   // the projections' results in host memory: room for count doubles
   double* results(size_t count);
+  // frees the host memory beyond kPinnedBytes (waits for the stream)
+  void trim();
 
   // partial-sum buffer of gemm_tn for (n, m, b); reserve_tn: for every
   // m <= mmax, b <= bmax (so captured launches allocate nothing)

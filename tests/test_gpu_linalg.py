@@ -49,3 +49,35 @@ def test_combine_matches_numpy(ctx, n, m, k, lda, ldo, alpha):
     out = Od.cpu().numpy()
     scale = max(1.0, np.abs(ref).max())
     assert np.abs(out - ref).max() <= 1e-12 * scale * max(1.0, m / 16)
+
+
+def test_large_small_matrices(ctx):
+    """Matrices beyond the pinned staging (more than 4 MiB) and at its edge."""
+    import torch
+    g = torch.Generator().manual_seed(5)
+    n = 700
+    for m in (724, 725, 900):  # 724 x 724 values are 4 MiB less 848 bytes
+        A = torch.randn(n, m, generator=g, dtype=torch.float64)
+        B = torch.randn(n, m, generator=g, dtype=torch.float64)
+        ref = A.numpy().T @ B.numpy()
+        out = ctx.project(A.cuda(), B.cuda())
+        assert np.abs(out - ref).max() <= 1e-12 * np.abs(ref).max(), m
+        Y = np.random.default_rng(m).standard_normal((m, m))
+        Od = torch.zeros(n, m, dtype=torch.float64, device="cuda")
+        ctx.combine(A.cuda(), Y, Od)
+        ref = A.numpy() @ Y
+        assert np.abs(Od.cpu().numpy() - ref).max() <= 1e-12 * np.abs(ref).max() * (m / 16), m
+
+
+def test_solve_with_a_wide_subspace(fci10):
+    """V^T HV of a wide subspace beyond the pinned memory that is kept."""
+    cfg, ints, _ = fci10
+    H = api.Hamiltonian(cfg, ints)
+    H.build()
+    ref = H.davidson(16, prec=api.FP64, tol=1e-5, graph=1)
+    out = H.davidson(16, prec=api.FP64, tol=1e-5, max_subspace=17000, graph=1)  # 17000 x 32 values
+    assert ref["converged"] and out["converged"]
+    np.testing.assert_allclose(out["evals"], ref["evals"], rtol=0, atol=1e-8)
+    again = H.davidson(16, prec=api.FP64, tol=1e-5, graph=1)
+    assert np.array_equal(again["evals"], ref["evals"])
+    H.close()
